@@ -106,7 +106,8 @@ def build_oracle(verbose: bool = False) -> None:
     """Build the checker: oracle/liboracle.so, and oracle/_ref when the reference is present."""
     root = PKG.parent / "oracle"
     _run(["make", "-s", "-C", str(root), "lib"], verbose)
-    if Path(os.environ.get("GPHI_REFERENCE", "/root/reference")).is_dir() and shutil.which("g++"):
+    ref = Path(os.environ.get("GPHI_REFERENCE", "/root/reference"))
+    if (ref / "tools").is_dir() and (ref / "apps").is_dir() and shutil.which("g++"):
         _run(["make", "-s", "-j8", "-C", str(root), "ref"], verbose)
 
 
