@@ -76,14 +76,18 @@ int gphi_open(const gphi_opts *opts, gphi_ctx **out)
 	}
 	if ((e = hipSetDevice(ctx->device)) != hipSuccess ||
 	    (e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking)) != hipSuccess ||
-	    (e = hipHostMalloc((void **)&ctx->h_ctrl, sizeof(gphi::StepCtrl), hipHostMallocDefault)) !=
-	        hipSuccess) {
+	    (e = hipHostMalloc((void **)&ctx->h_ctrl, sizeof(gphi::StepCtrl) + sizeof(gphi::LevelBoard),
+	                       hipHostMallocDefault)) != hipSuccess) {
 		int rc = set_error(nullptr, GPHI_E_HIP, "gphi_open: %s", hipGetErrorString(e));
 		if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
 		delete ctx;
 		return rc;
 	}
-	memset(ctx->h_ctrl, 0, sizeof(gphi::StepCtrl));
+	memset(ctx->h_ctrl, 0, sizeof(gphi::StepCtrl) + sizeof(gphi::LevelBoard));
+	ctx->h_board = reinterpret_cast<gphi::LevelBoard *>(ctx->h_ctrl + 1);
+	int khz = 0;
+	if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->device) == hipSuccess && khz > 0)
+		ctx->wall_clock_khz = khz;
 	gphi::noalloc_setup(ctx->device);  // device address of gphi_bfs_noalloc's scratch array
 	ctx->ev_ok = true;
 	for (auto &ev : ctx->ev)

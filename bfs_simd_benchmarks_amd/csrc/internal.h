@@ -95,6 +95,37 @@ struct QueueBufs {
 inline uint32_t queue_stride(uint32_t n_pad) { return n_pad; }
 inline uint32_t tile_lo_stride(uint64_t m) { return (uint32_t)(m / kSparseTile + 2); }
 
+// The level loop of small graphs (small.hip).  LevelRec: a level's totals, the
+// accumulators the level before adds to; a ring over the levels, whose entry
+// half a ring ahead is cleared as a level starts.  LevelBoard: what the
+// device tells the host, in pinned memory.
+constexpr uint32_t kLevelRing = 16;
+struct LevelRec {
+	uint32_t fsize;            // |F|
+	uint32_t chunks;           // chunks its dense sweep took
+	unsigned long long qpack;  // (queue entries << 32) | sum of out-degrees
+	unsigned long long reached, traversed;  // sums of |F| and of sum deg(F) up to this level
+	uint32_t pad[24];          // a 128-byte line each
+};
+static_assert(sizeof(LevelRec) == 128, "LevelRec is one line");
+struct LevelBoard {
+	unsigned long long progress;  // (levels started << 1) | ended
+	unsigned long long reached, traversed;
+	unsigned long long t_begin, t_end;  // device wall clock
+	uint32_t levels;
+	uint4 trace[GPHI_MAX_STEPS];  // per step: direction, |F|, sum deg(F), chunks swept
+};
+constexpr size_t kCtrlBytes = sizeof(StepCtrl) + kLevelRing * sizeof(LevelRec);
+// The graphs it serves (2048-edge chunks).  Measured against the five-kernel
+// loop without output: BFS 214 -> 96 us at 2^10 vertices (edge factor 16),
+// 326 -> 212 at 2^20, 549 -> 524 at 2^23 x 8, 840 -> 613 at 2^24 x 4, but 723 ->
+// 742 at 2^23 x 24 and 937 -> 951 at 2^24 x 16, where the live lists' balance
+// pays; SSSP 432 -> 167, 995 -> 773, 2914 -> 2557, 3539 -> 3319 and 4550 -> 4284,
+// 5022 -> 4572 us.
+constexpr uint32_t kSmallVerts = 1u << 24;
+constexpr uint32_t kSmallChunksBfs = 1u << 15;
+constexpr uint32_t kSmallChunksSssp = 1u << 17;
+
 struct DevGraph {
 	uint32_t n = 0;
 	uint64_t m = 0;
@@ -154,6 +185,8 @@ struct gphi_ctx {
 	std::string last;
 	// pinned host control block for per-step readback
 	gphi::StepCtrl *h_ctrl = nullptr;
+	gphi::LevelBoard *h_board = nullptr;  // in h_ctrl's allocation, written by small.hip's kernels
+	double wall_clock_khz = 1e5;          // rate of the device wall clock
 	// per-step timing: [0] start, [1] init done, [2+2k] sweep k done, [3+2k] update k
 	// done, [2*MAX+4+k] chunk selection of dense step k done
 	hipEvent_t ev[3 * GPHI_MAX_STEPS + 4];
@@ -183,6 +216,7 @@ struct gphi_graph {
 		return gphi::QueueBufs{queue, qoff, tile_lo, gphi::queue_stride(g.n_pad), gphi::tile_lo_stride(g.m)};
 	}
 	gphi::StepCtrl *ctrl = nullptr;
+	gphi::LevelRec *rec = nullptr;  // in ctrl's allocation (kCtrlBytes)
 	uint4 *blk_cnt = nullptr;  // per update block: |F|, queue entries, degree sum
 	uint2 *blk_base = nullptr; // per update block: queue and degree prefix
 	uint2 *wave_cnt = nullptr; // per update wavefront: queue entries, degree sum
@@ -264,8 +298,15 @@ int download_graph(gphi_graph *gr, uint32_t *deg, uint32_t *cols, uint32_t *cw, 
                    uint32_t *tt, uint32_t *tw);
 
 int ensure_traversal_state(gphi_graph *gr);
+// the level loop of small graphs without per-level timing (small.hip); the
+// traversal has ended, and st is filled in, when it returns
+bool small_graph(const DevGraph &G, bool bfs);
+template <bool kBfs>
+int small_level_loop(gphi_graph *gr, uint32_t src, gphi_stats *st);
 // the BFS level loop of run_bfs on gr's state buffers (set up by the caller)
 int bfs_level_loop(gphi_graph *gr, uint32_t src, gphi_stats *st);
+// blocks of `block` threads of a kernel that fit the device at once, a multiple of the XCD count
+unsigned resident_grid(const void *kernel, unsigned block = kBlock);
 uint32_t live_list_capacity(uint64_t nchunks);  // entries of one XCD's live-chunk list
 void launch_frontier_update_driven(gphi_graph *gr, uint32_t threshold);
 int run_bfs_batch(gphi_graph *gr, const uint32_t *srcs, uint32_t k, uint8_t *levels, gphi_stats *st);

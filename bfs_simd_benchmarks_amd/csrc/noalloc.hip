@@ -70,7 +70,8 @@ size_t carve_state(const DevGraph &G, uint8_t *base, gphi_graph *t)
 	t->queue = (uint32_t *)take(2 * (size_t)queue_stride(G.n_pad) * 4);  // two halves (QueueBufs)
 	t->qoff = (uint32_t *)take(2 * (size_t)queue_stride(G.n_pad) * 4);
 	t->tile_lo = (uint32_t *)take(2 * (size_t)tile_lo_stride(G.m) * 4);
-	t->ctrl = (StepCtrl *)take(sizeof(StepCtrl));
+	t->ctrl = (StepCtrl *)take(kCtrlBytes);
+	t->rec = reinterpret_cast<LevelRec *>(t->ctrl + 1);
 	t->live = (uint32_t *)take((size_t)live_list_capacity(G.nchunks) * kNumXcd * 4 + 4);
 	t->live_cnt = (uint32_t *)take(kLiveCntBytes);
 	t->trace = (uint4 *)take((GPHI_MAX_STEPS + 1) * sizeof(uint4));

@@ -1,0 +1,91 @@
+"""The two-launch level loop of small graphs (per-level timing off): levels,
+parents, trace and distances against the oracle where its shares can go wrong
+-- vertex counts around a lane's 8, a wavefront's 512 and a block's 2048 or
+8192 vertices, tile widths that split a lane's vertices, chunk counts around
+a block's share, frontiers without out-edges, and paths past the ring of
+level records."""
+import numpy as np
+import pytest
+
+import oracle as O
+import bfs_simd_benchmarks_amd as G
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def quiet():
+    with G.Context(0) as c:
+        c.set_level_timing(False)
+        yield c
+
+
+def random_graph(n, m, W, S, seed, wmax=0):
+    """m random edges plus a hub: vertex 0 points at every seventh vertex."""
+    rng = np.random.default_rng(seed)
+    hub = np.arange(1, n, 7, dtype=np.int64)
+    h = np.concatenate([rng.integers(0, n, m), np.zeros(len(hub), np.int64)])
+    t = np.concatenate([rng.integers(0, n, m), hub])
+    keep = h != t
+    e = np.unique(h[keep] * n + t[keep])
+    h, t = (e // n).astype(np.uint32), (e % n).astype(np.uint32)
+    w = rng.integers(1, wmax + 1, len(h)).astype(np.uint32) if wmax else None
+    return O.tile_edgelist(n, h, t, W, S, w) if wmax else O.tile_edgelist(n, h, t, W, S)
+
+
+def upload(ctx, g, weighted=False):
+    return ctx.graph_from_arrays(g.n, g.deg, W=g.W, S=g.S, csr_edges=g.cols,
+                                 csr_weights=g.cw if weighted else None, tile_heads=g.sh, tile_tails=g.st,
+                                 tile_weights=g.sw if weighted else None, tile_offsets=g.soff)
+
+
+@pytest.mark.parametrize("n,m,W,S", [(7, 9, 2, 1), (8, 20, 3, 2), (511, 1500, 12, 4), (512, 2048, 64, 2),
+                                     (2049, 9000, 100, 3), (8191, 40000, 512, 4), (8193, 200000, 1000, 8),
+                                     (270_001, 600_000, 1024, 16), (300_000, 4_000_000, 4096, 16)])
+def test_bfs(quiet, n, m, W, S):
+    g = random_graph(n, m, W, S, n)
+    gg = upload(quiet, g)
+    try:
+        for src in sorted({0, 1, n // 2, n - 1}):
+            print(f"case: small bfs n={n} m={m} W={W} src={src}", flush=True)
+            lv, pa, st = gg.bfs(src)
+            ref = O.bfs_levels(g.n, g.deg, g.cols, src)
+            assert np.array_equal(lv, ref), np.flatnonzero(lv != ref)[:10]
+            assert O.check_parents(g.n, g.deg, g.cols, src, lv, pa) == 0
+            _, _, tr = O.bfs_hybrid(g, src, 20)
+            assert np.array_equal(st.trace(), tr), (st.trace(), tr)
+            assert st.reached == int((ref >= 0).sum())
+            assert st.edges_traversed == int(g.deg[ref >= 0].astype(np.uint64).sum())
+            assert st.total_ms > 0
+    finally:
+        gg.free()
+
+
+@pytest.mark.parametrize("n", [18, 600])
+def test_bfs_long_path(quiet, n):
+    """More levels than the ring of level records (16) and than the trace (512)."""
+    g = O.tile_edgelist(n, np.arange(n - 1, dtype=np.uint32), np.arange(1, n, dtype=np.uint32), 16, 2)
+    gg = upload(quiet, g)
+    try:
+        print(f"case: small bfs path of {n}", flush=True)
+        lv, pa, st = gg.bfs(0)
+        assert np.array_equal(lv, np.arange(n))
+        assert np.array_equal(pa, np.maximum(np.arange(n) - 1, 0))
+        assert st.steps == min(n, G.MAX_STEPS) and st.reached == n and st.edges_traversed == n - 1
+    finally:
+        gg.free()
+
+
+@pytest.mark.parametrize("n,m,W,S,wmax", [(7, 9, 2, 1, 1), (513, 3000, 12, 4, 255), (8193, 200000, 1000, 8, 255),
+                                          (8193, 200000, 512, 8, 1 << 20), (270_001, 2_000_000, 1024, 16, 255)])
+def test_sssp(quiet, n, m, W, S, wmax):
+    g = random_graph(n, m, W, S, n + 1, wmax)
+    gg = upload(quiet, g, weighted=True)
+    try:
+        for src in sorted({0, n // 2, n - 1}):
+            print(f"case: small sssp n={n} m={m} W={W} wmax={wmax} src={src}", flush=True)
+            d, _ = gg.sssp(src)
+            ref = O.sssp_dijkstra(g.n, g.deg, g.cols, g.cw, src)
+            assert np.array_equal(d, ref), np.flatnonzero(d != ref)[:10]
+    finally:
+        gg.free()
