@@ -92,6 +92,7 @@ int gphi_open(const gphi_opts *opts, gphi_ctx **out)
 	ctx->ev_ok = true;
 	for (auto &ev : ctx->ev)
 		if (hipEventCreate(&ev) != hipSuccess) ctx->ev_ok = false;
+	gphi::out_context_opened();
 	*out = ctx;
 	return GPHI_OK;
 }
@@ -108,11 +109,13 @@ void gphi_close(gphi_ctx *ctx)
 {
 	if (!ctx) return;
 	(void)hipSetDevice(ctx->device);
+	if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
 	if (ctx->ev_ok)
 		for (auto &ev : ctx->ev) (void)hipEventDestroy(ev);
 	if (ctx->h_ctrl) (void)hipHostFree(ctx->h_ctrl);
 	if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
 	delete ctx;
+	gphi::out_context_closed();
 }
 
 const char *gphi_last_error(gphi_ctx *ctx)
@@ -252,6 +255,8 @@ void gphi_graph_free(gphi_graph *g)
 	if (!g) return;
 	std::lock_guard<std::mutex> lk(g->ctx->mu);
 	(void)hipSetDevice(g->ctx->device);
+	// a call may return before the last launches behind its results have run
+	(void)hipStreamSynchronize(g->ctx->stream);
 	gphi::free_graph_device(g);
 	delete g;
 }

@@ -1216,12 +1216,12 @@ int BatchRun::step(const uint32_t *srcs, uint32_t k)
 	return GPHI_OK;
 }
 
-// Levels of the given slots (n bytes each, 255 unreached) into host rows.
-int BatchRun::copy_rows(const uint32_t *slots, uint32_t ns, uint8_t *const *rows)
+// Levels of the given slots into host rows; no level is above the number of
+// levels expanded.
+template <class T>
+int BatchRun::copy_rows(const uint32_t *slots, uint32_t ns, T *const *rows)
 {
 	gphi_ctx *ctx = gr->ctx;
-	const DevGraph &G = gr->g;
-	hipStream_t s = ctx->stream;
 	u64 which[4] = {0, 0, 0, 0};
 	for (uint32_t i = 0; i < ns; ++i) {
 		if (slots[i] >= used) return set_error(ctx, GPHI_E_ARG, "slot %u is not in use", slots[i]);
@@ -1229,11 +1229,10 @@ int BatchRun::copy_rows(const uint32_t *slots, uint32_t ns, uint8_t *const *rows
 	}
 	int rc = finalize_rows(gr, nw, which);
 	if (rc) return rc;
-	for (uint32_t i = 0; i < ns; ++i)
-		GPHI_HIP(ctx, hipMemcpyAsync(rows[i], gr->b_level + (size_t)slots[i] * G.n_pad, G.n, hipMemcpyDeviceToHost, s));
-	GPHI_HIP(ctx, hipStreamSynchronize(s));
-	return GPHI_OK;
+	return out_batch_rows(gr, slots, levels, ns, rows);
 }
+template int BatchRun::copy_rows(const uint32_t *, uint32_t, uint8_t *const *);
+template int BatchRun::copy_rows(const uint32_t *, uint32_t, int32_t *const *);
 
 int run_bfs_batch(gphi_graph *gr, const uint32_t *srcs, uint32_t k, uint8_t *levels, gphi_stats *st)
 {
@@ -1254,12 +1253,13 @@ int run_bfs_batch(gphi_graph *gr, const uint32_t *srcs, uint32_t k, uint8_t *lev
 		st->edges_traversed = run.pairs[1];
 	}
 	if (levels) {
-		hipStream_t s = ctx->stream;
-		u64 which[4] = {0, 0, 0, 0};
-		for (uint32_t i = 0; i < k; ++i) which[i / 64] |= 1ull << (i % 64);
-		if ((rc = finalize_rows(gr, run.nw, which))) return rc;
-		GPHI_HIP(ctx, hipMemcpy2DAsync(levels, G.n, gr->b_level, G.n_pad, G.n, k, hipMemcpyDeviceToHost, s));
-		GPHI_HIP(ctx, hipStreamSynchronize(s));
+		uint32_t slots[kBatchMaxSources];
+		uint8_t *rows[kBatchMaxSources];
+		for (uint32_t i = 0; i < k; ++i) {
+			slots[i] = i;
+			rows[i] = levels + (size_t)i * G.n;
+		}
+		if ((rc = run.copy_rows(slots, k, rows))) return rc;
 	}
 	return GPHI_OK;
 }

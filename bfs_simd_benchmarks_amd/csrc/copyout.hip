@@ -1,0 +1,481 @@
+// copyout.hip -- results from HBM to the caller's host arrays.
+//
+// A hipMemcpy into pageable memory goes through the runtime's own staging
+// buffer and one host thread: 134 MB of levels took 13 ms (10 GB/s) and 1 MB
+// 0.4 ms, where the link carries 56 GB/s.  Here a kernel writes each piece of
+// the results into a slot of pinned memory, as narrow as the values allow,
+// and host threads turn finished slots into the caller's arrays while the
+// next ones cross the link:
+//
+//   levels  : 4 bits per level below 15 (every level of a shallow traversal),
+//             else 8, as level + 1 with 0 for unreached; widened by the host.
+//             The host's first touch of the array then sets the pace (about
+//             100 GB/s over 8 threads), not the link.
+//   others  : 4-byte words as they are
+//
+// A slot is finished when the flag beside it holds its sequence number: a
+// one-thread kernel stores it behind the kernel that filled the slot, and the
+// host sees it 5 us sooner than an event or a stream synchronization.
+//
+// Reference: the results stay in host memory there (apps/bfs_simd/bfs.cpp:
+// 753-963); this is the copy that takes their place.
+#include <hip/hip_runtime.h>
+
+#include <emmintrin.h>
+#include <sched.h>
+
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <mutex>
+#include <system_error>
+#include <thread>
+
+#include "internal.h"
+
+namespace gphi {
+
+namespace {
+
+constexpr size_t kSlotBytes = 2u << 20;
+constexpr uint32_t kSlots = 8;
+constexpr uint32_t kParts = 8;         // pieces of a slot the host threads take
+constexpr uint32_t kMaxHelpers = 7;    // host threads beside the caller's
+constexpr uint64_t kHelperBytes = 2u << 20;  // a helper per this much output (starting one takes about 20 us)
+constexpr unsigned kFillGrid = 256;    // blocks that fill a slot: enough to keep the link busy
+
+__global__ void slot_done_kernel(unsigned long long *flag, unsigned long long seq)
+{
+	__hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// four levels as bytes, each + 1 modulo 256 (255, unreached, becomes 0)
+__device__ __forceinline__ uint32_t inc_bytes(uint32_t x)
+{
+	return ((x & 0x7F7F7F7Fu) + 0x01010101u) ^ (x & 0x80808080u);
+}
+
+// the low nibbles of four bytes, in 16 bits
+__device__ __forceinline__ uint32_t squeeze(uint32_t x)
+{
+	x &= 0x0F0F0F0Fu;
+	x = (x | (x >> 4)) & 0x00FF00FFu;
+	return (x | (x >> 8)) & 0xFFFFu;
+}
+
+// 32 values of one row from element v (a multiple of 32) as level + 1 bytes
+struct WordLevels {  // int32 levels, valid where state is not 0
+	const int32_t *level;
+	const uint8_t *state;
+	__device__ __forceinline__ void load(uint32_t, uint32_t v, uint32_t (&x)[8]) const
+	{
+		const uint4 *l = reinterpret_cast<const uint4 *>(level + v);
+		const uint4 *s = reinterpret_cast<const uint4 *>(state + v);
+		const uint4 sa = s[0], sb = s[1];
+		const uint32_t st[8] = {sa.x, sa.y, sa.z, sa.w, sb.x, sb.y, sb.z, sb.w};
+#pragma unroll
+		for (int i = 0; i < 8; ++i) {
+			const uint4 q = l[i];
+			const uint32_t b[4] = {q.x, q.y, q.z, q.w};
+			x[i] = 0;
+#pragma unroll
+			for (int k = 0; k < 4; ++k)
+				x[i] |= ((st[i] >> (8 * k)) & 0xFFu ? (b[k] + 1u) & 0xFFu : 0u) << (8 * k);
+		}
+	}
+};
+struct ByteLevels {  // uint8 levels, 255 unreached; row r is row slot[r] of the array
+	const uint8_t *level;
+	uint32_t pitch;
+	uint8_t slot[kBatchMaxSources];
+	__device__ __forceinline__ void load(uint32_t row, uint32_t v, uint32_t (&x)[8]) const
+	{
+		const uint4 *p = reinterpret_cast<const uint4 *>(level + (uint64_t)slot[row] * pitch + v);
+		const uint4 a = p[0], b = p[1];
+		x[0] = a.x, x[1] = a.y, x[2] = a.z, x[3] = a.w, x[4] = b.x, x[5] = b.y, x[6] = b.z, x[7] = b.w;
+#pragma unroll
+		for (int i = 0; i < 8; ++i) x[i] = inc_bytes(x[i]);
+	}
+};
+
+// elements [first, first + count) of the rows laid end to end (rowlen each, a
+// multiple of 32), 32 per lane; kBits per element
+template <int kBits, class Src>
+__global__ __launch_bounds__(kBlock) void fill_levels_kernel(Src src, uint64_t first, uint64_t count, uint32_t rowlen,
+                                                             uint4 *__restrict__ out)
+{
+	for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < count / 32; i += (uint64_t)gridDim.x * kBlock) {
+		const uint64_t e = first + i * 32;
+		const uint32_t row = (uint32_t)(e / rowlen), v = (uint32_t)(e % rowlen);
+		uint32_t x[8];
+		src.load(row, v, x);
+		if (kBits == 4) {
+			out[i] = make_uint4(squeeze(x[0]) | squeeze(x[1]) << 16, squeeze(x[2]) | squeeze(x[3]) << 16,
+			                    squeeze(x[4]) | squeeze(x[5]) << 16, squeeze(x[6]) | squeeze(x[7]) << 16);
+		} else {
+			out[2 * i] = make_uint4(x[0], x[1], x[2], x[3]);
+			out[2 * i + 1] = make_uint4(x[4], x[5], x[6], x[7]);
+		}
+	}
+}
+
+// 4-byte words, 4 per lane; with a state array, -1 where it is 0
+__global__ __launch_bounds__(kBlock) void fill_words_kernel(const uint4 *__restrict__ src,
+                                                            const uint32_t *__restrict__ state, uint64_t first,
+                                                            uint64_t count, uint4 *__restrict__ out)
+{
+	for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < (count + 3) / 4;
+	     i += (uint64_t)gridDim.x * kBlock) {
+		uint4 x = src[first / 4 + i];
+		if (state) {
+			const uint32_t s = state[first / 4 + i];
+			if (!(s & 0xFFu)) x.x = ~0u;
+			if (!(s & 0xFF00u)) x.y = ~0u;
+			if (!(s & 0xFF0000u)) x.z = ~0u;
+			if (!(s & 0xFF000000u)) x.w = ~0u;
+		}
+		out[i] = x;
+	}
+}
+
+// rows of a vertex-major array (kSsspBatchMax words per vertex): a slot holds
+// the rows' values of `count` vertices from `first`, row by row; a lane per
+// vertex, so its reads share cache lines and a wavefront's writes of a row are
+// consecutive
+__global__ __launch_bounds__(kBlock) void fill_vertex_rows_kernel(const uint32_t *__restrict__ src, uint32_t k,
+                                                                  uint32_t first, uint32_t count,
+                                                                  uint32_t *__restrict__ out)
+{
+	for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < count; i += gridDim.x * kBlock) {
+		const uint4 *p = reinterpret_cast<const uint4 *>(src + (uint64_t)(first + i) * kSsspBatchMax);
+#pragma unroll
+		for (uint32_t q = 0; q < kSsspBatchMax / 4; ++q) {
+			if (4 * q >= k) break;
+			const uint4 x = p[q];
+			const uint32_t b[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+			for (uint32_t j = 0; j < 4; ++j)
+				if (4 * q + j < k) out[(4 * q + j) * count + i] = b[j];
+		}
+	}
+}
+
+// The host's widening of packed levels: element i of p (kBits each, level + 1)
+// to dst, for count elements from an even element.
+template <int kBits>
+void widen(const uint8_t *p, uint64_t i, uint64_t count, uint8_t *dst)
+{
+	const __m128i one = _mm_set1_epi8(1), low = _mm_set1_epi8(15);
+	uint64_t k = 0;
+	if (kBits == 4) {
+		const uint8_t *q = p + i / 2;
+		for (; k + 32 <= count; k += 32) {
+			const __m128i x = _mm_loadu_si128(reinterpret_cast<const __m128i *>(q + k / 2));
+			const __m128i a = _mm_and_si128(x, low), b = _mm_and_si128(_mm_srli_epi16(x, 4), low);
+			_mm_storeu_si128(reinterpret_cast<__m128i *>(dst + k), _mm_sub_epi8(_mm_unpacklo_epi8(a, b), one));
+			_mm_storeu_si128(reinterpret_cast<__m128i *>(dst + k + 16), _mm_sub_epi8(_mm_unpackhi_epi8(a, b), one));
+		}
+		for (; k < count; ++k) dst[k] = (uint8_t)(((q[k / 2] >> (4 * (k & 1))) & 15) - 1);
+	} else {
+		const uint8_t *q = p + i;
+		for (; k + 16 <= count; k += 16)
+			_mm_storeu_si128(reinterpret_cast<__m128i *>(dst + k),
+			                 _mm_sub_epi8(_mm_loadu_si128(reinterpret_cast<const __m128i *>(q + k)), one));
+		for (; k < count; ++k) dst[k] = (uint8_t)(q[k] - 1);
+	}
+}
+
+inline void widen16(__m128i x, int32_t *dst)  // 16 bytes to 16 words, each - 1
+{
+	const __m128i zero = _mm_setzero_si128(), one = _mm_set1_epi32(1);
+	const __m128i a = _mm_unpacklo_epi8(x, zero), b = _mm_unpackhi_epi8(x, zero);
+	__m128i *o = reinterpret_cast<__m128i *>(dst);
+	_mm_storeu_si128(o, _mm_sub_epi32(_mm_unpacklo_epi16(a, zero), one));
+	_mm_storeu_si128(o + 1, _mm_sub_epi32(_mm_unpackhi_epi16(a, zero), one));
+	_mm_storeu_si128(o + 2, _mm_sub_epi32(_mm_unpacklo_epi16(b, zero), one));
+	_mm_storeu_si128(o + 3, _mm_sub_epi32(_mm_unpackhi_epi16(b, zero), one));
+}
+
+template <int kBits>
+void widen(const uint8_t *p, uint64_t i, uint64_t count, int32_t *dst)
+{
+	const __m128i low = _mm_set1_epi8(15);
+	uint64_t k = 0;
+	if (kBits == 4) {
+		const uint8_t *q = p + i / 2;
+		for (; k + 32 <= count; k += 32) {
+			const __m128i x = _mm_loadu_si128(reinterpret_cast<const __m128i *>(q + k / 2));
+			const __m128i a = _mm_and_si128(x, low), b = _mm_and_si128(_mm_srli_epi16(x, 4), low);
+			widen16(_mm_unpacklo_epi8(a, b), dst + k);
+			widen16(_mm_unpackhi_epi8(a, b), dst + k + 16);
+		}
+		for (; k < count; ++k) dst[k] = (int32_t)((q[k / 2] >> (4 * (k & 1))) & 15) - 1;
+	} else {
+		const uint8_t *q = p + i;
+		for (; k + 16 <= count; k += 16) widen16(_mm_loadu_si128(reinterpret_cast<const __m128i *>(q + k)), dst + k);
+		for (; k < count; ++k) dst[k] = (int32_t)q[k] - 1;
+	}
+}
+
+// Pinned slots, leased for one copy-out.  Making a ring takes 0.3 ms (one
+// slot) to 1 ms (kSlots), which would be paid on every context's first call,
+// so finished copy-outs leave theirs for the next: up to kIdleRings of each
+// size stay with the process while it has a context, and none after that.
+struct Ring {
+	uint8_t *mem = nullptr;      // the slots, then their flags, a line apart
+	uint32_t slots = 0;
+	unsigned long long seq = 0;  // sequence number of the slot filled last
+};
+constexpr size_t kIdleRings = 4;
+std::mutex g_ring_mu;  // guards the three below
+Ring g_idle[2][kIdleRings];
+uint32_t g_idle_count[2] = {0, 0};
+uint32_t g_contexts = 0;
+
+int lease_ring(gphi_ctx *ctx, bool one, Ring *out)
+{
+	{
+		std::lock_guard<std::mutex> lk(g_ring_mu);
+		uint32_t &c = g_idle_count[one];
+		if (c) {
+			*out = g_idle[one][--c];
+			return GPHI_OK;
+		}
+	}
+	const uint32_t slots = one ? 1 : kSlots;
+	const hipError_t e = hipHostMalloc((void **)&out->mem, slots * (kSlotBytes + 128), hipHostMallocPortable);
+	if (e != hipSuccess) {
+		out->mem = nullptr;
+		return set_error(ctx, GPHI_E_OOM, "pinned staging of %u slots: %s", slots, hipGetErrorString(e));
+	}
+	memset(out->mem + slots * kSlotBytes, 0, slots * 128);
+	out->slots = slots;
+	return GPHI_OK;
+}
+
+void return_ring(bool one, const Ring &r)
+{
+	{
+		std::lock_guard<std::mutex> lk(g_ring_mu);
+		if (g_idle_count[one] < kIdleRings) {
+			g_idle[one][g_idle_count[one]++] = r;
+			return;
+		}
+	}
+	(void)hipHostFree(r.mem);
+}
+
+uint32_t helper_count(uint64_t nslots, uint64_t out_bytes)
+{
+	uint64_t t = std::min<uint64_t>(kMaxHelpers, out_bytes / kHelperBytes);
+	if (nslots <= 1 && out_bytes < 4 * kHelperBytes) t = 0;
+	if (t) {
+		cpu_set_t set;
+		const int cpus = sched_getaffinity(0, sizeof set, &set) == 0 ? CPU_COUNT(&set) : 1;
+		t = std::min<uint64_t>(t, (uint64_t)std::max(cpus - 1, 0));
+	}
+	return (uint32_t)t;
+}
+
+// fill(slot number, slot) enqueues the kernel that fills a slot; take(slot
+// number, part, slot) turns part 0..kParts-1 of a filled slot into output, on
+// any thread.  Returns when every part has been taken.
+template <class Fill, class Take>
+int stream_out(gphi_ctx *ctx, uint64_t nslots, uint64_t out_bytes, Fill fill, Take take)
+{
+	if (nslots == 0) return GPHI_OK;
+	const bool one = nslots == 1;
+	Ring ring;
+	int rc = lease_ring(ctx, one, &ring);
+	if (rc) return rc;
+	const uint32_t R = ring.slots;
+	hipStream_t s = ctx->stream;
+	uint8_t *mem = ring.mem;
+	auto flag = [&](uint64_t i) {
+		return reinterpret_cast<unsigned long long *>(mem + R * kSlotBytes + (i % R) * 128);
+	};
+	auto slot = [&](uint64_t i) { return mem + (i % R) * kSlotBytes; };
+	const unsigned long long seq0 = ring.seq + 1;  // slot i is filled when its flag is seq0 + i
+	ring.seq += nslots;
+	std::atomic<uint64_t> next{0}, ready{0};
+	std::atomic<uint32_t> taken[kSlots];
+	for (auto &x : taken) x.store(0);
+	std::atomic<bool> stop{false};
+	const uint64_t all = nslots * kParts;
+	// takes the next part; waits (or not) until its slot is filled
+	auto take_parts = [&](bool wait) {
+		for (;;) {
+			uint64_t p = next.load(std::memory_order_relaxed);
+			if (p >= all || stop.load(std::memory_order_relaxed)) return;
+			if (ready.load(std::memory_order_acquire) <= p / kParts) {
+				if (!wait) return;
+				_mm_pause();
+				continue;
+			}
+			if (!next.compare_exchange_weak(p, p + 1, std::memory_order_relaxed)) continue;
+			take(p / kParts, (uint32_t)(p % kParts), (const uint8_t *)slot(p / kParts));
+			taken[p / kParts % R].fetch_add(1, std::memory_order_release);
+		}
+	};
+	std::thread helpers[kMaxHelpers];
+	uint32_t nh = 0;
+	uint64_t issued = 0, spin = 0;
+	auto issue = [&] {
+		// a slot is filled again once its last contents were taken
+		while (issued < nslots &&
+		       (issued < R || taken[issued % R].load(std::memory_order_acquire) == issued / R * kParts)) {
+			fill(issued, slot(issued));
+			slot_done_kernel<<<1, 1, 0, s>>>(flag(issued), seq0 + issued);
+			++issued;
+		}
+	};
+	issue();
+	const uint32_t want = helper_count(nslots, out_bytes);
+	try {
+		for (; nh < want; ++nh) helpers[nh] = std::thread(take_parts, true);
+	} catch (const std::system_error &) {
+		// fewer helpers: the calling thread takes every part that is left
+	}
+	while (ready.load(std::memory_order_relaxed) < nslots) {
+		const uint64_t r = ready.load(std::memory_order_relaxed);
+		if (r < issued && __atomic_load_n(flag(r), __ATOMIC_ACQUIRE) >= seq0 + r) {
+			ready.store(r + 1, std::memory_order_release);
+			spin = 0;
+		} else if (++spin % 4096 == 0) {
+			const hipError_t e = hipStreamQuery(s);
+			if (e != hipSuccess && e != hipErrorNotReady) {
+				rc = hip_fail(ctx, e, "copy-out", __FILE__, __LINE__);
+				break;
+			}
+		}
+		issue();
+		if (nh == 0) take_parts(false);
+		_mm_pause();
+	}
+	if (rc) stop.store(true);
+	take_parts(true);
+	for (uint32_t i = 0; i < nh; ++i) helpers[i].join();
+	if (rc) {
+		// the device failed with fills under way: the ring is not used again
+		return rc;
+	}
+	return_ring(one, ring);
+	GPHI_HIP(ctx, hipGetLastError());
+	return GPHI_OK;
+}
+
+// part `part` of kParts of `count` elements, cut at multiples of 64
+inline void part_range(uint64_t count, uint32_t part, uint64_t *lo, uint64_t *hi)
+{
+	const uint64_t per = (count / kParts + 63) / 64 * 64 + 64;
+	*lo = std::min(count, part * per);
+	*hi = std::min(count, *lo + per);
+	if (part == kParts - 1) *hi = count;
+}
+
+unsigned fill_grid(uint64_t lanes) { return (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(kFillGrid, (lanes + kBlock - 1) / kBlock)); }
+
+// nrows rows of n levels each into rows[i]; every level is below 2^kBits - 1
+template <int kBits, class Src, class T>
+int out_level_rows(gphi_ctx *ctx, Src src, uint32_t n, uint32_t nrows, T *const *rows)
+{
+	const uint32_t rowlen = (n + 31) / 32 * 32;
+	const uint64_t total = (uint64_t)rowlen * nrows, per = kSlotBytes * 8 / kBits;
+	const uint64_t nslots = (total + per - 1) / per;
+	hipStream_t s = ctx->stream;
+	return stream_out(
+	    ctx, nslots, (uint64_t)n * nrows * sizeof(T),
+	    [&](uint64_t i, uint8_t *slot) {
+		    const uint64_t count = std::min(per, total - i * per);
+		    fill_levels_kernel<kBits><<<fill_grid(count / 32), kBlock, 0, s>>>(src, i * per, count, rowlen,
+		                                                                       reinterpret_cast<uint4 *>(slot));
+	    },
+	    [&](uint64_t i, uint32_t part, const uint8_t *slot) {
+		    uint64_t lo, hi;
+		    part_range(std::min(per, total - i * per), part, &lo, &hi);
+		    while (lo < hi) {  // the stretch of one row at a time
+			    const uint64_t e = i * per + lo;
+			    const uint32_t row = (uint32_t)(e / rowlen), v = (uint32_t)(e % rowlen);
+			    const uint64_t len = std::min<uint64_t>(hi - lo, rowlen - v);
+			    if (v < n) widen<kBits>(slot, lo, std::min<uint64_t>(len, n - v), rows[row] + v);
+			    lo += len;
+		    }
+	    });
+}
+
+}  // namespace
+
+int out_words(gphi_ctx *ctx, const void *dev, const uint8_t *state, uint32_t n, void *dst)
+{
+	const uint64_t per = kSlotBytes / 4, nslots = ((uint64_t)n + per - 1) / per;
+	hipStream_t s = ctx->stream;
+	return stream_out(
+	    ctx, nslots, (uint64_t)n * 4,
+	    [&](uint64_t i, uint8_t *slot) {
+		    const uint64_t count = std::min<uint64_t>(per, n - i * per);
+		    fill_words_kernel<<<fill_grid(count / 4 + 1), kBlock, 0, s>>>(
+		        static_cast<const uint4 *>(dev), reinterpret_cast<const uint32_t *>(state), i * per, count,
+		        reinterpret_cast<uint4 *>(slot));
+	    },
+	    [&](uint64_t i, uint32_t part, const uint8_t *slot) {
+		    uint64_t lo, hi;
+		    part_range(std::min<uint64_t>(per, n - i * per), part, &lo, &hi);
+		    if (lo < hi) memcpy(static_cast<uint8_t *>(dst) + (i * per + lo) * 4, slot + lo * 4, (hi - lo) * 4);
+	    });
+}
+
+int out_bfs_levels(gphi_graph *gr, uint32_t deepest, int32_t *levels)
+{
+	const WordLevels src{gr->level, gr->flag};
+	if (deepest <= 14) return out_level_rows<4>(gr->ctx, src, gr->g.n, 1, &levels);
+	if (deepest <= 254) return out_level_rows<8>(gr->ctx, src, gr->g.n, 1, &levels);
+	return out_words(gr->ctx, gr->level, gr->flag, gr->g.n, levels);
+}
+
+template <class T>
+int out_batch_rows(gphi_graph *gr, const uint32_t *slots, uint32_t deepest, uint32_t nrows, T *const *rows)
+{
+	ByteLevels src{gr->b_level, gr->g.n_pad, {}};
+	for (uint32_t i = 0; i < nrows; ++i) src.slot[i] = (uint8_t)slots[i];
+	if (deepest <= 14) return out_level_rows<4>(gr->ctx, src, gr->g.n, nrows, rows);
+	return out_level_rows<8>(gr->ctx, src, gr->g.n, nrows, rows);
+}
+template int out_batch_rows(gphi_graph *, const uint32_t *, uint32_t, uint32_t, uint8_t *const *);
+template int out_batch_rows(gphi_graph *, const uint32_t *, uint32_t, uint32_t, int32_t *const *);
+
+int out_sssp_rows(gphi_graph *gr, uint32_t k, uint32_t *const *rows)
+{
+	gphi_ctx *ctx = gr->ctx;
+	const uint32_t n = gr->g.n;
+	const uint32_t per = (uint32_t)(kSlotBytes / 4 / k) / 64 * 64;  // vertices per slot
+	const uint64_t nslots = ((uint64_t)n + per - 1) / per;
+	hipStream_t s = ctx->stream;
+	return stream_out(
+	    ctx, nslots, (uint64_t)n * k * 4,
+	    [&](uint64_t i, uint8_t *slot) {
+		    const uint32_t first = (uint32_t)(i * per), count = std::min(per, n - first);
+		    fill_vertex_rows_kernel<<<fill_grid(count), kBlock, 0, s>>>(gr->sb_dist, k, first, count,
+		                                                                reinterpret_cast<uint32_t *>(slot));
+	    },
+	    [&](uint64_t i, uint32_t part, const uint8_t *slot) {
+		    const uint32_t first = (uint32_t)(i * per), count = std::min(per, n - first);
+		    for (uint32_t r = part; r < k; r += kParts)
+			    if (rows[r]) memcpy(rows[r] + first, slot + (size_t)r * count * 4, (size_t)count * 4);
+	    });
+}
+
+void out_context_opened()
+{
+	std::lock_guard<std::mutex> lk(g_ring_mu);
+	++g_contexts;
+}
+
+void out_context_closed()
+{
+	std::lock_guard<std::mutex> lk(g_ring_mu);
+	if (--g_contexts) return;
+	for (int k = 0; k < 2; ++k)
+		while (g_idle_count[k]) (void)hipHostFree(g_idle[k][--g_idle_count[k]].mem);
+}
+
+}  // namespace gphi

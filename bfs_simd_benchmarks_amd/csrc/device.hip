@@ -1278,7 +1278,7 @@ static float ev_ms(hipEvent_t a, hipEvent_t b)
 }
 
 template <bool kBfs>
-static int frontier_loop(gphi_graph *gr, uint32_t src, gphi_stats *st)
+static int frontier_loop(gphi_graph *gr, uint32_t src, gphi_stats *st, uint32_t *steps_out)
 {
 	gphi_ctx *ctx = gr->ctx;
 	DevGraph &G = gr->g;
@@ -1291,14 +1291,14 @@ static int frontier_loop(gphi_graph *gr, uint32_t src, gphi_stats *st)
 	// total time from two events; per-level events only with level timing on
 	const bool total_timing = st != nullptr && ctx->ev_ok;
 	const bool timing = total_timing && ctx->level_timing;
-	if (!timing && small_graph(G, kBfs)) return small_level_loop<kBfs>(gr, src, st);
+	if (!timing && small_graph(G, kBfs)) return small_level_loop<kBfs>(gr, src, st, steps_out);
 	constexpr uint32_t kEvEnd = 3 * GPHI_MAX_STEPS + 3;  // end of the last group (no level timing)
 	if (total_timing) GPHI_HIP(ctx, hipEventRecord(ev[0], s));
 
 	// state initialisation (the reference's untimed set-up, bfs.cpp:771-797).
 	// BFS levels and parents are written for reached vertices only and never
-	// read during the traversal: the -1 of unreached ones is filled in by
-	// bfs_finalize_kernel when they are copied out.
+	// read during the traversal: the -1 of unreached ones is filled in when
+	// they are copied out.
 	if (!kBfs) fill_u32_kernel<<<grid_for(G.n_pad, kBlock, 4096), kBlock, 0, s>>>(gr->dist, G.n_pad, INT_MAX);
 	{
 		const uint64_t items = std::max<uint64_t>({G.n_pad / 16, G.n_words, G.side, kLiveCntBytes / 4});
@@ -1376,6 +1376,7 @@ static int frontier_loop(gphi_graph *gr, uint32_t src, gphi_stats *st)
 		if (enq > G.n + 2 + kLevelGroup) return set_error(ctx, GPHI_E_STATE, "frontier loop did not terminate");
 	}
 	const uint32_t steps = hc->level;  // frontiers expanded
+	if (steps_out) *steps_out = steps;
 	if (st) {
 		const uint32_t ns = std::min<uint32_t>(steps, GPHI_MAX_STEPS);
 		std::vector<uint4> tr(ns);
@@ -1442,19 +1443,6 @@ void launch_frontier_update_driven(gphi_graph *gr, uint32_t threshold)
 	                                            nullptr);
 }
 
-// level and parent -1 for the vertices a BFS did not reach (state 0; every
-// reached vertex ends in kVisited)
-__global__ __launch_bounds__(kBlock) void bfs_finalize_kernel(uint32_t n, const uint8_t *__restrict__ state,
-                                                              int32_t *__restrict__ level,
-                                                              int32_t *__restrict__ parent)
-{
-	for (uint32_t v = blockIdx.x * kBlock + threadIdx.x; v < n; v += gridDim.x * kBlock)
-		if (state[v] == 0) {
-			if (level) level[v] = -1;
-			if (parent) parent[v] = -1;
-		}
-}
-
 int run_bfs(gphi_graph *gr, uint32_t src, int32_t *levels, int32_t *parents, gphi_stats *st)
 {
 	gphi_ctx *ctx = gr->ctx;
@@ -1463,18 +1451,15 @@ int run_bfs(gphi_graph *gr, uint32_t src, int32_t *levels, int32_t *parents, gph
 	int rc = ensure_state(gr);
 	if (rc) return rc;
 	if (st) memset(st, 0, sizeof(*st));
-	if ((rc = frontier_loop<true>(gr, src, st))) return rc;
-	hipStream_t s = ctx->stream;
-	if (levels || parents)
-		bfs_finalize_kernel<<<grid_for(G.n, kBlock, 8192), kBlock, 0, s>>>(
-		    G.n, gr->flag, levels ? gr->level : nullptr, parents ? gr->parent : nullptr);
-	if (levels) GPHI_HIP(ctx, hipMemcpyAsync(levels, gr->level, (size_t)G.n * 4, hipMemcpyDeviceToHost, s));
-	if (parents) GPHI_HIP(ctx, hipMemcpyAsync(parents, gr->parent, (size_t)G.n * 4, hipMemcpyDeviceToHost, s));
-	GPHI_HIP(ctx, hipStreamSynchronize(s));
+	uint32_t steps = 0;
+	if ((rc = frontier_loop<true>(gr, src, st, &steps))) return rc;
+	// levels and parents were written for reached vertices only (state not 0)
+	if (levels && (rc = out_bfs_levels(gr, steps, levels))) return rc;
+	if (parents && (rc = out_words(ctx, gr->parent, gr->flag, G.n, parents))) return rc;
 	return GPHI_OK;
 }
 
-int bfs_level_loop(gphi_graph *gr, uint32_t src, gphi_stats *st) { return frontier_loop<true>(gr, src, st); }
+int bfs_level_loop(gphi_graph *gr, uint32_t src, gphi_stats *st) { return frontier_loop<true>(gr, src, st, nullptr); }
 
 uint32_t live_list_capacity(uint64_t nchunks) { return live_list_cap(nchunks); }
 
@@ -1488,10 +1473,8 @@ int run_sssp(gphi_graph *gr, uint32_t src, uint32_t *dist, gphi_stats *st)
 	if (rc) return rc;
 	if (!gr->dist && (rc = dmalloc(ctx, (void **)&gr->dist, (size_t)G.n_pad * 4, nullptr))) return rc;
 	if (st) memset(st, 0, sizeof(*st));
-	if ((rc = frontier_loop<false>(gr, src, st))) return rc;
-	if (dist)
-		GPHI_HIP(ctx, hipMemcpyAsync(dist, gr->dist, (size_t)G.n * 4, hipMemcpyDeviceToHost, ctx->stream));
-	GPHI_HIP(ctx, hipStreamSynchronize(ctx->stream));
+	if ((rc = frontier_loop<false>(gr, src, st, nullptr))) return rc;
+	if (dist && (rc = out_words(ctx, gr->dist, nullptr, G.n, dist))) return rc;
 	if (st) {
 		// reached = vertices with a finite distance (a vertex may be expanded
 		// several times by a label-correcting sweep, so the trace overcounts)
@@ -1753,7 +1736,7 @@ int run_pagerank(gphi_graph *gr, uint32_t iters, float damping, float init, floa
 	}
 	GPHI_HIP(ctx, hipGetLastError());
 	if (ctx->ev_ok) GPHI_HIP(ctx, hipEventRecord(ctx->ev[1], s));
-	if (rank) GPHI_HIP(ctx, hipMemcpyAsync(rank, gr->rank, (size_t)G.n * 4, hipMemcpyDeviceToHost, s));
+	if (rank && (rc = out_words(ctx, gr->rank, nullptr, G.n, rank))) return rc;
 	GPHI_HIP(ctx, hipStreamSynchronize(s));
 	if (ms) *ms = ctx->ev_ok ? ev_ms(ctx->ev[0], ctx->ev[1]) : 0.f;
 	return GPHI_OK;
@@ -1882,7 +1865,7 @@ int run_bellman_ford(gphi_graph *gr, uint32_t src, uint32_t max_sweeps, uint32_t
 	(void)hipFree(counts);
 	if (err) return err;
 	if (ctx->ev_ok) GPHI_HIP(ctx, hipEventRecord(ctx->ev[1], s));
-	if (dist) GPHI_HIP(ctx, hipMemcpyAsync(dist, gr->dist, (size_t)G.n * 4, hipMemcpyDeviceToHost, s));
+	if (dist && (rc = out_words(ctx, gr->dist, nullptr, G.n, dist))) return rc;
 	GPHI_HIP(ctx, hipStreamSynchronize(s));
 	if (ms) *ms = ctx->ev_ok ? ev_ms(ctx->ev[0], ctx->ev[1]) : 0.f;
 	if (sweeps_run) *sweeps_run = run;

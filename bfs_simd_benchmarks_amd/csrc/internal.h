@@ -302,9 +302,24 @@ int ensure_traversal_state(gphi_graph *gr);
 // traversal has ended, and st is filled in, when it returns
 bool small_graph(const DevGraph &G, bool bfs);
 template <bool kBfs>
-int small_level_loop(gphi_graph *gr, uint32_t src, gphi_stats *st);
+int small_level_loop(gphi_graph *gr, uint32_t src, gphi_stats *st, uint32_t *steps);
 // the BFS level loop of run_bfs on gr's state buffers (set up by the caller)
 int bfs_level_loop(gphi_graph *gr, uint32_t src, gphi_stats *st);
+
+// results to host arrays (copyout.hip); the caller's arrays are complete on return
+// n 4-byte words; with state bytes, -1 where the byte is 0
+int out_words(gphi_ctx *ctx, const void *dev, const uint8_t *state, uint32_t n, void *dst);
+// BFS levels of gr's last traversal, none above `deepest`
+int out_bfs_levels(gphi_graph *gr, uint32_t deepest, int32_t *levels);
+// rows of the multi-source levels, row i that of slot slots[i]; unreached is
+// 255 (uint8) or -1 (int32)
+template <class T>
+int out_batch_rows(gphi_graph *gr, const uint32_t *slots, uint32_t deepest, uint32_t nrows, T *const *rows);
+// the first k sources' distances of the multi-source SSSP (null rows are skipped)
+int out_sssp_rows(gphi_graph *gr, uint32_t k, uint32_t *const *rows);
+// gphi_open / gphi_close: the staging memory is freed with the last context
+void out_context_opened();
+void out_context_closed();
 // blocks of `block` threads of a kernel that fit the device at once, a multiple of the XCD count
 unsigned resident_grid(const void *kernel, unsigned block = kBlock);
 uint32_t live_list_capacity(uint64_t nchunks);  // entries of one XCD's live-chunk list
@@ -346,8 +361,9 @@ struct BatchRun {
 	int step(const uint32_t *srcs, uint32_t k);
 	int run_to_end(gphi_stats *st);  // the remaining levels, on the device
 	int read_totals();               // pairs[] from the device
-	// levels of the given slots into host rows of n bytes (255 unreached)
-	int copy_rows(const uint32_t *slots, uint32_t ns, uint8_t *const *rows);
+	// levels of the given slots into host rows of n (unreached: 255 in uint8 rows, -1 in int32 ones)
+	template <class T>
+	int copy_rows(const uint32_t *slots, uint32_t ns, T *const *rows);
 	int seed(const uint32_t *srcs, uint32_t k, uint32_t start_level);
 };
 

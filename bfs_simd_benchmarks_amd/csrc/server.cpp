@@ -154,14 +154,6 @@ uint64_t sssp_batch_bytes(const DevGraph &G)
 	       (G.coo_w8 ? 1 : 4) * G.m;
 }
 
-// BFS levels of a finished slot into the query's int32 buffer (-1 unreached)
-void store_levels(const std::vector<uint8_t> &row, uint32_t n, Query &q)
-{
-	if (!q.out) return;
-	int32_t *o = static_cast<int32_t *>(q.out);
-	for (uint32_t v = 0; v < n; ++v) o[v] = row[v] == 255 ? -1 : (int32_t)row[v];
-}
-
 void complete(gphi_server *S, const std::vector<std::shared_ptr<Query>> &qs, int rc, double t)
 {
 	{
@@ -184,7 +176,6 @@ void run_continuous(gphi_server *S, Lane *L, std::vector<std::shared_ptr<Query>>
 	std::vector<std::shared_ptr<Query>> slot_q;  // per slot
 	std::vector<uint8_t> finished;               // per slot: answered
 	std::vector<uint32_t> srcs;
-	std::vector<uint8_t> row(L->n);
 	uint64_t launch;
 	{
 		std::lock_guard<std::mutex> lk(S->mu);
@@ -199,6 +190,30 @@ void run_continuous(gphi_server *S, Lane *L, std::vector<std::shared_ptr<Query>>
 		slot_q.push_back(q);
 		finished.push_back(0);
 	}
+	// copies out and answers the unanswered slots that `which` picks
+	auto answer = [&](auto which) -> int {
+		uint32_t slots[kBatchMaxSources], ns = 0;
+		int32_t *rows[kBatchMaxSources];
+		std::vector<std::shared_ptr<Query>> qs;
+		for (uint32_t s = 0; s < run.used; ++s) {
+			if (finished[s] || !which(s)) continue;
+			if (slot_q[s]->out) {
+				slots[ns] = s;
+				rows[ns++] = static_cast<int32_t *>(slot_q[s]->out);
+			}
+			qs.push_back(slot_q[s]);
+		}
+		if (qs.empty()) return GPHI_OK;
+		if (ns) {
+			const int r = run.copy_rows(slots, ns, rows);
+			if (r) return r;
+		}
+		for (auto &q : qs) q->batch = run.used;
+		for (uint32_t s = 0; s < run.used; ++s)
+			if (!finished[s] && which(s)) finished[s] = 1;
+		complete(S, qs, GPHI_OK, now_us());
+		return GPHI_OK;
+	};
 	while (rc == GPHI_OK && !run.done) {
 		// arrivals join at this level boundary, up to the free slots
 		std::vector<std::shared_ptr<Query>> join;
@@ -226,32 +241,19 @@ void run_continuous(gphi_server *S, Lane *L, std::vector<std::shared_ptr<Query>>
 		}
 		rc = run.step(srcs.data(), (uint32_t)srcs.size());
 		if (rc) break;
-		// slots whose frontier emptied: copy their levels out and answer them
-		for (uint32_t s = 0; s < run.used && rc == GPHI_OK; ++s) {
-			if (finished[s] || ((run.live[s / 64] >> (s % 64)) & 1ull)) continue;
-			if (slot_q[s]->out) {
-				uint8_t *r = row.data();
-				rc = run.copy_rows(&s, 1, &r);
-				if (rc == GPHI_OK) store_levels(row, L->n, *slot_q[s]);
-			}
-			finished[s] = 1;
-			slot_q[s]->batch = run.used;
-			if (rc == GPHI_OK) complete(S, {slot_q[s]}, GPHI_OK, now_us());
-		}
+		// slots whose frontier emptied: copy their levels out together and
+		// answer them
+		rc = answer([&](uint32_t s) { return ((run.live[s / 64] >> (s % 64)) & 1ull) == 0; });
 	}
 	// the traversal ended (or failed): answer whatever is left
+	if (rc == GPHI_OK) rc = answer([](uint32_t) { return true; });
+	const double t1 = now_us();
 	std::vector<std::shared_ptr<Query>> rest;
 	for (uint32_t s = 0; s < slot_q.size(); ++s) {
 		if (finished[s]) continue;
-		if (rc == GPHI_OK && slot_q[s]->out) {
-			uint8_t *r = row.data();
-			rc = run.copy_rows(&s, 1, &r);
-			if (rc == GPHI_OK) store_levels(row, L->n, *slot_q[s]);
-		}
 		slot_q[s]->batch = (uint32_t)slot_q.size();
 		rest.push_back(slot_q[s]);
 	}
-	const double t1 = now_us();
 	if (!rest.empty()) complete(S, rest, rc, t1);
 	if (rc == GPHI_OK && !slot_q.empty()) ema(L->bfs_runs.t[RunCosts::size_class(slot_q.size())], t1 - t0);
 	std::lock_guard<std::mutex> lk(S->mu);

@@ -432,7 +432,7 @@ bool small_graph(const DevGraph &G, bool bfs)
 }
 
 template <bool kBfs>
-int small_level_loop(gphi_graph *gr, uint32_t src, gphi_stats *st)
+int small_level_loop(gphi_graph *gr, uint32_t src, gphi_stats *st, uint32_t *steps)
 {
 	gphi_ctx *ctx = gr->ctx;
 	const DevGraph &G = gr->g;
@@ -504,6 +504,7 @@ int small_level_loop(gphi_graph *gr, uint32_t src, gphi_stats *st)
 		if (p & 1ull) break;
 		seen = (uint32_t)(p >> 1) - 1;
 	}
+	if (steps) *steps = board->levels;
 	if (st) {
 		const uint32_t ns = std::min<uint32_t>(board->levels, GPHI_MAX_STEPS);
 		st->steps = ns;
@@ -520,7 +521,7 @@ int small_level_loop(gphi_graph *gr, uint32_t src, gphi_stats *st)
 	}
 	return GPHI_OK;
 }
-template int small_level_loop<true>(gphi_graph *, uint32_t, gphi_stats *);
-template int small_level_loop<false>(gphi_graph *, uint32_t, gphi_stats *);
+template int small_level_loop<true>(gphi_graph *, uint32_t, gphi_stats *, uint32_t *);
+template int small_level_loop<false>(gphi_graph *, uint32_t, gphi_stats *, uint32_t *);
 
 }  // namespace gphi

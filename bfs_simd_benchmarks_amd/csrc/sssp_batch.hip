@@ -275,13 +275,6 @@ __global__ __launch_bounds__(kBlock) void ssspb_pull_heavy_kernel(const StepCtrl
 	}
 }
 
-// row s (source s's distances) of the vertex-major array, for the copy-out
-__global__ void ssspb_row_kernel(uint32_t n, uint32_t s, const uint32_t *__restrict__ dist, uint32_t *__restrict__ row)
-{
-	for (uint32_t v = blockIdx.x * kBlock + threadIdx.x; v < n; v += gridDim.x * kBlock)
-		row[v] = dist[(uint64_t)v * kSsspBatchMax + s];
-}
-
 }  // namespace
 
 // The traversal state, in-edge arrays with their weights, and the distance
@@ -368,20 +361,7 @@ int run_sssp_batch(gphi_graph *gr, const uint32_t *srcs, uint32_t k, uint32_t *c
 	if (timing) GPHI_HIP(ctx, hipEventRecord(ctx->ev[1], s));
 	bool any_row = false;
 	for (uint32_t i = 0; rows && i < k; ++i) any_row |= rows[i] != nullptr;
-	if (any_row) {
-		if (!gr->dist && hipMalloc((void **)&gr->dist, (size_t)G.n_pad * 4) != hipSuccess) {
-			gr->dist = nullptr;
-			return set_error(ctx, GPHI_E_OOM, "hipMalloc of the distance row failed");
-		}
-		// row i through the n-entry staging row (stream order keeps each copy
-		// ahead of the next row's kernel)
-		for (uint32_t i = 0; i < k; ++i) {
-			if (!rows[i]) continue;
-			ssspb_row_kernel<<<std::min<unsigned>((G.n + kBlock - 1) / kBlock, 8192), kBlock, 0, s>>>(
-			    G.n, i, gr->sb_dist, gr->dist);
-			GPHI_HIP(ctx, hipMemcpyAsync(rows[i], gr->dist, (size_t)G.n * 4, hipMemcpyDeviceToHost, s));
-		}
-	}
+	if (any_row && (rc = out_sssp_rows(gr, k, rows))) return rc;
 	GPHI_HIP(ctx, hipStreamSynchronize(s));
 	if (st) {
 		st->steps = hc->level;
