@@ -18,12 +18,18 @@
 // the level of every (source, vertex) pair equals that source's own BFS level.
 // Levels are stored as uint8, source-major; 255 = unreached.
 //
-// The level loop runs on the device, as the single-source one does: every
-// kernel of a level reads the direction and sizes from the control block and
-// returns at once when it has nothing to do, so the host enqueues groups of
-// levels and reads the block back once per group.  A step marks the vertices
-// whose next mask it set in a bitmap, and the per-level update visits only
-// those (and the previous frontier), not every vertex.
+// The level loop is that of levels.h, four launches per level: on a dense step
+// the pull of the vertices with few in-edges, beside the queue of the sparse
+// sources below; the pull of the others' pieces, beside the push of the sparse
+// sources, or on a sparse step the CSR push; the update; and the advance of the
+// union frontier, beside the reduction of the live sources.  (A launch for each
+// part, and one for each of the steps and filter settings it serves, made
+// thirteen per level, sixteen levels for nine: 0.55 of the 2.2 ms of a 64-source
+// traversal of rmat22 and most of the 1.6 ms of 256 sources on 300007 vertices,
+// now 1.5 and 0.9.)  A
+// step marks the vertices whose next mask it set in a bitmap, and the
+// per-level update visits only those (and the previous frontier), not every
+// vertex.
 //
 // The union direction rule can make a dense step for sources whose own
 // frontiers are still small.  A pull finds such a source only far into a
@@ -45,7 +51,7 @@
 #include <cstring>
 #include <vector>
 
-#include "internal.h"
+#include "levels.h"
 
 namespace gphi {
 
@@ -54,29 +60,31 @@ namespace {
 constexpr uint8_t kUnreached = 255;
 typedef unsigned long long u64;
 
-// b_aux layout (uint32 words): sources to seed, their slots, per-slot start level
-constexpr uint32_t kAuxSrc = 0, kAuxSlot = kBatchMaxSources, kAuxStart = 2 * kBatchMaxSources;
-constexpr uint32_t kAuxWords = 3 * kBatchMaxSources;
 // the sources of a dense step whose frontiers have few out-edges (sparse
 // sources, batch_live_kernel); their mask sits beside the live mask
 constexpr uint32_t kSparseWord = 4;     // live[4..7]: the sparse sources of the next frontier
 constexpr uint32_t kSparseCount = 8;    // live[8]: entries of the sparse-source queue
-constexpr uint32_t kSparseOverflow = 9; // live[9]: the queue overflowed (the pulls take the sparse sources)
 // sparse: fewer than M / 1536 frontier out-edges (estimated).  Measured at
 // scale 25 over ratios 640..2560: 960..1920 is best, past it the pull keeps
 // scanning for the sources left to it, below it the push takes too many
 constexpr uint32_t kSparseRatio = 1536;
 constexpr uint32_t kCountSample = 16;   // after a dense step, every 16th block counts new vertices per source
 
-__device__ __forceinline__ bool test_bit32(const uint32_t *__restrict__ bm, uint32_t v)
-{
-	return (bm[v >> 5] >> (v & 31)) & 1u;
-}
-
 __device__ __forceinline__ void mark_touched(uint32_t *touched, uint32_t v)
 {
 	atomicOr(touched + (v >> 5), 1u << (v & 31));
 }
+
+// What the kernels of a traversal share.
+struct Batch : Frontier {
+	uint32_t n, npieces, light_blocks, heavy_blocks;
+	u64 m;
+	const uint32_t *row_off, *cols, *in_off, *in_src;
+	const uint2 *pieces;
+	u64 *front, *seen, *next, *live, *slots, *totals;
+	uint32_t *touched, *scount, *slot_start, *failed;
+	uint8_t *level8;
+};
 
 template <int NW>
 struct Mask {
@@ -152,37 +160,37 @@ __device__ __forceinline__ void or_front(const u64 *__restrict__ front, uint32_t
 // outside the frontier has front = 0, so the frontier bitmap is only a
 // filter: worth a 4-byte probe of a cache-resident word per edge when the
 // frontier is small (most heads then skip the gather), not when it is large.
-template <int NW, bool kFilter, uint32_t K>
-__device__ __forceinline__ void gather_fronts(const uint32_t (&h)[K], const uint32_t *__restrict__ cur,
+template <int NW, uint32_t K>
+__device__ __forceinline__ void gather_fronts(bool filter, const uint32_t (&h)[K], const uint32_t *__restrict__ cur,
                                               const u64 *__restrict__ front, u64 (&acc)[NW])
 {
 	uint32_t use = 0;
 #pragma unroll
-	for (uint32_t j = 0; j < K; ++j)
-		if (h[j] != 0xFFFFFFFFu && (!kFilter || test_bit32(cur, h[j]))) use |= 1u << j;
+	for (uint32_t j = 0; j < K; ++j) use |= (h[j] != 0xFFFFFFFFu ? 1u : 0u) << j;
+	if (filter) {  // uniform
+		uint32_t w[K];
+#pragma unroll
+		for (uint32_t j = 0; j < K; ++j) w[j] = (use >> j) & 1u ? cur[h[j] >> 5] : 0u;
+#pragma unroll
+		for (uint32_t j = 0; j < K; ++j)
+			if (!((w[j] >> (h[j] & 31)) & 1u)) use &= ~(1u << j);
+	}
 #pragma unroll
 	for (uint32_t j = 0; j < K; ++j)
 		if ((use >> j) & 1u) or_front<NW>(front, h[j], acc);
 }
 
-// The pull kernels of a dense step: a variant runs only on a dense step and
-// only if its filter setting is the one the step's union frontier calls for
-// (the frontier filter pays while the union frontier is under 1/8 of the
-// vertices).
-template <bool kFilter>
-__device__ __forceinline__ bool pull_runs(const StepCtrl *ctrl, uint32_t n)
-{
-	return !ctrl->done && ctrl->dir == 1 && (ctrl->fsize < n / 8) == kFilter;
-}
+// The frontier filter pays while the union frontier is under 1/8 of the
+// vertices.
+__device__ __forceinline__ bool filter_pays(const Step &st, uint32_t n) { return st.fsize < n / 8; }
 
 // The sources a dense step pulls: the live ones, less the sparse ones, which
-// batch_sparse_src_push_kernel pushes (unless their queue overflowed).
+// push_sparse_sources pushes.
 template <int NW>
 __device__ __forceinline__ void pulled_sources(const u64 *__restrict__ live, u64 (&pull)[NW])
 {
-	const bool pushed = live[kSparseOverflow] == 0;
 #pragma unroll
-	for (int i = 0; i < NW; ++i) pull[i] = live[i] & (pushed ? ~live[kSparseWord + i] : ~0ull);
+	for (int i = 0; i < NW; ++i) pull[i] = live[i] & ~live[kSparseWord + i];
 }
 
 // Pull for vertices with 1..kPullLight in-edges.  Each lane first reads its
@@ -204,20 +212,19 @@ static_assert(kLightGroup * kLightGroup == 64, "light pull: groups per wavefront
 
 __device__ __forceinline__ uint32_t shfl_u32(uint32_t x, uint32_t src) { return (uint32_t)__shfl((int)x, (int)src, 64); }
 
-template <int NW, bool kFilter>
-__global__ __launch_bounds__(kBlock) void batch_pull_light_kernel(
-    uint32_t n, const StepCtrl *__restrict__ ctrl, const uint32_t *__restrict__ in_off,
-    const uint32_t *__restrict__ in_src, const uint32_t *__restrict__ cur, const u64 *__restrict__ front,
-    const u64 *__restrict__ seen, const u64 *__restrict__ live, u64 *__restrict__ next,
-    uint32_t *__restrict__ touched)
+template <int NW>
+__device__ __forceinline__ void pull_light(const Batch &t, bool filter, uint32_t bid, uint32_t nb)
 {
-	if (!pull_runs<kFilter>(ctrl, n)) return;
+	const uint32_t n = t.n;
+	const uint32_t *__restrict__ in_off = t.in_off, *__restrict__ in_src = t.in_src, *__restrict__ cur = t.cur;
+	const u64 *__restrict__ front = t.front, *__restrict__ seen = t.seen;
+	u64 *__restrict__ next = t.next;
+	uint32_t *__restrict__ touched = t.touched;
 	u64 pull[NW];
-	pulled_sources<NW>(live, pull);
+	pulled_sources<NW>(t.live, pull);
 	const uint32_t lane = threadIdx.x & 63, g = lane % kLightGroup, grp = lane / kLightGroup;
-	// blocks walk the vertices kBlock at a time: a resident-size grid, so a
-	// launch on a step it has nothing to do in returns at once
-	for (uint32_t vb = blockIdx.x * kBlock; vb < n; vb += gridDim.x * kBlock) {
+	// blocks walk the vertices kBlock at a time
+	for (uint32_t vb = bid * kBlock; vb < n; vb += nb * kBlock) {
 	const uint32_t v0 = vb + (threadIdx.x & ~63u);  // first vertex of the wavefront
 	const uint32_t v = v0 + lane;
 	uint32_t e0 = 0, cnt = 0;
@@ -243,7 +250,7 @@ __global__ __launch_bounds__(kBlock) void batch_pull_light_kernel(
 		u64 acc[NW];
 #pragma unroll
 		for (int i = 0; i < NW; ++i) acc[i] = 0;
-		gather_fronts<NW, kFilter, kLightSlots>(h, cur, front, acc);
+		gather_fronts<NW, kLightSlots>(filter, h, cur, front, acc);
 		bool hit = false;
 #pragma unroll
 		for (int i = 0; i < NW; ++i) {
@@ -290,7 +297,7 @@ __global__ __launch_bounds__(kBlock) void batch_pull_light_kernel(
 			const uint32_t k = j * kLightGroup + g;
 			h1[j] = k < gcnt ? in_src[ge0 + k] : 0xFFFFFFFFu;
 		}
-		gather_fronts<NW, kFilter, kFirst>(h1, cur, front, acc);
+		gather_fronts<NW, kFirst>(filter, h1, cur, front, acc);
 #pragma unroll
 		for (int i = 0; i < NW; ++i)
 #pragma unroll
@@ -308,7 +315,7 @@ __global__ __launch_bounds__(kBlock) void batch_pull_light_kernel(
 			u64 acc2[NW];
 #pragma unroll
 			for (int i = 0; i < NW; ++i) acc2[i] = 0;
-			gather_fronts<NW, kFilter, kLightSlots - kFirst>(h2, cur, front, acc2);
+			gather_fronts<NW, kLightSlots - kFirst>(filter, h2, cur, front, acc2);
 #pragma unroll
 			for (int i = 0; i < NW; ++i) {
 #pragma unroll
@@ -342,26 +349,27 @@ __global__ __launch_bounds__(kBlock) void batch_pull_light_kernel(
 // Pull for vertices with more than kPullLight in-edges: a wavefront per piece
 // of up to kPullPiece in-edges, 64 · kUnroll edges between checks of the stop rule.
 // Pieces of one vertex combine with one atomicOr per word.  The sparse
-// sources (few frontier out-edges, batch_live_kernel) are left to
-// batch_sparse_src_push_kernel: a pull finds them only far into a vertex's
+// sources (few frontier out-edges, reduce_live) are left to
+// push_sparse_sources: a pull finds them only far into a vertex's
 // in-edges, so wanting them would keep most pieces scanning to their end.
-template <int NW, bool kFilter>
-__global__ __launch_bounds__(kBlock) void batch_pull_heavy_kernel(
-    uint32_t n, const StepCtrl *__restrict__ ctrl, uint32_t npieces, const uint2 *__restrict__ pieces,
-    const uint32_t *__restrict__ in_off, const uint32_t *__restrict__ in_src, const uint32_t *__restrict__ cur,
-    const u64 *__restrict__ front, const u64 *__restrict__ seen, const u64 *__restrict__ live, u64 *next,
-    uint32_t *touched)
+template <int NW>
+__device__ __forceinline__ void pull_heavy(const Batch &t, bool filter, uint32_t bid, uint32_t nb)
 {
-	if (!pull_runs<kFilter>(ctrl, n)) return;
+	const uint32_t *__restrict__ in_off = t.in_off, *__restrict__ in_src = t.in_src, *__restrict__ cur = t.cur;
+	const u64 *__restrict__ front = t.front, *__restrict__ seen = t.seen;
+	const uint2 *__restrict__ pieces = t.pieces;
+	const uint32_t npieces = t.npieces;
+	u64 *next = t.next;
+	uint32_t *touched = t.touched;
 	u64 pull[NW];
-	pulled_sources<NW>(live, pull);
+	pulled_sources<NW>(t.live, pull);
 	// loads in flight per lane between checks of the stop rule: a vertex stops
 	// as soon as every wanted source is found, so short rounds (64 or 128
 	// edges) beat deeper unrolling here
 	constexpr uint32_t kUnroll = NW == 1 ? 1 : 2;
 	const uint32_t lane = threadIdx.x & 63;
-	const uint32_t nwaves = (gridDim.x * kBlock) >> 6;
-	for (uint32_t p = (blockIdx.x * kBlock + threadIdx.x) >> 6; p < npieces; p += nwaves) {
+	const uint32_t nwaves = (nb * kBlock) >> 6;
+	for (uint32_t p = (bid * kBlock + threadIdx.x) >> 6; p < npieces; p += nwaves) {
 		const uint2 pc = pieces[p];
 		const uint32_t v = pc.x;
 		const uint32_t e1 = min(pc.y + kPullPiece, in_off[v + 1]);
@@ -393,7 +401,7 @@ __global__ __launch_bounds__(kBlock) void batch_pull_heavy_kernel(
 				const uint32_t j = off + 64 * kUnroll + u * 64 + lane;
 				hn[u] = j < cnt ? in_src[pc.y + j] : 0xFFFFFFFFu;
 			}
-			gather_fronts<NW, kFilter, kUnroll>(h, cur, front, acc);
+			gather_fronts<NW, kUnroll>(filter, h, cur, front, acc);
 			u64 miss = 0;
 #pragma unroll
 			for (int i = 0; i < NW; ++i) {
@@ -420,20 +428,18 @@ __global__ __launch_bounds__(kBlock) void batch_pull_heavy_kernel(
 // CSR push from the union-frontier queue (same edge partition as the
 // single-source push: tiles of kSparseTile edges starting at tile_lo)
 template <int NW>
-__global__ __launch_bounds__(kBlock) void batch_sparse_kernel(
-    const StepCtrl *__restrict__ ctrl, QueueBufs qb, const uint32_t *__restrict__ row_off,
-    const uint32_t *__restrict__ cols, const u64 *__restrict__ front, const u64 *__restrict__ seen, u64 *next,
-    uint32_t *touched)
+__device__ __forceinline__ void push_union(const Batch &t, uint32_t level, const Step &st)
 {
 	__shared__ uint32_t s_off[kSparseTile + 2];
 	__shared__ uint32_t s_u[kSparseTile + 2];
 	__shared__ uint32_t s_base[kSparseTile + 2];
-	if (ctrl->done || ctrl->dir != 0) return;
-	const uint32_t qsize = ctrl->qsize, qdeg = ctrl->fdeg;
-	const uint32_t par = ctrl->level & 1u;  // the half the frontier update wrote
-	const uint32_t *__restrict__ queue = qb.queue + par * qb.qstride;
-	const uint32_t *__restrict__ qoff = qb.qoff + par * qb.qstride;
-	const uint32_t *__restrict__ tile_lo = qb.tile_lo + par * qb.tstride;
+	const uint32_t *__restrict__ row_off = t.row_off, *__restrict__ cols = t.cols;
+	const u64 *__restrict__ front = t.front, *__restrict__ seen = t.seen;
+	const uint32_t qsize = st.qsize, qdeg = st.fdeg;
+	const uint32_t par = level & 1u;  // the half the advance wrote
+	const uint32_t *__restrict__ queue = t.qb.queue + par * t.qb.qstride;
+	const uint32_t *__restrict__ qoff = t.qb.qoff + par * t.qb.qstride;
+	const uint32_t *__restrict__ tile_lo = t.qb.tile_lo + par * t.qb.tstride;
 	const uint32_t ntile = (qdeg + kSparseTile - 1) / kSparseTile;
 	for (uint32_t k = blockIdx.x; k < ntile; k += gridDim.x) {
 		const uint32_t lo = tile_lo[k];
@@ -459,7 +465,7 @@ __global__ __launch_bounds__(kBlock) void batch_sparse_kernel(
 			}
 			const uint32_t u = s_u[a];
 			const uint32_t v = cols[s_base[a] + (e - s_off[a])];
-			push_mask<NW>(load_mask<NW>(front, u), v, seen, next, touched);
+			push_mask<NW>(load_mask<NW>(front, u), v, seen, t.next, t.touched);
 		}
 		__syncthreads();
 	}
@@ -477,26 +483,28 @@ __global__ __launch_bounds__(kBlock) void batch_sparse_kernel(
 // advance into one of kLiveSlots slots and add the new pairs (and their
 // out-degrees) to the totals.
 //
-// Two launch shapes, each returning at once on the other's steps: after a
-// dense step (kSpan = false) a block per kBlock vertices, since the pulls
-// touch most vertices and independent blocks hide their latency best; after a
-// sparse step (kSpan = true) a block per kUpdateSpan vertices, which reads
-// their touched and frontier words in one round into LDS and then walks
-// them, so that a step touching few vertices costs one load round per block,
-// not one per kBlock vertices.
-constexpr uint32_t kUpdateSpan = 4096;  // vertices per block after a sparse step (divides N_pad)
+// Two shapes: a block per kBlock vertices (kSpan = false) after a dense step
+// or a push along many edges, which touch most vertices, since independent
+// blocks hide their latency best; a block per kUpdateSpan vertices (kSpan =
+// true) after a push along few, which reads their touched and frontier words
+// in one round into LDS and then walks them, so that a step touching few
+// vertices costs one load round per block, not one per kBlock vertices.
+constexpr uint32_t kUpdateSpan = 4096;  // vertices per block of the span shape (divides N_pad)
+constexpr uint32_t kSpanShare = 64;     // few: under a 64th as many edges as vertices (a half: 5% slower on rmat22)
 constexpr uint32_t kLiveSlots = 64;
 constexpr uint32_t kLiveStride = 16;  // u64 words per slot (one 128-byte line)
 constexpr uint32_t kSlotPairs = 8;    // slot words 8, 9: new pairs and their out-degrees
 
 template <int NW, bool kSpan>
-__global__ __launch_bounds__(kBlock) void batch_update_kernel(
-    uint32_t n, uint32_t n_pitch, uint32_t next_level, StepCtrl *ctrl, const uint32_t *__restrict__ cur,
-    uint32_t *__restrict__ touched, u64 *__restrict__ front, u64 *__restrict__ seen, u64 *__restrict__ next,
-    uint8_t *__restrict__ level, uint8_t *__restrict__ flag, const uint32_t *__restrict__ slot_start,
-    const uint32_t *__restrict__ deg, u64 *slots, uint32_t *scount)
+__device__ __forceinline__ void update_block(const Batch &t, uint32_t next_level)
 {
-	if (ctrl->done || (ctrl->dir == 0) != kSpan) return;
+	const uint32_t n = t.n, n_pitch = t.n_pad;
+	const uint32_t *__restrict__ cur = t.cur, *__restrict__ slot_start = t.slot_start, *__restrict__ deg = t.deg;
+	uint32_t *__restrict__ touched = t.touched;
+	u64 *__restrict__ front = t.front, *__restrict__ seen = t.seen, *__restrict__ next = t.next;
+	uint8_t *__restrict__ level = t.level8, *__restrict__ flag = t.flag;
+	u64 *slots = t.slots;
+	uint32_t *scount = t.scount;
 	__shared__ uint32_t s_words[kSpan ? 2 * kUpdateSpan / 32 : 1];  // touched words, then frontier words
 	__shared__ u64 s_or[kBlock / 64][NW];
 	__shared__ u64 s_cnt[kBlock / 64][2];
@@ -555,8 +563,8 @@ __global__ __launch_bounds__(kBlock) void batch_update_kernel(
 			tw = in ? touched[v >> 5] : 0u;
 			cw = in ? cur[v >> 5] : 0u;
 		}
-		const bool t = (tw >> (v & 31)) & 1u, c = (cw >> (v & 31)) & 1u;
-		if (!__ballot(t || c)) continue;  // uniform
+		const bool hit = (tw >> (v & 31)) & 1u, c = (cw >> (v & 31)) & 1u;
+		if (!__ballot(hit || c)) continue;  // uniform
 		if (!kSpan && (v & 31) == 0 && tw) touched[v >> 5] = 0u;  // clear for the next step
 		u64 nw[NW];
 		u64 anyn = 0;
@@ -564,7 +572,7 @@ __global__ __launch_bounds__(kBlock) void batch_update_kernel(
 		for (int j = 0; j < NW; ++j) {
 			nw[j] = 0;
 			const uint64_t idx = (uint64_t)v * NW + j;
-			if (t) {
+			if (hit) {
 				const u64 nx = next[idx];
 				const u64 sn = seen[idx];
 				nw[j] = nx & ~sn;
@@ -611,10 +619,9 @@ __global__ __launch_bounds__(kBlock) void batch_update_kernel(
 		for (int j = 0; j < NW; ++j) s_or[wid][j] = wor[j];
 		s_cnt[wid][0] = pairs;
 		s_cnt[wid][1] = pdeg;
-		// a level of 255 or more would read as unreached: the live kernel
-		// stops the traversal (no block of this launch may see done change,
-		// since every block of it reads done to decide whether to run)
-		if (over) ctrl->err = 1;
+		// a level of 255 or more would read as unreached: the advance stops
+		// the traversal
+		if (over) *t.failed = 1;
 	}
 	__syncthreads();
 	if (threadIdx.x < NW) {
@@ -660,14 +667,9 @@ __global__ __launch_bounds__(kBlock) void batch_update_kernel(
 // about kSparseRatio in-edges per vertex, so on a dense step the heavy pull
 // leaves them to a push from their frontier.  One wavefront.
 template <int NW>
-__global__ void batch_live_kernel(StepCtrl *ctrl, u64 *live, u64 *slots, u64 *sums, uint32_t *scount, u64 m)
+__device__ __forceinline__ void reduce_live(const Batch &t, uint32_t lane)
 {
-	if (ctrl->done) return;
-	if (ctrl->err) {  // the update met a level past 254: stop here
-		if (threadIdx.x == 0) ctrl->done = 1;
-		return;
-	}
-	const uint32_t lane = threadIdx.x;
+	u64 *live = t.live, *slots = t.slots;
 	u64 lv[NW];
 #pragma unroll
 	for (int i = 0; i < NW; ++i) {
@@ -677,13 +679,13 @@ __global__ void batch_live_kernel(StepCtrl *ctrl, u64 *live, u64 *slots, u64 *su
 		if (lane == 0) live[i] = lv[i];
 	}
 	// the step's new pairs and their out-degrees, into the totals
-	u64 *t = slots + (uint64_t)lane * kLiveStride + kSlotPairs;
-	const u64 p = wave_add(t[0]), d = wave_add(t[1]);
-	t[0] = 0;
-	t[1] = 0;
+	u64 *sp = slots + (uint64_t)lane * kLiveStride + kSlotPairs;
+	const u64 p = wave_add(sp[0]), d = wave_add(sp[1]);
+	sp[0] = 0;
+	sp[1] = 0;
 	if (lane == 0) {
-		sums[0] += p;
-		sums[1] += d;
+		t.totals[0] += p;
+		t.totals[1] += d;
 	}
 	// lane l: source i * 64 + l; its count summed over the slots (and cleared)
 	const double mean_deg = p ? (double)d / (double)p : 0.0;
@@ -692,18 +694,15 @@ __global__ void batch_live_kernel(StepCtrl *ctrl, u64 *live, u64 *slots, u64 *su
 		const uint32_t src = i * 64 + lane;
 		uint32_t c = 0;
 		for (uint32_t k = 0; k < kLiveSlots; ++k) {
-			uint32_t *q = scount + k * kBatchMaxSources + src;
+			uint32_t *q = t.scount + k * kBatchMaxSources + src;
 			c += *q;
 			*q = 0;
 		}
-		const bool sparse = ((lv[i] >> lane) & 1ull) && (double)c * mean_deg * kSparseRatio < (double)m;
-		const u64 sp = __ballot(sparse);
-		if (lane == 0) live[kSparseWord + i] = sp;
+		const bool sparse = ((lv[i] >> lane) & 1ull) && (double)c * mean_deg * kSparseRatio < (double)t.m;
+		const u64 sm = __ballot(sparse);
+		if (lane == 0) live[kSparseWord + i] = sm;
 	}
-	if (lane == 0) {
-		live[kSparseCount] = 0;
-		live[kSparseOverflow] = 0;
-	}
+	if (lane == 0) live[kSparseCount] = 0;
 }
 
 // inclusive prefix sum over the wavefront
@@ -720,21 +719,17 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x)
 
 // The queue of a dense step's sparse sources: an entry (vertex, chunk) per
 // kSparseTile out-edges of each vertex whose front mask holds a sparse
-// source, in the queue half of the step's parity (a dense step's frontier
-// update leaves that half unused).  Runs after the frontier update has set
-// the step's direction; nothing to do unless the step is dense and has
-// sparse sources.  A lane per vertex, a block-stride walk; live[kSparseCount]
-// counts the entries (cleared by the live kernel), and an entry past the
-// half's capacity sets live[kSparseOverflow], which hands the sparse sources
-// back to the pulls.
+// source, in the queue half of the step's parity (which only a sparse step
+// reads).  A half holds an entry per vertex and kSparseTile edges, so it
+// cannot overflow.  A lane per vertex, a block-stride walk;
+// live[kSparseCount] counts the entries (cleared by reduce_live).
 template <int NW>
-__global__ __launch_bounds__(kBlock) void batch_sparse_queue_kernel(uint32_t n, uint32_t n_pad,
-                                                                    const StepCtrl *__restrict__ ctrl, u64 *live,
-                                                                    const u64 *__restrict__ front,
-                                                                    const uint32_t *__restrict__ row_off,
-                                                                    QueueBufs qb)
+__device__ __forceinline__ void queue_sparse_sources(const Batch &t, uint32_t level, uint32_t bid, uint32_t nb)
 {
-	if (ctrl->done || ctrl->dir != 1) return;
+	const uint32_t n = t.n, n_pad = t.n_pad;
+	u64 *live = t.live;
+	const u64 *__restrict__ front = t.front;
+	const uint32_t *__restrict__ row_off = t.row_off;
 	u64 sp[NW], any = 0;
 #pragma unroll
 	for (int i = 0; i < NW; ++i) {
@@ -742,11 +737,11 @@ __global__ __launch_bounds__(kBlock) void batch_sparse_queue_kernel(uint32_t n, 
 		any |= sp[i];
 	}
 	if (!any) return;
-	const uint32_t par = ctrl->level & 1u;
-	uint32_t *__restrict__ queue = qb.queue + par * qb.qstride;
-	uint32_t *__restrict__ qchunk = qb.qoff + par * qb.qstride;
+	const uint32_t par = level & 1u;
+	uint32_t *__restrict__ queue = t.qb.queue + par * t.qb.qstride;
+	uint32_t *__restrict__ qchunk = t.qb.qoff + par * t.qb.qstride;
 	const uint32_t lane = threadIdx.x & 63;
-	for (uint32_t v = blockIdx.x * kBlock + threadIdx.x; v < n_pad; v += gridDim.x * kBlock) {
+	for (uint32_t v = bid * kBlock + threadIdx.x; v < n_pad; v += nb * kBlock) {
 		bool hit = false;
 		if (v < n) {
 #pragma unroll
@@ -759,10 +754,6 @@ __global__ __launch_bounds__(kBlock) void batch_sparse_queue_kernel(uint32_t n, 
 		u64 base = 0;
 		if (lane == 0) base = atomicAdd(live + kSparseCount, (u64)tot);
 		base = (u64)__shfl((long long)base, 0, 64);
-		if (base + tot > qb.qstride) {
-			if (lane == 0) live[kSparseOverflow] = 1;
-			continue;
-		}
 		for (uint32_t c = 0; c < nc; ++c) {
 			const uint32_t i = (uint32_t)base + incl - nc + c;
 			queue[i] = v;
@@ -773,15 +764,13 @@ __global__ __launch_bounds__(kBlock) void batch_sparse_queue_kernel(uint32_t n, 
 
 // The sparse sources of a dense step, pushed along the out-edges of their
 // frontier (the queue above): next[t] |= (front[h] & sparse) & ~seen[t].  A
-// wavefront per entry, after the pulls (the light pull stores next and the
-// touched words outright).
+// wavefront per entry, in the launch after the light pull's, which stores
+// next and the touched words outright.
 template <int NW>
-__global__ __launch_bounds__(kBlock) void batch_sparse_src_push_kernel(
-    const StepCtrl *__restrict__ ctrl, const u64 *__restrict__ live, QueueBufs qb,
-    const uint32_t *__restrict__ row_off, const uint32_t *__restrict__ cols, const u64 *__restrict__ front,
-    const u64 *__restrict__ seen, u64 *next, uint32_t *touched)
+__device__ __forceinline__ void push_sparse_sources(const Batch &t, uint32_t level, uint32_t bid, uint32_t nb)
 {
-	if (ctrl->done || ctrl->dir != 1 || live[kSparseOverflow]) return;
+	const u64 *__restrict__ live = t.live, *__restrict__ front = t.front, *__restrict__ seen = t.seen;
+	const uint32_t *__restrict__ row_off = t.row_off, *__restrict__ cols = t.cols;
 	Mask<NW> sp;
 	u64 any = 0;
 #pragma unroll
@@ -791,81 +780,145 @@ __global__ __launch_bounds__(kBlock) void batch_sparse_src_push_kernel(
 	}
 	if (!any) return;
 	const uint32_t cnt = (uint32_t)live[kSparseCount];
-	const uint32_t par = ctrl->level & 1u;
-	const uint32_t *__restrict__ queue = qb.queue + par * qb.qstride;
-	const uint32_t *__restrict__ qchunk = qb.qoff + par * qb.qstride;
+	const uint32_t par = level & 1u;
+	const uint32_t *__restrict__ queue = t.qb.queue + par * t.qb.qstride;
+	const uint32_t *__restrict__ qchunk = t.qb.qoff + par * t.qb.qstride;
 	const uint32_t lane = threadIdx.x & 63;
-	const uint32_t nwaves = (gridDim.x * kBlock) >> 6;
-	for (uint32_t q = (blockIdx.x * kBlock + threadIdx.x) >> 6; q < cnt; q += nwaves) {
+	const uint32_t nwaves = (nb * kBlock) >> 6;
+	for (uint32_t q = (bid * kBlock + threadIdx.x) >> 6; q < cnt; q += nwaves) {
 		const uint32_t h = queue[q];
 		const uint32_t e0 = row_off[h] + qchunk[q] * kSparseTile;
 		const uint32_t e1 = min(e0 + kSparseTile, row_off[h + 1]);
 		Mask<NW> f = load_mask<NW>(front, h);
 #pragma unroll
 		for (int i = 0; i < NW; ++i) f.w[i] &= sp.w[i];
-		for (uint32_t e = e0 + lane; e < e1; e += 64) push_mask<NW>(f, cols[e], seen, next, touched);
+		for (uint32_t e = e0 + lane; e < e1; e += 64) push_mask<NW>(f, cols[e], seen, t.next, t.touched);
 	}
 }
 
 // Sources joining the traversal (at its start, or between two levels): slot
-// s gets vertex v at level 0 relative to start_level; v enters the union
-// frontier of the next step through its state byte.  One block.
-__global__ void batch_seed_kernel(const uint32_t *__restrict__ aux, uint32_t count, uint32_t start_level,
-                                  uint32_t nw, uint32_t n_pitch, u64 *front, u64 *seen, uint8_t *level,
-                                  uint8_t *flag, u64 *live, uint32_t *slot_start, const uint32_t *__restrict__ deg,
-                                  u64 *sums)
+// first + i gets vertex src[i] at level 0 relative to start_level; the vertex
+// enters the union frontier of the next step through its state byte, and the
+// live mask, the totals and the source's vertex count through the slots the
+// update adds to.  One block.
+struct Seeds {
+	uint32_t src[kBatchMaxSources];
+};
+__global__ void batch_seed_kernel(Batch t, Seeds seeds, uint32_t first, uint32_t count, uint32_t start_level,
+                                  uint32_t nw)
 {
 	for (uint32_t i = threadIdx.x; i < count; i += blockDim.x) {
-		const uint32_t v = aux[kAuxSrc + i], s = aux[kAuxSlot + i];
+		const uint32_t v = seeds.src[i], s = first + i;
 		const u64 bit = 1ull << (s % 64);
-		atomicOr(front + (uint64_t)v * nw + s / 64, bit);
-		atomicOr(seen + (uint64_t)v * nw + s / 64, bit);
-		atomicOr(live + s / 64, bit);
-		level[(uint64_t)s * n_pitch + v] = 0;
-		slot_start[s] = start_level;
-		flag[v] = 1;
-		atomicAdd(sums, 1ull);
-		atomicAdd(sums + 1, (u64)deg[v]);
+		atomicOr(t.front + (uint64_t)v * nw + s / 64, bit);
+		atomicOr(t.seen + (uint64_t)v * nw + s / 64, bit);
+		atomicOr(t.slots + s / 64, bit);
+		atomicAdd(t.slots + kSlotPairs, 1ull);
+		atomicAdd(t.slots + kSlotPairs + 1, (u64)t.deg[v]);
+		atomicAdd(t.scount + s, 1u);
+		t.level8[(uint64_t)s * t.n_pad + v] = 0;
+		t.slot_start[s] = start_level;
+		t.flag[v] = 1;
 	}
 }
 
 // Per-traversal clears of the masks, state bytes, bitmaps, live words, slot
-// start levels and totals; the control block is set up for the first
-// frontier update (which opens level 0).
-__global__ __launch_bounds__(kBlock) void batch_clear_kernel(uint64_t mask_words, uint32_t n_pad, uint32_t n_words,
-                                                             u64 *front, u64 *seen, u64 *next, uint8_t *flag,
-                                                             uint32_t *cur, uint32_t *touched, u64 *live_all,
-                                                             uint32_t live_words, uint32_t *slot_start,
-                                                             u64 *sums, uint32_t *scount, StepCtrl *ctrl, bool clean)
+// start levels and totals; the level records are set up for the advance that
+// opens level 0 (that of the level before it, UINT32_MAX).
+__global__ __launch_bounds__(kBlock) void batch_clear_kernel(Batch t, uint64_t mask_words, uint32_t n_words,
+                                                             uint32_t live_words, bool clean)
 {
 	const uint64_t stride = (uint64_t)gridDim.x * kBlock;
 	const uint64_t i0 = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
 	// clean: the last traversal on these buffers ran to its end, which leaves
 	// front, next and the touched bitmap all zero (only seen keeps its bits)
 	for (uint64_t i = i0; i < mask_words; i += stride) {
-		seen[i] = 0;
+		t.seen[i] = 0;
 		if (!clean) {
-			front[i] = 0;
-			next[i] = 0;
+			t.front[i] = 0;
+			t.next[i] = 0;
 		}
 	}
-	for (uint64_t i = i0; i < n_pad / 16; i += stride) reinterpret_cast<uint4 *>(flag)[i] = make_uint4(0, 0, 0, 0);
+	for (uint64_t i = i0; i < t.n_pad / 16; i += stride) reinterpret_cast<uint4 *>(t.flag)[i] = make_uint4(0, 0, 0, 0);
 	for (uint64_t i = i0; i < n_words; i += stride) {
-		cur[i] = 0;
-		if (!clean) touched[i] = 0;
+		t.cur[i] = 0;
+		if (!clean) t.touched[i] = 0;
 	}
-	for (uint64_t i = i0; i < live_words; i += stride) live_all[i] = 0;
-	for (uint64_t i = i0; i < kBatchMaxSources; i += stride) slot_start[i] = 0;
-	for (uint64_t i = i0; i < kLiveSlots * kBatchMaxSources; i += stride) scount[i] = 0;
-	if (i0 < 2) sums[i0] = 0;
+	for (uint64_t i = i0; i < live_words; i += stride) t.live[i] = 0;
+	for (uint64_t i = i0; i < kBatchMaxSources; i += stride) t.slot_start[i] = 0;
+	for (uint64_t i = i0; i < kLiveSlots * kBatchMaxSources; i += stride) t.scount[i] = 0;
+	if (i0 < kLevelRing) {
+		LevelRec r = {};
+		if (i0 == UINT32_MAX % kLevelRing) r.fsize = 1;
+		t.rec[i0] = r;
+	}
+	if (i0 < 2) t.totals[i0] = 0;
 	if (i0 == 0) {
-		ctrl->level = UINT32_MAX;  // the first frontier update opens level 0
-		ctrl->done = 0;
-		ctrl->err = 0;
-		ctrl->dir = 0;
-		ctrl->reached = 0;
-		ctrl->traversed = 0;
+		*t.failed = 0;
+		t.board->t_begin = wall_clock64();
 	}
+}
+
+// ---- the four launches of a level ----
+
+template <int NW>
+__global__ __launch_bounds__(kBlock) void batch_light_kernel(Batch t, uint32_t level)
+{
+	const Step st = step_of(t, level);
+	if (blockIdx.x == 0 && threadIdx.x == 0) publish_level(t, level, st.fsize, st.fdeg, st.dense);
+	if (st.fsize == 0 || !st.dense) return;
+	if (blockIdx.x >= t.light_blocks)
+		queue_sparse_sources<NW>(t, level, blockIdx.x - t.light_blocks, gridDim.x - t.light_blocks);
+	else
+		pull_light<NW>(t, filter_pays(st, t.n), blockIdx.x, t.light_blocks);
+}
+
+// (the CSR push of a sparse step shares this launch and not the light pull's,
+// whose registers it would add to)
+template <int NW>
+__global__ __launch_bounds__(kBlock) void batch_heavy_kernel(Batch t, uint32_t level)
+{
+	const Step st = step_of(t, level);
+	if (st.fsize == 0) return;
+	if (!st.dense)
+		push_union<NW>(t, level, st);
+	else if (blockIdx.x >= t.heavy_blocks)
+		push_sparse_sources<NW>(t, level, blockIdx.x - t.heavy_blocks, gridDim.x - t.heavy_blocks);
+	else
+		pull_heavy<NW>(t, filter_pays(st, t.n), blockIdx.x, t.heavy_blocks);
+}
+
+template <int NW>
+__global__ __launch_bounds__(kBlock) void batch_update_kernel(Batch t, uint32_t level)
+{
+	const Step st = step_of(t, level);
+	if (st.fsize == 0) return;
+	if (!st.dense && st.fdeg < t.n / kSpanShare) {
+		if (blockIdx.x < t.n_pad / kUpdateSpan) update_block<NW, true>(t, level + 1);
+	} else {
+		update_block<NW, false>(t, level + 1);
+	}
+}
+
+// the advance of the union frontier, and in one more block the live sources
+template <int NW, uint32_t kThreads>
+__global__ __launch_bounds__(kThreads) void batch_advance_kernel(Batch t, uint32_t level)
+{
+	if (blockIdx.x + 1 < gridDim.x)
+		advance_block<false, kThreads>(t, level);
+	else if (rec_of(t, level)->fsize && threadIdx.x < 64)
+		reduce_live<NW>(t, threadIdx.x);
+}
+
+// what the host wants to know between two levels of a traversal it steps
+// through: whether the next frontier is empty, the live sources, an error
+__global__ void batch_report_kernel(Batch t, uint32_t level, uint32_t nw, u64 seq)
+{
+	LevelBoard *b = t.board;
+	const LevelRec *r = rec_of(t, level);
+	for (uint32_t i = 0; i < nw; ++i) b->live[i] = t.live[i];
+	b->err = *t.failed;
+	__hip_atomic_store(&b->step_seq, seq << 1 | (r->fsize == 0), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // level 255 for every (slot, vertex) pair of the given slots the traversal
@@ -897,70 +950,60 @@ float ev_ms(hipEvent_t a, hipEvent_t b)
 }
 
 constexpr unsigned kBatchSparseGrid = 2048;
-constexpr unsigned kBatchWalkGrid = 8192;  // blocks of the kernels that walk every vertex
-constexpr uint32_t kBatchLevelGroup = 8;  // levels enqueued per read-back of the control block
+constexpr unsigned kBatchWalkGrid = 8192;   // blocks of the light pull, which walks every vertex
+constexpr unsigned kBatchQueueGrid = 1024;  // blocks of the sparse sources' queue, beside it
 
-u64 *live_words(gphi_graph *gr) { return gr->b_live; }
-u64 *live_slots(gphi_graph *gr) { return gr->b_live + kLiveStride; }
-uint32_t *slot_starts(gphi_graph *gr) { return gr->b_aux + kAuxStart; }
-
-// The expansion of one level and its update: the CSR push (sparse step) or
-// the pulls (dense step) -- each kernel returns at once unless the control
-// block says it is its step -- then the update of the vertices the step
-// touched, then the live-source mask.
-template <int NW>
-void enqueue_expand(gphi_graph *gr)
+Batch make_batch(gphi_graph *gr)
 {
 	const DevGraph &G = gr->g;
-	hipStream_t s = gr->ctx->stream;
-	batch_sparse_kernel<NW><<<kBatchSparseGrid, kBlock, 0, s>>>(gr->ctrl, gr->queue_bufs(), G.row_off, G.cols,
-	                                                           gr->b_front, gr->b_seen, gr->b_next, gr->b_touch);
-	const unsigned lg = std::min<unsigned>(grid_n(G.n), kBatchWalkGrid);
-	const u64 *live = live_words(gr);
-	batch_pull_light_kernel<NW, true><<<lg, kBlock, 0, s>>>(G.n, gr->ctrl, gr->in_off, gr->in_src, gr->cur, gr->b_front,
-	                                                       gr->b_seen, live, gr->b_next, gr->b_touch);
-	batch_pull_light_kernel<NW, false><<<lg, kBlock, 0, s>>>(G.n, gr->ctrl, gr->in_off, gr->in_src, gr->cur, gr->b_front,
-	                                                        gr->b_seen, live, gr->b_next, gr->b_touch);
-	if (gr->npieces) {
-		const unsigned hg = std::min<uint32_t>((gr->npieces + 3) / 4, 16384);
-		batch_pull_heavy_kernel<NW, true><<<hg, kBlock, 0, s>>>(G.n, gr->ctrl, gr->npieces, gr->pieces, gr->in_off,
-		                                                       gr->in_src, gr->cur, gr->b_front, gr->b_seen, live,
-		                                                       gr->b_next, gr->b_touch);
-		batch_pull_heavy_kernel<NW, false><<<hg, kBlock, 0, s>>>(G.n, gr->ctrl, gr->npieces, gr->pieces, gr->in_off,
-		                                                        gr->in_src, gr->cur, gr->b_front, gr->b_seen, live,
-		                                                        gr->b_next, gr->b_touch);
-	}
-	batch_sparse_src_push_kernel<NW><<<kBatchSparseGrid, kBlock, 0, s>>>(gr->ctrl, live, gr->queue_bufs(), G.row_off,
-	                                                                   G.cols, gr->b_front, gr->b_seen, gr->b_next,
-	                                                                   gr->b_touch);
+	Batch t = {};
+	static_cast<Frontier &>(t) = make_frontier(gr, (uint32_t)G.m / gr->ctx->t_ratio);
+	t.n = G.n, t.m = G.m, t.npieces = gr->npieces;
+	t.row_off = G.row_off, t.cols = G.cols, t.in_off = gr->in_off, t.in_src = gr->in_src, t.pieces = gr->pieces;
+	t.front = gr->b_front, t.seen = gr->b_seen, t.next = gr->b_next;
+	t.live = gr->b_live, t.slots = gr->b_live + kLiveStride, t.totals = gr->b_sums;
+	t.touched = gr->b_touch, t.scount = gr->b_scount, t.slot_start = gr->b_aux, t.level8 = gr->b_level;
+	t.failed = gr->b_aux + kBatchMaxSources;
+	t.err = t.failed;
+	t.sums = t.totals;
+	t.light_blocks = std::min<unsigned>(grid_n(G.n), kBatchWalkGrid);
+	t.heavy_blocks = std::min<uint32_t>((gr->npieces + 3) / 4, 16384);
+	return t;
 }
 
 template <int NW>
-void enqueue_update(gphi_graph *gr, uint32_t next_level)
+void enqueue_expand(gphi_graph *gr, const Batch &t, uint32_t level)
 {
-	const DevGraph &G = gr->g;
 	hipStream_t s = gr->ctx->stream;
-	// after a dense step, a block per kBlock vertices; after a sparse one, a
-	// block per kUpdateSpan vertices (each launch returns at once on the
-	// other's steps)
-	batch_update_kernel<NW, false><<<grid_n(G.n), kBlock, 0, s>>>(
-	    G.n, G.n_pad, next_level, gr->ctrl, gr->cur, gr->b_touch, gr->b_front, gr->b_seen, gr->b_next, gr->b_level,
-	    gr->flag, slot_starts(gr), G.deg, live_slots(gr), gr->b_scount);
-	batch_update_kernel<NW, true><<<G.n_pad / kUpdateSpan, kBlock, 0, s>>>(
-	    G.n, G.n_pad, next_level, gr->ctrl, gr->cur, gr->b_touch, gr->b_front, gr->b_seen, gr->b_next, gr->b_level,
-	    gr->flag, slot_starts(gr), G.deg, live_slots(gr), gr->b_scount);
-	batch_live_kernel<NW><<<1, 64, 0, s>>>(gr->ctrl, live_words(gr), live_slots(gr), gr->b_sums, gr->b_scount,
-	                                       (u64)G.m);
+	const unsigned queue_blocks = std::min<unsigned>(grid_n(t.n_pad), kBatchQueueGrid);
+	batch_light_kernel<NW><<<t.light_blocks + queue_blocks, kBlock, 0, s>>>(t, level);
+	batch_heavy_kernel<NW><<<t.heavy_blocks + kBatchSparseGrid, kBlock, 0, s>>>(t, level);
+	batch_update_kernel<NW><<<std::max<unsigned>(grid_n(t.n), t.n_pad / kUpdateSpan), kBlock, 0, s>>>(t, level);
 }
 
-// the sparse-source queue of the next step (after the frontier update has
-// set its direction)
 template <int NW>
-void enqueue_sparse_queue(gphi_graph *gr)
+void enqueue_advance(gphi_graph *gr, const Batch &t, uint32_t level)
 {
-	const DevGraph &G = gr->g;
-	batch_sparse_queue_kernel<NW><<<std::min<unsigned>(grid_n(G.n_pad), kBatchWalkGrid), kBlock, 0, gr->ctx->stream>>>(
-	    G.n, G.n_pad, gr->ctrl, live_words(gr), gr->b_front, G.row_off, gr->queue_bufs());
+	hipStream_t s = gr->ctx->stream;
+	const unsigned nblk = advance_blocks(t.n_pad) + 1;
+	if (advance_threads(t.n_pad) == 256)
+		batch_advance_kernel<NW, 256><<<nblk, 256, 0, s>>>(t, level);
+	else
+		batch_advance_kernel<NW, 1024><<<nblk, 1024, 0, s>>>(t, level);
+}
+
+void enqueue_expand(gphi_graph *gr, uint32_t nw, const Batch &t, uint32_t level)
+{
+	if (nw == 1) enqueue_expand<1>(gr, t, level);
+	else if (nw == 2) enqueue_expand<2>(gr, t, level);
+	else enqueue_expand<4>(gr, t, level);
+}
+
+void enqueue_advance(gphi_graph *gr, uint32_t nw, const Batch &t, uint32_t level)
+{
+	if (nw == 1) enqueue_advance<1>(gr, t, level);
+	else if (nw == 2) enqueue_advance<2>(gr, t, level);
+	else enqueue_advance<4>(gr, t, level);
 }
 
 template <int NW>
@@ -978,30 +1021,6 @@ int finalize_rows(gphi_graph *gr, uint32_t nw, const u64 *which)
 	int rc = nw == 1 ? launch_finalize<1>(gr, which) : nw == 2 ? launch_finalize<2>(gr, which) : launch_finalize<4>(gr, which);
 	if (rc) return set_error(gr->ctx, rc, "batched BFS: finalize launch failed");
 	return GPHI_OK;
-}
-
-void enqueue_level(gphi_graph *gr, uint32_t nw, uint32_t next_level, bool expand_half)
-{
-	if (expand_half) {
-		if (nw == 1) enqueue_expand<1>(gr);
-		else if (nw == 2) enqueue_expand<2>(gr);
-		else enqueue_expand<4>(gr);
-	} else {
-		if (nw == 1) enqueue_update<1>(gr, next_level);
-		else if (nw == 2) enqueue_update<2>(gr, next_level);
-		else enqueue_update<4>(gr, next_level);
-	}
-}
-
-// the frontier update of the union frontier (mark / scan / emit of the
-// single-source loop), in its device-driven form: it opens the next level;
-// then the next step's sparse-source queue
-void enqueue_frontier(gphi_graph *gr, uint32_t nw)
-{
-	launch_frontier_update_driven(gr, (uint32_t)gr->g.m / gr->ctx->t_ratio);
-	if (nw == 1) enqueue_sparse_queue<1>(gr);
-	else if (nw == 2) enqueue_sparse_queue<2>(gr);
-	else enqueue_sparse_queue<4>(gr);
 }
 
 }  // namespace
@@ -1036,7 +1055,7 @@ int batch_prepare(gphi_graph *gr, uint32_t nw)
 	// the touched bitmap, then the per-source counts
 	if (e == hipSuccess)
 		e = hipMalloc((void **)&gr->b_touch, ((size_t)G.n_words + (size_t)kLiveSlots * kBatchMaxSources) * 4);
-	if (e == hipSuccess) e = hipMalloc((void **)&gr->b_aux, (size_t)kAuxWords * 4);
+	if (e == hipSuccess) e = hipMalloc((void **)&gr->b_aux, (size_t)(kBatchMaxSources + 1) * 4);
 	if (e != hipSuccess)
 		return set_error(ctx, GPHI_E_OOM, "batched BFS buffers (%zu MB): %s",
 		                 (3 * mb + (size_t)nw * 64 * G.n_pad) >> 20, hipGetErrorString(e));
@@ -1072,20 +1091,21 @@ int BatchRun::begin(gphi_graph *g, uint32_t capacity, const uint32_t *srcs, uint
 	// the buffers hold gr->batch_words >= nw words per vertex; a traversal runs
 	// at its own width nw (the masks are addressed with that pitch)
 	mask_words = (uint64_t)G.n_pad * nw;
-	const uint64_t items = std::max<uint64_t>({mask_words, G.n_pad / 16, G.n_words, kBatchMaxSources});
+	const uint64_t items = std::max<uint64_t>({mask_words, G.n_pad / 16, G.n_words, kBatchMaxSources, kLevelRing});
 	// the front and next masks and the touched bitmap are left all zero by a
 	// traversal that ran to its end; they need clearing only over words no
 	// such traversal has covered since the buffers were made
 	prev_clean = gr->batch_clean_words;
 	const bool clean = prev_clean >= mask_words;
 	gr->batch_clean_words = 0;  // until this traversal ends
+	const Batch t = make_batch(gr);
+	reset_board(ctx->h_board);
 	batch_clear_kernel<<<(unsigned)std::min<uint64_t>(grid_n(items), 16384), kBlock, 0, s>>>(
-	    mask_words, G.n_pad, G.n_words, gr->b_front, gr->b_seen, gr->b_next, gr->flag, gr->cur, gr->b_touch,
-	    gr->b_live, (1 + kLiveSlots) * kLiveStride, slot_starts(gr), gr->b_sums, gr->b_scount, gr->ctrl, clean);
+	    t, mask_words, G.n_words, (1 + kLiveSlots) * kLiveStride, clean);
 	GPHI_HIP(ctx, hipGetLastError());
 	if ((rc = seed(srcs, k, 0))) return rc;
-	// the first frontier update: the sources form the union frontier of level 0
-	enqueue_frontier(gr, nw);
+	// the sources form the union frontier of level 0
+	enqueue_advance(gr, nw, t, UINT32_MAX);
 	GPHI_HIP(ctx, hipGetLastError());
 	return GPHI_OK;
 }
@@ -1094,19 +1114,9 @@ int BatchRun::seed(const uint32_t *srcs, uint32_t k, uint32_t start_level)
 {
 	if (k == 0) return GPHI_OK;
 	gphi_ctx *ctx = gr->ctx;
-	const DevGraph &G = gr->g;
-	hipStream_t s = ctx->stream;
-	for (uint32_t i = 0; i < k; ++i) {
-		aux[kAuxSrc + i] = srcs[i];
-		aux[kAuxSlot + i] = used + i;
-	}
-	// aux is not written again before the stream is synchronized: every
-	// caller of seed synchronizes before its next seed
-	GPHI_HIP(ctx, hipMemcpyAsync(gr->b_aux + kAuxSrc, aux + kAuxSrc, (size_t)k * 4, hipMemcpyHostToDevice, s));
-	GPHI_HIP(ctx, hipMemcpyAsync(gr->b_aux + kAuxSlot, aux + kAuxSlot, (size_t)k * 4, hipMemcpyHostToDevice, s));
-	batch_seed_kernel<<<1, kBlock, 0, s>>>(gr->b_aux, k, start_level, nw, G.n_pad, gr->b_front, gr->b_seen,
-	                                        gr->b_level, gr->flag, live_words(gr), slot_starts(gr), G.deg,
-	                                        gr->b_sums);
+	Seeds seeds = {};
+	std::copy(srcs, srcs + k, seeds.src);
+	batch_seed_kernel<<<1, kBlock, 0, ctx->stream>>>(make_batch(gr), seeds, used, k, start_level, nw);
 	GPHI_HIP(ctx, hipGetLastError());
 	for (uint32_t i = 0; i < k; ++i) {
 		slot_src.push_back(srcs[i]);
@@ -1116,55 +1126,42 @@ int BatchRun::seed(const uint32_t *srcs, uint32_t k, uint32_t start_level)
 	return GPHI_OK;
 }
 
-// Runs levels on the device until the traversal ends, kBatchLevelGroup levels
-// per read-back of the control block (no admissions).
+// Runs levels until the traversal ends (no admissions).
 int BatchRun::run_to_end(gphi_stats *st)
 {
 	gphi_ctx *ctx = gr->ctx;
 	hipStream_t s = ctx->stream;
-	StepCtrl *hc = ctx->h_ctrl;
+	const LevelBoard *board = ctx->h_board;
 	hipEvent_t *ev = ctx->ev;
-	const bool total_timing = st != nullptr && ctx->ev_ok;
-	const bool timing = total_timing && ctx->level_timing;
-	constexpr uint32_t kEvEnd = 3 * GPHI_MAX_STEPS + 3;
+	const bool timing = st != nullptr && ctx->ev_ok && ctx->level_timing;
 	if (timing) GPHI_HIP(ctx, hipEventRecord(ev[1], s));
-	uint32_t enq = 0;
-	for (;;) {
-		for (uint32_t q = 0; q < kBatchLevelGroup; ++q, ++enq) {
-			const bool ev_step = timing && enq < GPHI_MAX_STEPS - 1;
-			enqueue_level(gr, nw, enq + 1, true);
-			if (ev_step) GPHI_HIP(ctx, hipEventRecord(ev[2 + 2 * enq], s));
-			enqueue_level(gr, nw, enq + 1, false);
-			enqueue_frontier(gr, nw);
-			if (ev_step) GPHI_HIP(ctx, hipEventRecord(ev[3 + 2 * enq], s));
-		}
-		GPHI_HIP(ctx, hipGetLastError());
-		if (total_timing && !timing) GPHI_HIP(ctx, hipEventRecord(ev[kEvEnd], s));
-		GPHI_HIP(ctx, hipMemcpyAsync(hc, gr->ctrl, sizeof(StepCtrl), hipMemcpyDeviceToHost, s));
-		GPHI_HIP(ctx, hipStreamSynchronize(s));
-		if (hc->err) return set_error(ctx, GPHI_E_RANGE, "a batched BFS deeper than 254 levels does not fit uint8 levels");
-		if (hc->done) break;
-		// every level ends the traversal, advances it, or (past level 254) stops it with err
-		if (enq > 256 + kBatchLevelGroup)
-			return set_error(ctx, GPHI_E_STATE, "batched traversal did not terminate");
-	}
-	levels = hc->level;
+	const Batch t = make_batch(gr);
+	const int rc = follow_levels(ctx, [&](uint32_t level) {
+		const bool ev_step = timing && level < GPHI_MAX_STEPS - 1;
+		enqueue_expand(gr, nw, t, level);
+		if (ev_step) GPHI_HIP(ctx, hipEventRecord(ev[2 + 2 * level], s));
+		enqueue_advance(gr, nw, t, level);
+		if (ev_step) GPHI_HIP(ctx, hipEventRecord(ev[3 + 2 * level], s));
+		return GPHI_OK;
+	});
+	if (rc) return rc;
+	if (board->err) return set_error(ctx, GPHI_E_RANGE, "a batched BFS deeper than 254 levels does not fit uint8 levels");
+	levels = board->levels;
 	done = true;
+	pairs[0] = board->reached;
+	pairs[1] = board->traversed;
 	gr->batch_clean_words = std::max(prev_clean, mask_words);
 	if (st) {
 		const uint32_t ns = std::min<uint32_t>(levels, GPHI_MAX_STEPS);
-		std::vector<uint4> tr(ns);
-		if (ns) {
-			GPHI_HIP(ctx, hipMemcpyAsync(tr.data(), gr->trace, ns * sizeof(uint4), hipMemcpyDeviceToHost, s));
-			GPHI_HIP(ctx, hipStreamSynchronize(s));
-		}
 		st->steps = ns;
 		for (uint32_t k = 0; k < ns; ++k) {
-			st->dir[k] = tr[k].x;
-			st->fsize[k] = tr[k].y;
-			st->fdeg[k] = tr[k].z;
+			st->dir[k] = board->trace[k].x;
+			st->fsize[k] = board->trace[k].y;
+			st->fdeg[k] = board->trace[k].z;
 		}
+		st->total_ms = board_ms(ctx);
 		if (timing) {
+			GPHI_HIP(ctx, hipStreamSynchronize(s));
 			st->init_ms = ev_ms(ev[0], ev[1]);
 			hipEvent_t prev = ev[1];
 			const uint32_t nt = std::min<uint32_t>(levels, GPHI_MAX_STEPS - 1);
@@ -1174,44 +1171,35 @@ int BatchRun::run_to_end(gphi_stats *st)
 				prev = ev[3 + 2 * q];
 			}
 			st->total_ms = nt ? ev_ms(ev[0], ev[1 + 2 * nt]) : st->init_ms;
-		} else {
-			st->total_ms = total_timing ? ev_ms(ev[0], ev[kEvEnd]) : 0.f;
 		}
 	}
-	return read_totals();
-}
-
-int BatchRun::read_totals()
-{
-	gphi_ctx *ctx = gr->ctx;
-	GPHI_HIP(ctx, hipMemcpyAsync(pairs, gr->b_sums, 16, hipMemcpyDeviceToHost, ctx->stream));
-	GPHI_HIP(ctx, hipStreamSynchronize(ctx->stream));
 	return GPHI_OK;
 }
 
 // One level, then the admission of k new sources (they join the union
-// frontier of the next level), then the frontier update; reads the control
-// block and the live-source mask back.
+// frontier of the next level), then the advance; the host waits for its
+// report of the live sources.
 int BatchRun::step(const uint32_t *srcs, uint32_t k)
 {
 	gphi_ctx *ctx = gr->ctx;
-	hipStream_t s = ctx->stream;
-	StepCtrl *hc = ctx->h_ctrl;
+	LevelBoard *board = ctx->h_board;
 	if (done) return set_error(ctx, GPHI_E_STATE, "the batched traversal has ended");
 	if (used + k > cap) return set_error(ctx, GPHI_E_ARG, "no free slot for %u more sources", k);
 	const uint32_t next_level = levels + 1;
-	enqueue_level(gr, nw, next_level, true);
-	enqueue_level(gr, nw, next_level, false);
+	const Batch t = make_batch(gr);
+	enqueue_expand(gr, nw, t, levels);
 	int rc = seed(srcs, k, next_level);
 	if (rc) return rc;
-	enqueue_frontier(gr, nw);
+	enqueue_advance(gr, nw, t, levels);
+	const unsigned long long seq = (board->step_seq >> 1) + 1;
+	batch_report_kernel<<<1, 1, 0, ctx->stream>>>(t, next_level, nw, seq);
 	GPHI_HIP(ctx, hipGetLastError());
-	GPHI_HIP(ctx, hipMemcpyAsync(hc, gr->ctrl, sizeof(StepCtrl), hipMemcpyDeviceToHost, s));
-	GPHI_HIP(ctx, hipMemcpyAsync(live, live_words(gr), (size_t)nw * 8, hipMemcpyDeviceToHost, s));
-	GPHI_HIP(ctx, hipStreamSynchronize(s));
-	if (hc->err) return set_error(ctx, GPHI_E_RANGE, "a batched BFS deeper than 254 levels does not fit uint8 levels");
+	unsigned long long p;
+	if ((rc = wait_progress(ctx, &board->step_seq, seq - 1, &p))) return rc;
+	if (board->err) return set_error(ctx, GPHI_E_RANGE, "a batched BFS deeper than 254 levels does not fit uint8 levels");
+	for (uint32_t i = 0; i < nw; ++i) live[i] = board->live[i];
 	levels = next_level;
-	done = hc->done != 0;
+	done = (p & 1ull) != 0;
 	if (done) gr->batch_clean_words = std::max(prev_clean, mask_words);
 	return GPHI_OK;
 }

@@ -38,9 +38,9 @@ namespace gphi {
 namespace {
 
 constexpr size_t kSlotBytes = 2u << 20;
-constexpr uint32_t kSlots = 8;
+constexpr uint32_t kSlots = 24;
 constexpr uint32_t kParts = 8;         // pieces of a slot the host threads take
-constexpr uint32_t kMaxHelpers = 7;    // host threads beside the caller's
+constexpr uint32_t kMaxHelpers = 11;   // host threads beside the caller's
 constexpr uint64_t kHelperBytes = 2u << 20;  // a helper per this much output (starting one takes about 20 us)
 constexpr unsigned kFillGrid = 256;    // blocks that fill a slot: enough to keep the link busy
 
@@ -226,7 +226,7 @@ struct Ring {
 	uint32_t slots = 0;
 	unsigned long long seq = 0;  // sequence number of the slot filled last
 };
-constexpr size_t kIdleRings = 4;
+constexpr size_t kIdleRings = 2;
 std::mutex g_ring_mu;  // guards the three below
 Ring g_idle[2][kIdleRings];
 uint32_t g_idle_count[2] = {0, 0};

@@ -506,8 +506,8 @@ static int alloc_state(gphi_graph *gr)
 	if ((rc = dmalloc(ctx, (void **)&gr->cur, (size_t)G.n_words * 4, nullptr))) return rc;
 	if ((rc = dmalloc(ctx, (void **)&gr->row_stamp, ((size_t)G.side + 1) * 4, nullptr))) return rc;
 	if ((rc = dmalloc(ctx, (void **)&gr->col_unvis, ((size_t)G.side + 1) * 4, nullptr))) return rc;
-	if ((rc = dmalloc(ctx, (void **)&gr->queue, 2 * (size_t)queue_stride(G.n_pad) * 4, nullptr))) return rc;
-	if ((rc = dmalloc(ctx, (void **)&gr->qoff, 2 * (size_t)queue_stride(G.n_pad) * 4, nullptr))) return rc;
+	if ((rc = dmalloc(ctx, (void **)&gr->queue, 2 * (size_t)queue_stride(G.n_pad, G.m) * 4, nullptr))) return rc;
+	if ((rc = dmalloc(ctx, (void **)&gr->qoff, 2 * (size_t)queue_stride(G.n_pad, G.m) * 4, nullptr))) return rc;
 	if ((rc = dmalloc(ctx, (void **)&gr->tile_lo, 2 * (size_t)tile_lo_stride(G.m) * 4, nullptr))) return rc;
 	if ((rc = dmalloc(ctx, (void **)&gr->ctrl, kCtrlBytes, nullptr))) return rc;
 	gr->rec = reinterpret_cast<LevelRec *>(gr->ctrl + 1);
@@ -1422,26 +1422,6 @@ static int frontier_loop(gphi_graph *gr, uint32_t src, gphi_stats *st, uint32_t 
 
 // ---- helpers shared with other translation units (batch.hip) ----
 int ensure_traversal_state(gphi_graph *gr) { return ensure_state(gr); }
-
-// Frontier update from the state bytes (mark / scan / emit) in the
-// device-driven form: nothing when the control block says the traversal is
-// done; otherwise the next level's union frontier, its direction and queue,
-// and ctrl->level advanced by one (from UINT32_MAX, the first update opens
-// level 0).  No level writes.
-void launch_frontier_update_driven(gphi_graph *gr, uint32_t threshold)
-{
-	DevGraph &G = gr->g;
-	hipStream_t s = gr->ctx->stream;
-	const unsigned nblk = G.n_pad / kPadVerts;
-	frontier_mark_kernel<false><<<nblk, kBlock, 0, s>>>(G.W, kLevelFromCtrl, gr->flag, G.deg, gr->level,
-	                                                   gr->visited, gr->cur, gr->row_stamp, gr->col_unvis,
-	                                                   gr->blk_cnt, gr->wave_cnt, gr->ctrl);
-	frontier_scan_kernel<<<1, kScanThreads, 0, s>>>(nblk, threshold, gr->blk_cnt, gr->blk_base, gr->live_cnt,
-	                                              gr->ctrl, gr->trace, false);
-	frontier_emit_kernel<<<nblk, kBlock, 0, s>>>(gr->ctrl, G.deg, gr->cur, gr->blk_cnt, gr->blk_base,
-	                                            gr->wave_cnt, gr->queue_bufs(), false, G.n, G.W, G.side, gr->visited,
-	                                            nullptr);
-}
 
 int run_bfs(gphi_graph *gr, uint32_t src, int32_t *levels, int32_t *parents, gphi_stats *st)
 {

@@ -92,10 +92,12 @@ struct QueueBufs {
 	uint32_t *queue, *qoff, *tile_lo;  // half 0
 	uint32_t qstride, tstride;         // half 1 starts this many entries later
 };
-inline uint32_t queue_stride(uint32_t n_pad) { return n_pad; }
+// an entry per vertex, or (the sparse-source queue of batch.hip) per vertex and
+// kSparseTile out-edges begun
+inline uint32_t queue_stride(uint32_t n_pad, uint64_t m) { return n_pad + (uint32_t)(m / kSparseTile); }
 inline uint32_t tile_lo_stride(uint64_t m) { return (uint32_t)(m / kSparseTile + 2); }
 
-// The level loop of small graphs (small.hip).  LevelRec: a level's totals, the
+// The level loop of levels.h.  LevelRec: a level's totals, the
 // accumulators the level before adds to; a ring over the levels, whose entry
 // half a ring ahead is cleared as a level starts.  LevelBoard: what the
 // device tells the host, in pinned memory.
@@ -103,16 +105,20 @@ constexpr uint32_t kLevelRing = 16;
 struct LevelRec {
 	uint32_t fsize;            // |F|
 	uint32_t chunks;           // chunks its dense sweep took
-	unsigned long long qpack;  // (queue entries << 32) | sum of out-degrees
 	unsigned long long reached, traversed;  // sums of |F| and of sum deg(F) up to this level
-	uint32_t pad[24];          // a 128-byte line each
+	uint32_t pad0[26];
+	// on a line of its own: the advance's blocks each add to both lines
+	unsigned long long qpack;  // (queue entries << 32) | sum of out-degrees
+	uint32_t pad1[30];
 };
-static_assert(sizeof(LevelRec) == 128, "LevelRec is one line");
+static_assert(sizeof(LevelRec) == 256, "LevelRec is two lines");
 struct LevelBoard {
 	unsigned long long progress;  // (levels started << 1) | ended
 	unsigned long long reached, traversed;
 	unsigned long long t_begin, t_end;  // device wall clock
-	uint32_t levels;
+	uint32_t levels, err;
+	unsigned long long live[4];         // multi-source: sources with a non-empty frontier,
+	unsigned long long step_seq;        // as of the step (BatchRun::step) with this number
 	uint4 trace[GPHI_MAX_STEPS];  // per step: direction, |F|, sum deg(F), chunks swept
 };
 constexpr size_t kCtrlBytes = sizeof(StepCtrl) + kLevelRing * sizeof(LevelRec);
@@ -213,7 +219,7 @@ struct gphi_graph {
 	uint32_t *queue = nullptr, *qoff = nullptr, *tile_lo = nullptr;
 	gphi::QueueBufs queue_bufs() const
 	{
-		return gphi::QueueBufs{queue, qoff, tile_lo, gphi::queue_stride(g.n_pad), gphi::tile_lo_stride(g.m)};
+		return gphi::QueueBufs{queue, qoff, tile_lo, gphi::queue_stride(g.n_pad, g.m), gphi::tile_lo_stride(g.m)};
 	}
 	gphi::StepCtrl *ctrl = nullptr;
 	gphi::LevelRec *rec = nullptr;  // in ctrl's allocation (kCtrlBytes)
@@ -251,7 +257,7 @@ struct gphi_graph {
 	unsigned long long *b_live = nullptr;  // sources with a non-empty frontier, then the per-block slots
 	uint32_t *b_touch = nullptr;           // bitmap: vertices whose next mask got a bit this step
 	uint32_t *b_scount = nullptr;          // in b_touch's allocation: new vertices per source, per slot
-	uint32_t *b_aux = nullptr;             // sources to seed, their slots, per-slot start levels
+	uint32_t *b_aux = nullptr;             // per-slot start levels, then the error flag
 	// multi-source SSSP (sssp_batch.hip): kSsspBatchMax distances per vertex
 	// (vertex-major, n_pad rows), then the sources
 	uint32_t *sb_dist = nullptr;
@@ -323,7 +329,6 @@ void out_context_closed();
 // blocks of `block` threads of a kernel that fit the device at once, a multiple of the XCD count
 unsigned resident_grid(const void *kernel, unsigned block = kBlock);
 uint32_t live_list_capacity(uint64_t nchunks);  // entries of one XCD's live-chunk list
-void launch_frontier_update_driven(gphi_graph *gr, uint32_t threshold);
 int run_bfs_batch(gphi_graph *gr, const uint32_t *srcs, uint32_t k, uint8_t *levels, gphi_stats *st);
 // the multi-source state of gr for nw mask words: traversal state, in-edge
 // arrays, masks, levels (idempotent)
@@ -351,16 +356,13 @@ struct BatchRun {
 	uint64_t prev_clean = 0;                     // gr->batch_clean_words when the run began
 	unsigned long long live[4] = {0, 0, 0, 0};   // sources with a non-empty frontier (after step)
 	unsigned long long pairs[2] = {0, 0};        // reached (source, vertex) pairs, their out-degrees
-	uint32_t aux[3 * kBatchMaxSources] = {};     // staging of the sources to seed
-
 	// clears the state and seeds k sources (slots 0..k-1); capacity picks the
 	// mask width (1..256 sources)
 	int begin(gphi_graph *g, uint32_t capacity, const uint32_t *srcs, uint32_t k);
-	// one level, then k new sources join (slots used..used+k-1); reads back
-	// the control block and the live mask
+	// one level, then k new sources join (slots used..used+k-1); learns the
+	// live mask and whether the traversal ended
 	int step(const uint32_t *srcs, uint32_t k);
 	int run_to_end(gphi_stats *st);  // the remaining levels, on the device
-	int read_totals();               // pairs[] from the device
 	// levels of the given slots into host rows of n (unreached: 255 in uint8 rows, -1 in int32 ones)
 	template <class T>
 	int copy_rows(const uint32_t *slots, uint32_t ns, T *const *rows);

@@ -67,8 +67,8 @@ size_t carve_state(const DevGraph &G, uint8_t *base, gphi_graph *t)
 	t->cur = (uint32_t *)take((size_t)G.n_words * 4);
 	t->row_stamp = (uint32_t *)take(((size_t)G.side + 1) * 4);
 	t->col_unvis = (uint32_t *)take(((size_t)G.side + 1) * 4);
-	t->queue = (uint32_t *)take(2 * (size_t)queue_stride(G.n_pad) * 4);  // two halves (QueueBufs)
-	t->qoff = (uint32_t *)take(2 * (size_t)queue_stride(G.n_pad) * 4);
+	t->queue = (uint32_t *)take(2 * (size_t)queue_stride(G.n_pad, G.m) * 4);  // two halves (QueueBufs)
+	t->qoff = (uint32_t *)take(2 * (size_t)queue_stride(G.n_pad, G.m) * 4);
 	t->tile_lo = (uint32_t *)take(2 * (size_t)tile_lo_stride(G.m) * 4);
 	t->ctrl = (StepCtrl *)take(kCtrlBytes);
 	t->rec = reinterpret_cast<LevelRec *>(t->ctrl + 1);

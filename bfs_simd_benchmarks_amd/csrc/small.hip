@@ -14,15 +14,7 @@
 //             stamps, column counts -- and its queue, at positions reserved
 //             with one atomic per block, so that no scan comes between
 //
-// A level's totals are the accumulators the advance of the level before it
-// added to (LevelRec, a ring over the levels); every block of the next
-// expansion reads them and applies the direction rule itself.
-//
-// The first block of an expansion writes the level it starts, and at the end
-// the totals, to pinned host memory (LevelBoard).  The host keeps kAhead
-// levels enqueued past the one it sees there, so the device never waits for
-// it, and stops when it sees the end: nothing is read back, and at most
-// kAhead levels are launched for nothing.
+// How the direction is decided and the host follows: levels.h.
 //
 // Reference: the level loop of apps/bfs_simd/bfs.cpp:795-910 and
 // apps/sssp_simd/sssp.cpp:1000-1100.
@@ -32,34 +24,25 @@
 #include <climits>
 #include <cstring>
 
-#include "sweep.h"
+#include "levels.h"
 
 namespace gphi {
 
 namespace {
 
-constexpr uint32_t kAhead = 2;  // levels enqueued past the one the device has started
-
 // What the kernels of one traversal share.
-struct Trav {
-	uint32_t n, n_pad, n_words, W, side, threshold, win_rows;
+struct Trav : Frontier {
+	uint32_t n, n_words, side, win_rows;
 	uint32_t nchunks, run, slots;  // chunks per run, chunks tested per block
-	const uint32_t *row_off, *cols, *csr_w, *deg;
+	const uint32_t *row_off, *cols, *csr_w;
 	const uint32_t *heads, *tails, *coo_w;
 	const uint16_t *heads16, *tails16;
 	const uint8_t *coo_w8;
 	const ChunkMeta *meta;
 	const ChunkPack *pack;
-	int32_t *level, *parent;
+	int32_t *parent;
 	uint32_t *dist;
-	uint8_t *flag;
-	uint32_t *visited, *cur, *row_stamp, *col_unvis;
-	QueueBufs qb;
-	LevelRec *rec;
-	LevelBoard *board;
 };
-
-__device__ __forceinline__ LevelRec *rec_of(const Trav &t, uint32_t level) { return t.rec + level % kLevelRing; }
 
 // All state of a traversal set up for its source, in one launch: every word
 // is written once, with the source's part in it.
@@ -107,47 +90,6 @@ __global__ __launch_bounds__(kBlock) void small_init_kernel(Trav t, uint32_t src
 		t.qb.queue[0] = src;
 		t.qb.qoff[0] = 0;
 		t.board->t_begin = wall_clock64();
-	}
-}
-
-// The start of a level, one thread: the previous step's chunk count and this
-// step's trace entry, the totals, the ring entry of a later level, and the
-// progress word.  The end is stored with a system-scope release, after which
-// the host may read the whole board.
-__device__ void publish_level(const Trav &t, uint32_t level, uint32_t fsize, uint32_t fdeg, uint32_t dir)
-{
-	LevelRec *r = rec_of(t, level);
-	LevelBoard *b = t.board;
-	unsigned long long reached = 0, traversed = 0;
-	bool ended = false;
-	if (level) {
-		const LevelRec *p = rec_of(t, level - 1);
-		reached = p->reached;
-		traversed = p->traversed;
-		ended = p->fsize == 0;
-		if (!ended && level <= GPHI_MAX_STEPS) b->trace[level - 1].w = p->chunks;
-	}
-	if (!ended) {
-		r->reached = reached + fsize;
-		r->traversed = traversed + fdeg;
-		*rec_of(t, level + kLevelRing / 2) = LevelRec{};
-		if (fsize) {
-			if (level < GPHI_MAX_STEPS) {
-				b->trace[level].x = dir;
-				b->trace[level].y = fsize;
-				b->trace[level].z = fdeg;
-				b->trace[level].w = 0u;
-			}
-			__hip_atomic_store(&b->progress, (unsigned long long)(level + 1) << 1, __ATOMIC_RELAXED,
-			                   __HIP_MEMORY_SCOPE_SYSTEM);
-		} else {
-			b->reached = reached;
-			b->traversed = traversed;
-			b->levels = level;
-			b->t_end = wall_clock64();
-			__hip_atomic_store(&b->progress, ((unsigned long long)(level + 1) << 1) | 1ull, __ATOMIC_RELEASE,
-			                   __HIP_MEMORY_SCOPE_SYSTEM);
-		}
 	}
 }
 
@@ -255,15 +197,12 @@ __global__ __launch_bounds__(kBlock, kWeights ? 5 : 7) void small_expand_kernel(
 	constexpr uint32_t kMem = std::max<uint32_t>(3 * kPushEntry, (kBfs ? 2 : 1) * kWinWords);
 	__shared__ uint4 s_mem[(kMem + 3) / 4];
 	LevelRec *r = rec_of(t, level);
-	const uint32_t fsize = r->fsize;
-	const unsigned long long qp = r->qpack;
-	const uint32_t fdeg = (uint32_t)qp;
-	// the first step is sparse (apps/bfs_simd/bfs.cpp:807), then the rule of :829-834
-	const bool dense = level > 0 && fsize + fdeg > t.threshold;
-	if (blockIdx.x == 0 && threadIdx.x == 0) publish_level(t, level, fsize, fdeg, dense);
-	if (fsize == 0) return;
+	const Step st = step_of(t, level);
+	const bool dense = level > 0 && st.dense;  // the first step is sparse (apps/bfs_simd/bfs.cpp:807)
+	if (blockIdx.x == 0 && threadIdx.x == 0) publish_level(t, level, st.fsize, st.fdeg, dense);
+	if (st.fsize == 0) return;
 	if (!dense) {
-		small_push<kBfs>(reinterpret_cast<uint32_t *>(s_mem), t, level, (uint32_t)(qp >> 32), fdeg);
+		small_push<kBfs>(reinterpret_cast<uint32_t *>(s_mem), t, level, st.qsize, st.fdeg);
 		return;
 	}
 	// this block's share of the chunks: runs of t.run consecutive chunks (they
@@ -294,133 +233,10 @@ __global__ __launch_bounds__(kBlock, kWeights ? 5 : 7) void small_expand_kernel(
 		                               t.flag);
 }
 
-// The next frontier from the state bytes and its queue, in one pass.  A lane
-// owns kLaneVerts consecutive vertices: a frontier of a few thousand vertices
-// then spreads over enough wavefronts that none has more than one round of
-// degree loads, one prefix sum and kLaneVerts queue entries per lane to do
-// (a lane per 32-vertex word, as in frontier_mark_kernel, took 16 us on the
-// 9 blocks of a 65536-vertex graph).  A block adds its totals to the next
-// level's accumulators, which gives it its queue position and degree prefix;
-// the blocks' shares of the queue come in any order.  Once the degrees added
-// so far pass the direction rule's threshold the next step is dense and needs
-// no queue.
-// Blocks are 256 threads up to kAdvanceNarrow vertices and 1024 above: a block
-// makes two atomics, all on one line (on 1.6M vertices 256-thread blocks took
-// 19 us for a dense level, 15 of them the atomics, and 1024-thread ones 11;
-// on 65536 vertices, with nothing to queue for, they took 5.4 and 6.0).
-constexpr uint32_t kLaneVerts = 8;
-constexpr uint32_t kAdvanceNarrow = 1u << 18;
-static_assert(kPadVerts % (1024 * kLaneVerts) == 0, "whole blocks over the padded vertices");
-
 template <bool kBfs, uint32_t kThreads>
-__global__ __launch_bounds__(kThreads) void small_advance_kernel(Trav t, uint32_t level)
+__global__ __launch_bounds__(kThreads) void small_advance_kernel(Frontier t, uint32_t level)
 {
-	if (rec_of(t, level)->fsize == 0) return;
-	LevelRec *nr = rec_of(t, level + 1);
-	const uint32_t next_level = level + 1;
-	const uint32_t i = blockIdx.x * kThreads + threadIdx.x, v0 = i * kLaneVerts;
-	const uint32_t lane = lane_id(), wid = threadIdx.x >> 6;
-	uint2 *fp = reinterpret_cast<uint2 *>(t.flag) + i;
-	const uint2 f8 = *fp;
-	uint32_t bits = 0;
-#pragma unroll
-	for (int k = 0; k < 4; ++k) {
-		bits |= ((f8.x >> (8 * k)) & 1u) << k;
-		bits |= ((f8.y >> (8 * k)) & 1u) << (4 + k);
-	}
-	// byte i of the bitmaps: bits of the lane's vertices
-	reinterpret_cast<uint8_t *>(t.cur)[i] = (uint8_t)bits;
-	uint32_t d[kLaneVerts], q = 0, dsum = 0;
-#pragma unroll
-	for (uint32_t k = 0; k < kLaneVerts; ++k) d[k] = 0;
-	if (bits) {
-		const uint4 da = reinterpret_cast<const uint4 *>(t.deg + v0)[0], db = reinterpret_cast<const uint4 *>(t.deg + v0)[1];
-		if (kBfs) {
-			constexpr uint32_t kLow = 0x01010101u;  // state 1 -> kVisited
-			*fp = make_uint2(f8.x + (f8.x & kLow), f8.y + (f8.y & kLow));
-			reinterpret_cast<uint8_t *>(t.visited)[i] |= (uint8_t)bits;
-#pragma unroll
-			for (uint32_t k = 0; k < kLaneVerts; ++k)
-				if ((bits >> k) & 1u) t.level[v0 + k] = (int32_t)next_level;
-		} else {
-			*fp = make_uint2(0, 0);
-		}
-		const uint32_t dd[kLaneVerts] = {da.x, da.y, da.z, da.w, db.x, db.y, db.z, db.w};
-#pragma unroll
-		for (uint32_t k = 0; k < kLaneVerts; ++k) {
-			d[k] = (bits >> k) & 1u ? dd[k] : 0u;
-			q += d[k] > 0;
-			dsum += d[k];
-		}
-		if (t.W % kLaneVerts == 0) {  // one row for the lane's vertices
-			if (q) t.row_stamp[v0 / t.W] = next_level;
-		} else {
-#pragma unroll
-			for (uint32_t k = 0; k < kLaneVerts; ++k)
-				if (d[k]) t.row_stamp[(v0 + k) / t.W] = next_level;
-		}
-	}
-	const uint32_t nf = (uint32_t)__popc(bits);
-	__shared__ uint32_t s_red[3][kThreads / 64];
-	__shared__ unsigned long long s_base;
-	uint32_t ftot, qtot, dtot;
-	const uint32_t qx = wave_excl_scan(q, &qtot), dx = wave_excl_scan(dsum, &dtot);
-	ftot = wave_sum(nf);
-	if (lane == 0) {
-		s_red[0][wid] = ftot;
-		s_red[1][wid] = qtot;
-		s_red[2][wid] = dtot;
-	}
-	__syncthreads();
-	if (threadIdx.x == 0) {
-		uint32_t f = 0, qb = 0, db = 0;
-		for (uint32_t k = 0; k < kThreads / 64; ++k) {
-			f += s_red[0][k];
-			qb += s_red[1][k];
-			db += s_red[2][k];
-		}
-		unsigned long long base = ~0ull;
-		if (f) atomicAdd(&nr->fsize, f);
-		if (qb) {
-			base = atomicAdd(&nr->qpack, ((unsigned long long)qb << 32) | db);
-			if ((uint32_t)base + db > t.threshold) base = ~0ull;  // the next step is dense
-		}
-		s_base = base;
-	}
-	if (kBfs && ftot) {
-		// column counts of unvisited vertices: one atomic per wavefront when
-		// its vertices share a column, else one per lane (or vertex)
-		const uint32_t wv0 = v0 - lane * kLaneVerts;
-		if (wv0 / t.W == (wv0 + 64 * kLaneVerts - 1) / t.W) {
-			if (lane == 0) atomicSub(t.col_unvis + wv0 / t.W, ftot);
-		} else if (t.W % kLaneVerts == 0) {
-			if (nf) atomicSub(t.col_unvis + v0 / t.W, nf);
-		} else {
-			for (uint32_t b = bits; b; b &= b - 1) atomicSub(t.col_unvis + (v0 + __ffs(b) - 1) / t.W, 1u);
-		}
-	}
-	__syncthreads();
-	if (s_base == ~0ull || q == 0) return;
-	uint32_t pos = (uint32_t)(s_base >> 32) + qx, off = (uint32_t)s_base + dx;
-	for (uint32_t k = 0; k < wid; ++k) {
-		pos += s_red[1][k];
-		off += s_red[2][k];
-	}
-	const uint32_t par = next_level & 1u;
-	uint32_t *__restrict__ queue = t.qb.queue + par * t.qb.qstride;
-	uint32_t *__restrict__ qoff = t.qb.qoff + par * t.qb.qstride;
-	uint32_t *__restrict__ tile_lo = t.qb.tile_lo + par * t.qb.tstride;
-#pragma unroll
-	for (uint32_t k = 0; k < kLaneVerts; ++k) {
-		if (!d[k]) continue;
-		queue[pos] = v0 + k;
-		qoff[pos] = off;
-		// tiles of the next push whose first edge falls in [off, off + d)
-		for (uint32_t x = (off + kSparseTile - 1) / kSparseTile; (uint64_t)x * kSparseTile < (uint64_t)off + d[k]; ++x)
-			tile_lo[x] = pos;
-		pos += 1;
-		off += d[k];
-	}
+	advance_block<kBfs, kThreads>(t, level);
 }
 
 }  // namespace
@@ -438,21 +254,16 @@ int small_level_loop(gphi_graph *gr, uint32_t src, gphi_stats *st, uint32_t *ste
 	const DevGraph &G = gr->g;
 	hipStream_t s = ctx->stream;
 	LevelBoard *board = ctx->h_board;
-	Trav t;
-	t.n = G.n, t.n_pad = G.n_pad, t.n_words = G.n_words, t.W = G.W, t.side = G.side;
-	t.threshold = (uint32_t)G.m / ctx->t_ratio;
+	Trav t = {};
+	static_cast<Frontier &>(t) = make_frontier(gr, (uint32_t)G.m / ctx->t_ratio);
+	t.n = G.n, t.n_words = G.n_words, t.side = G.side;
 	t.win_rows = dense_window_rows(G.W);
 	t.nchunks = (uint32_t)G.nchunks;
-	t.row_off = G.row_off, t.cols = G.cols, t.csr_w = G.csr_w, t.deg = G.deg;
+	t.row_off = G.row_off, t.cols = G.cols, t.csr_w = G.csr_w;
 	t.heads = G.heads, t.tails = G.tails, t.coo_w = G.coo_w;
 	t.heads16 = G.heads16, t.tails16 = G.tails16, t.coo_w8 = G.coo_w8;
 	t.meta = G.meta, t.pack = G.pack;
-	t.level = gr->level, t.parent = gr->parent, t.dist = gr->dist;
-	t.flag = gr->flag, t.visited = gr->visited, t.cur = gr->cur;
-	t.row_stamp = gr->row_stamp, t.col_unvis = gr->col_unvis;
-	t.qb = gr->queue_bufs();
-	t.rec = gr->rec;
-	t.board = board;
+	t.parent = gr->parent, t.dist = gr->dist;
 	// Every block is resident at once.  A block takes runs of chunks, as long
 	// as they leave no block with more than a tenth over its share.
 	static const unsigned resident[3] = {resident_grid(reinterpret_cast<const void *>(small_expand_kernel<0>)),
@@ -466,44 +277,24 @@ int small_level_loop(gphi_graph *gr, uint32_t src, gphi_stats *st, uint32_t *ste
 		if (t.run == 1 || (uint64_t)t.slots * grid <= t.nchunks + t.nchunks / 10) break;
 	}
 	if (t.slots > kBlock) return set_error(ctx, GPHI_E_STATE, "%u chunks exceed the small level loop", t.nchunks);
-	const unsigned adv = G.n_pad <= kAdvanceNarrow ? 256 : 1024, nblk = G.n_pad / (adv * kLaneVerts);
-	*(volatile unsigned long long *)&board->progress = 0;
+	const unsigned adv = advance_threads(G.n_pad), nblk = advance_blocks(G.n_pad);
+	reset_board(board);
 	const uint64_t items = std::max<uint64_t>({G.n_pad / (kBfs ? 16 : 1), G.n_words, G.side});
 	small_init_kernel<kBfs><<<(unsigned)std::min<uint64_t>((items + kBlock - 1) / kBlock, 2048), kBlock, 0, s>>>(t, src);
-	uint32_t enq = 0, seen = 0, idle = 0;
-	for (;;) {
-		for (; enq <= seen + kAhead; ++enq) {
-			if (kBfs)
-				small_expand_kernel<0><<<grid, kBlock, 0, s>>>(t, enq);
-			else if (G.coo_w8)
-				small_expand_kernel<1><<<grid, kBlock, 0, s>>>(t, enq);
-			else
-				small_expand_kernel<4><<<grid, kBlock, 0, s>>>(t, enq);
-			if (adv == 256)
-				small_advance_kernel<kBfs, 256><<<nblk, 256, 0, s>>>(t, enq);
-			else
-				small_advance_kernel<kBfs, 1024><<<nblk, 1024, 0, s>>>(t, enq);
-		}
-		GPHI_HIP(ctx, hipGetLastError());
-		// the level the device has started last; the stream is looked at now
-		// and then, so that an error on the device ends the wait
-		unsigned long long p;
-		for (uint32_t spin = 0;; ++spin) {
-			p = __atomic_load_n(&board->progress, __ATOMIC_ACQUIRE);
-			if ((p & 1ull) || (p >> 1) > seen + 1) break;
-			if (spin % 4096 == 4095) {
-				const hipError_t e = hipStreamQuery(s);
-				if (e != hipSuccess && e != hipErrorNotReady)
-					return hip_fail(ctx, e, "level loop", __FILE__, __LINE__);
-				// an idle stream has published every enqueued level
-				if (e == hipSuccess && ++idle > 2) return set_error(ctx, GPHI_E_STATE, "level loop made no progress");
-			}
-			__builtin_ia32_pause();
-		}
-		idle = 0;
-		if (p & 1ull) break;
-		seen = (uint32_t)(p >> 1) - 1;
-	}
+	const int rc = follow_levels(ctx, [&](uint32_t level) {
+		if (kBfs)
+			small_expand_kernel<0><<<grid, kBlock, 0, s>>>(t, level);
+		else if (G.coo_w8)
+			small_expand_kernel<1><<<grid, kBlock, 0, s>>>(t, level);
+		else
+			small_expand_kernel<4><<<grid, kBlock, 0, s>>>(t, level);
+		if (adv == 256)
+			small_advance_kernel<kBfs, 256><<<nblk, 256, 0, s>>>(t, level);
+		else
+			small_advance_kernel<kBfs, 1024><<<nblk, 1024, 0, s>>>(t, level);
+		return GPHI_OK;
+	});
+	if (rc) return rc;
 	if (steps) *steps = board->levels;
 	if (st) {
 		const uint32_t ns = std::min<uint32_t>(board->levels, GPHI_MAX_STEPS);
@@ -517,7 +308,7 @@ int small_level_loop(gphi_graph *gr, uint32_t src, gphi_stats *st, uint32_t *ste
 		}
 		st->reached = board->reached;
 		st->edges_traversed = board->traversed;
-		st->total_ms = (float)((double)(board->t_end - board->t_begin) / ctx->wall_clock_khz);
+		st->total_ms = board_ms(ctx);
 	}
 	return GPHI_OK;
 }

@@ -13,27 +13,27 @@
 // distances whatever the order of the relaxations, so each row equals that
 // source's single-source result (and Dijkstra's).
 //
-// The steps reuse the single-source machinery: a direction rule on the
-// union frontier (|F| + sum deg > M / 2, see kSsspBatchDenseDiv), the frontier update in its
-// device-driven form (state byte 1 = some distance dropped) and the CSR push
-// of a sparse step over the union queue.  A dense step is a pull over the
-// in-edges and their weights (build_in_weights), skipping heads outside the
-// frontier bitmap, so that a tail's 16 distances take one write, not an
-// atomic per improved source.
+// The level loop is that of levels.h, two launches per level (expand,
+// advance; state byte 1 = some distance dropped), with a direction rule on the
+// union frontier of its own (|F| + sum deg > M / 2, see kSsspBatchDenseDiv).
+// A sparse step is the CSR push over the union queue.  A dense step is a pull
+// over the in-edges and their weights (build_in_weights), skipping heads
+// outside the frontier bitmap, so that a tail's 16 distances take one write,
+// not an atomic per improved source; vertices of few in-edges and the pieces
+// of the others share the launch, the pieces first.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cstring>
 
-#include "internal.h"
+#include "levels.h"
 
 namespace gphi {
 
 namespace {
 
 constexpr uint32_t kInf = 2147483647u;  // unreached, as sssp.cpp:994-998
-constexpr uint32_t kSsspLevelGroup = 8;  // levels enqueued per read-back of the control block
-constexpr unsigned kSsspGrid = 8192;  // blocks of the push and pull launches (grid-stride loops)
+constexpr unsigned kSsspGrid = 8192;  // most blocks of the push, and of each pull (grid-stride loops)
 // A step is dense when the union frontier's |F| + sum deg(F) exceeds M / 2,
 // not M / T_RATIO as in the single-source rule: a push step relaxes 16
 // distances per frontier edge with one row gather, while a pull step reads
@@ -77,53 +77,60 @@ __device__ __forceinline__ bool relax_row(const uint32_t (&dh)[kSsspBatchMax], u
 	return better;
 }
 
-// all distances kInf, state bytes and frontier bitmap clear, control block
-// set for the first frontier update (which opens level 0)
-__global__ __launch_bounds__(kBlock) void ssspb_clear_kernel(uint32_t n_pad, uint32_t n_words, uint4 *dist4,
-                                                             uint8_t *flag, uint32_t *cur, StepCtrl *ctrl)
+// What the kernels of a traversal share.
+struct SsspBatch : Frontier {
+	uint32_t n, npieces, heavy_blocks;
+	const uint32_t *row_off, *cols, *csr_w, *in_off, *in_src, *w32;
+	const uint8_t *w8;
+	const uint2 *pieces;
+	uint32_t *dist;
+};
+
+// all distances kInf, state bytes and frontier bitmap clear, level records set
+// for the advance that opens level 0 (that of the level before it, UINT32_MAX)
+__global__ __launch_bounds__(kBlock) void ssspb_clear_kernel(SsspBatch t, uint32_t n_words)
 {
 	const uint64_t stride = (uint64_t)gridDim.x * kBlock;
 	const uint64_t i0 = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-	for (uint64_t i = i0; i < (uint64_t)n_pad * kSsspBatchMax / 4; i += stride)
-		dist4[i] = make_uint4(kInf, kInf, kInf, kInf);
-	for (uint64_t i = i0; i < n_pad / 16; i += stride) reinterpret_cast<uint4 *>(flag)[i] = make_uint4(0, 0, 0, 0);
-	for (uint64_t i = i0; i < n_words; i += stride) cur[i] = 0;
-	if (i0 == 0) {
-		ctrl->level = UINT32_MAX;
-		ctrl->done = 0;
-		ctrl->err = 0;
-		ctrl->dir = 0;
-		ctrl->reached = 0;
-		ctrl->traversed = 0;
+	for (uint64_t i = i0; i < (uint64_t)t.n_pad * kSsspBatchMax / 4; i += stride)
+		reinterpret_cast<uint4 *>(t.dist)[i] = make_uint4(kInf, kInf, kInf, kInf);
+	for (uint64_t i = i0; i < t.n_pad / 16; i += stride) reinterpret_cast<uint4 *>(t.flag)[i] = make_uint4(0, 0, 0, 0);
+	for (uint64_t i = i0; i < n_words; i += stride) t.cur[i] = 0;
+	if (i0 < kLevelRing) {
+		LevelRec r = {};
+		if (i0 == UINT32_MAX % kLevelRing) r.fsize = 1;
+		t.rec[i0] = r;
 	}
+	if (i0 == 0) t.board->t_begin = wall_clock64();
 }
 
 // source i at slot i: distance 0, in the first frontier
-__global__ void ssspb_seed_kernel(const uint32_t *__restrict__ srcs, uint32_t k, uint32_t *dist, uint8_t *flag)
+struct SsspSeeds {
+	uint32_t src[kSsspBatchMax];
+};
+__global__ void ssspb_seed_kernel(SsspBatch t, SsspSeeds seeds, uint32_t k)
 {
-	for (uint32_t i = threadIdx.x; i < k; i += blockDim.x) {
-		dist[(uint64_t)srcs[i] * kSsspBatchMax + i] = 0;
-		flag[srcs[i]] = 1;
-	}
+	const uint32_t i = threadIdx.x;
+	if (i >= k) return;
+	t.dist[(uint64_t)seeds.src[i] * kSsspBatchMax + i] = 0;
+	t.flag[seeds.src[i]] = 1;
 }
 
 // Sparse step: the edge-balanced CSR push over the union queue (tiles of
 // kSparseTile edges from tile_lo, as the single-source push).
-__global__ __launch_bounds__(kBlock) void ssspb_sparse_kernel(const StepCtrl *__restrict__ ctrl, QueueBufs qb,
-                                                              const uint32_t *__restrict__ row_off,
-                                                              const uint32_t *__restrict__ cols,
-                                                              const uint32_t *__restrict__ csr_w, uint32_t *dist,
-                                                              uint8_t *flag)
+__device__ __forceinline__ void push_union(const SsspBatch &t, uint32_t level, const Step &st)
 {
 	__shared__ uint32_t s_off[kSparseTile + 2];
 	__shared__ uint32_t s_u[kSparseTile + 2];
 	__shared__ uint32_t s_base[kSparseTile + 2];
-	if (ctrl->done || ctrl->dir != 0) return;
-	const uint32_t qsize = ctrl->qsize, qdeg = ctrl->fdeg;
-	const uint32_t par = ctrl->level & 1u;  // the half the frontier update wrote
-	const uint32_t *__restrict__ queue = qb.queue + par * qb.qstride;
-	const uint32_t *__restrict__ qoff = qb.qoff + par * qb.qstride;
-	const uint32_t *__restrict__ tile_lo = qb.tile_lo + par * qb.tstride;
+	const uint32_t *__restrict__ row_off = t.row_off, *__restrict__ cols = t.cols, *__restrict__ csr_w = t.csr_w;
+	uint32_t *dist = t.dist;
+	uint8_t *flag = t.flag;
+	const uint32_t qsize = st.qsize, qdeg = st.fdeg;
+	const uint32_t par = level & 1u;  // the half the advance wrote
+	const uint32_t *__restrict__ queue = t.qb.queue + par * t.qb.qstride;
+	const uint32_t *__restrict__ qoff = t.qb.qoff + par * t.qb.qstride;
+	const uint32_t *__restrict__ tile_lo = t.qb.tile_lo + par * t.qb.tstride;
 	const uint32_t ntile = (qdeg + kSparseTile - 1) / kSparseTile;
 	for (uint32_t k = blockIdx.x; k < ntile; k += gridDim.x) {
 		const uint32_t lo = tile_lo[k];
@@ -201,16 +208,15 @@ __device__ __forceinline__ void pull_edges(uint32_t e, uint32_t e_end, uint32_t 
 // vertices with 1..kPullLight in-edges, a lane each (it owns the vertex:
 // plain stores)
 template <bool kW8>
-__global__ __launch_bounds__(kBlock) void ssspb_pull_light_kernel(const StepCtrl *__restrict__ ctrl, uint32_t n,
-                                                                  const uint32_t *__restrict__ in_off,
-                                                                  const uint32_t *__restrict__ in_src,
-                                                                  const uint32_t *__restrict__ w32,
-                                                                  const uint8_t *__restrict__ w8,
-                                                                  const uint32_t *__restrict__ cur, uint32_t *dist,
-                                                                  uint8_t *flag)
+__device__ __forceinline__ void pull_light(const SsspBatch &b, uint32_t bid, uint32_t nb)
 {
-	if (ctrl->done || ctrl->dir != 1) return;
-	for (uint32_t t = blockIdx.x * kBlock + threadIdx.x; t < n; t += gridDim.x * kBlock) {
+	const uint32_t n = b.n;
+	const uint32_t *__restrict__ in_off = b.in_off, *__restrict__ in_src = b.in_src, *__restrict__ w32 = b.w32;
+	const uint32_t *__restrict__ cur = b.cur;
+	const uint8_t *__restrict__ w8 = b.w8;
+	uint32_t *dist = b.dist;
+	uint8_t *flag = b.flag;
+	for (uint32_t t = bid * kBlock + threadIdx.x; t < n; t += nb * kBlock) {
 		const uint32_t e0 = in_off[t], e1 = in_off[t + 1];
 		if (e1 == e0 || e1 - e0 > kPullLight) continue;
 		uint32_t cand[kSsspBatchMax];
@@ -234,18 +240,17 @@ __global__ __launch_bounds__(kBlock) void ssspb_pull_light_kernel(const StepCtrl
 // each: lane minima, a wavefront minimum per source, then lane s lowers
 // source s's distance (atomicMin: a vertex's pieces may run at once)
 template <bool kW8>
-__global__ __launch_bounds__(kBlock) void ssspb_pull_heavy_kernel(const StepCtrl *__restrict__ ctrl, uint32_t npieces,
-                                                                  const uint2 *__restrict__ pieces,
-                                                                  const uint32_t *__restrict__ in_off,
-                                                                  const uint32_t *__restrict__ in_src,
-                                                                  const uint32_t *__restrict__ w32,
-                                                                  const uint8_t *__restrict__ w8,
-                                                                  const uint32_t *__restrict__ cur, uint32_t *dist,
-                                                                  uint8_t *flag)
+__device__ __forceinline__ void pull_heavy(const SsspBatch &b, uint32_t bid, uint32_t nb)
 {
-	if (ctrl->done || ctrl->dir != 1) return;
-	const uint32_t lane = threadIdx.x & 63, nwaves = (gridDim.x * kBlock) >> 6;
-	for (uint32_t p = (blockIdx.x * kBlock + threadIdx.x) >> 6; p < npieces; p += nwaves) {
+	const uint32_t *__restrict__ in_off = b.in_off, *__restrict__ in_src = b.in_src, *__restrict__ w32 = b.w32;
+	const uint32_t *__restrict__ cur = b.cur;
+	const uint8_t *__restrict__ w8 = b.w8;
+	const uint2 *__restrict__ pieces = b.pieces;
+	const uint32_t npieces = b.npieces;
+	uint32_t *dist = b.dist;
+	uint8_t *flag = b.flag;
+	const uint32_t lane = threadIdx.x & 63, nwaves = (nb * kBlock) >> 6;
+	for (uint32_t p = (bid * kBlock + threadIdx.x) >> 6; p < npieces; p += nwaves) {
 		const uint2 pc = pieces[p];
 		const uint32_t t = pc.x, e1 = min(pc.y + kPullPiece, in_off[t + 1]);
 		uint32_t cand[kSsspBatchMax];
@@ -275,6 +280,26 @@ __global__ __launch_bounds__(kBlock) void ssspb_pull_heavy_kernel(const StepCtrl
 	}
 }
 
+template <bool kW8>
+__global__ __launch_bounds__(kBlock) void ssspb_expand_kernel(SsspBatch t, uint32_t level)
+{
+	const Step st = step_of(t, level);
+	if (blockIdx.x == 0 && threadIdx.x == 0) publish_level(t, level, st.fsize, st.fdeg, st.dense);
+	if (st.fsize == 0) return;
+	if (!st.dense)
+		push_union(t, level, st);
+	else if (blockIdx.x < t.heavy_blocks)
+		pull_heavy<kW8>(t, blockIdx.x, t.heavy_blocks);
+	else
+		pull_light<kW8>(t, blockIdx.x - t.heavy_blocks, gridDim.x - t.heavy_blocks);
+}
+
+template <uint32_t kThreads>
+__global__ __launch_bounds__(kThreads) void ssspb_advance_kernel(Frontier t, uint32_t level)
+{
+	advance_block<false, kThreads>(t, level);
+}
+
 }  // namespace
 
 // The traversal state, in-edge arrays with their weights, and the distance
@@ -289,7 +314,7 @@ int sssp_batch_prepare(gphi_graph *gr)
 	if (rc) return rc;
 	if ((rc = build_in_edges(gr)) || (rc = build_in_weights(gr))) return rc;
 	if (!gr->sb_dist) {
-		const size_t bytes = (size_t)G.n_pad * kSsspBatchMax * 4 + (size_t)kSsspBatchMax * 4;
+		const size_t bytes = (size_t)G.n_pad * kSsspBatchMax * 4;
 		if (take_injected_alloc_failure())
 			return set_error(ctx, GPHI_E_OOM, "hipMalloc(%zu bytes) failed: injected failure", bytes);
 		if (hipMalloc((void **)&gr->sb_dist, bytes) != hipSuccess) {
@@ -311,64 +336,49 @@ int run_sssp_batch(gphi_graph *gr, const uint32_t *srcs, uint32_t k, uint32_t *c
 		if (srcs[i] >= G.n) return set_error(ctx, GPHI_E_RANGE, "source %u >= N %u", srcs[i], G.n);
 	int rc = sssp_batch_prepare(gr);
 	if (rc) return rc;
-	uint32_t *d_srcs = gr->sb_dist + (size_t)G.n_pad * kSsspBatchMax;
 	if (st) memset(st, 0, sizeof(*st));
 	hipStream_t s = ctx->stream;
-	const bool timing = st != nullptr && ctx->ev_ok;
-	if (timing) GPHI_HIP(ctx, hipEventRecord(ctx->ev[0], s));
+	SsspBatch t = {};
+	static_cast<Frontier &>(t) = make_frontier(gr, (uint32_t)(G.m / kSsspBatchDenseDiv));
+	t.n = G.n, t.npieces = gr->npieces;
+	t.row_off = G.row_off, t.cols = G.cols, t.csr_w = G.csr_w;
+	t.in_off = gr->in_off, t.in_src = gr->in_src, t.w32 = gr->in_w32, t.w8 = gr->in_w8, t.pieces = gr->pieces;
+	t.dist = gr->sb_dist;
+	t.heavy_blocks = std::min<unsigned>((gr->npieces + 3) / 4, kSsspGrid);
+	const unsigned light_blocks = std::min<unsigned>((G.n + kBlock - 1) / kBlock, kSsspGrid);
+	const unsigned push_blocks = (unsigned)std::min<uint64_t>(G.m / kSparseTile + 1, kSsspGrid);
+	const unsigned grid = std::max(t.heavy_blocks + light_blocks, push_blocks);
+	const unsigned adv = advance_threads(G.n_pad), nblk = advance_blocks(G.n_pad);
+	reset_board(ctx->h_board);
 	const uint64_t items = std::max<uint64_t>((uint64_t)G.n_pad * kSsspBatchMax / 4, G.n_words);
-	ssspb_clear_kernel<<<(unsigned)std::min<uint64_t>((items + kBlock - 1) / kBlock, 16384), kBlock, 0, s>>>(
-	    G.n_pad, G.n_words, reinterpret_cast<uint4 *>(gr->sb_dist), gr->flag, gr->cur, gr->ctrl);
-	GPHI_HIP(ctx, hipMemcpyAsync(d_srcs, srcs, (size_t)k * 4, hipMemcpyHostToDevice, s));
-	ssspb_seed_kernel<<<1, 64, 0, s>>>(d_srcs, k, gr->sb_dist, gr->flag);
-	const uint32_t threshold = (uint32_t)(G.m / kSsspBatchDenseDiv);
-	launch_frontier_update_driven(gr, threshold);  // opens level 0: the sources
-	GPHI_HIP(ctx, hipGetLastError());
-	const unsigned lgrid = std::min<unsigned>((G.n + kBlock - 1) / kBlock, kSsspGrid);
-	const unsigned hgrid = std::max<unsigned>(1, std::min<unsigned>((gr->npieces + 3) / 4, kSsspGrid));
-	StepCtrl *hc = ctx->h_ctrl;
-	uint32_t enq = 0;
-	for (;;) {
-		for (uint32_t q = 0; q < kSsspLevelGroup; ++q, ++enq) {
-			ssspb_sparse_kernel<<<kSsspGrid, kBlock, 0, s>>>(gr->ctrl, gr->queue_bufs(), G.row_off, G.cols,
-			                                                 G.csr_w, gr->sb_dist, gr->flag);
-			if (gr->in_w8) {
-				ssspb_pull_light_kernel<true><<<lgrid, kBlock, 0, s>>>(gr->ctrl, G.n, gr->in_off, gr->in_src,
-				                                                       nullptr, gr->in_w8, gr->cur, gr->sb_dist,
-				                                                       gr->flag);
-				if (gr->npieces)
-					ssspb_pull_heavy_kernel<true><<<hgrid, kBlock, 0, s>>>(gr->ctrl, gr->npieces, gr->pieces,
-					                                                       gr->in_off, gr->in_src, nullptr,
-					                                                       gr->in_w8, gr->cur, gr->sb_dist, gr->flag);
-			} else {
-				ssspb_pull_light_kernel<false><<<lgrid, kBlock, 0, s>>>(gr->ctrl, G.n, gr->in_off, gr->in_src,
-				                                                        gr->in_w32, nullptr, gr->cur, gr->sb_dist,
-				                                                        gr->flag);
-				if (gr->npieces)
-					ssspb_pull_heavy_kernel<false><<<hgrid, kBlock, 0, s>>>(gr->ctrl, gr->npieces, gr->pieces,
-					                                                        gr->in_off, gr->in_src, gr->in_w32,
-					                                                        nullptr, gr->cur, gr->sb_dist, gr->flag);
-			}
-			launch_frontier_update_driven(gr, threshold);
-		}
-		GPHI_HIP(ctx, hipGetLastError());
-		GPHI_HIP(ctx, hipMemcpyAsync(hc, gr->ctrl, sizeof(StepCtrl), hipMemcpyDeviceToHost, s));
-		GPHI_HIP(ctx, hipStreamSynchronize(s));
-		if (hc->done) break;
-		// every step lowers some distance, and distances are bounded
-		if (enq > (1u << 20)) return set_error(ctx, GPHI_E_STATE, "SSSP batch did not terminate");
-	}
-	if (timing) GPHI_HIP(ctx, hipEventRecord(ctx->ev[1], s));
+	ssspb_clear_kernel<<<(unsigned)std::min<uint64_t>((items + kBlock - 1) / kBlock, 16384), kBlock, 0, s>>>(t, G.n_words);
+	SsspSeeds seeds = {};
+	std::copy(srcs, srcs + k, seeds.src);
+	ssspb_seed_kernel<<<1, 64, 0, s>>>(t, seeds, k);
+	auto advance = [&](uint32_t level) {
+		if (adv == 256)
+			ssspb_advance_kernel<256><<<nblk, 256, 0, s>>>(t, level);
+		else
+			ssspb_advance_kernel<1024><<<nblk, 1024, 0, s>>>(t, level);
+	};
+	advance(UINT32_MAX);  // opens level 0: the sources
+	// every step lowers some distance, and distances are bounded
+	rc = follow_levels(ctx, [&](uint32_t level) -> int {
+		if (level > (1u << 20)) return set_error(ctx, GPHI_E_STATE, "SSSP batch did not terminate");
+		if (gr->in_w8)
+			ssspb_expand_kernel<true><<<grid, kBlock, 0, s>>>(t, level);
+		else
+			ssspb_expand_kernel<false><<<grid, kBlock, 0, s>>>(t, level);
+		advance(level);
+		return GPHI_OK;
+	});
+	if (rc) return rc;
 	bool any_row = false;
 	for (uint32_t i = 0; rows && i < k; ++i) any_row |= rows[i] != nullptr;
 	if (any_row && (rc = out_sssp_rows(gr, k, rows))) return rc;
-	GPHI_HIP(ctx, hipStreamSynchronize(s));
 	if (st) {
-		st->steps = hc->level;
-		if (timing) {
-			float ms = 0.f;
-			if (hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[1]) == hipSuccess) st->total_ms = ms;
-		}
+		st->steps = ctx->h_board->levels;
+		st->total_ms = board_ms(ctx);
 	}
 	return GPHI_OK;
 }
