@@ -7,9 +7,9 @@
 //   update      : frontier bookkeeping + direction rule (update_dense :91-179,
 //                 update_sparse :467-509, to_dense :54-88, to_sparse :400-465,
 //                 heuristic :829-834) fused into one vertex pass
-// The same chunked tile sweep serves SSSP (apps/sssp_simd/sssp.cpp:344-445),
-// PageRank (apps/pageRank_simd/page_rank.cpp:128-199) and hop relaxation
-// (apps/bellman-ford_simd/bellman-ford.cpp:129-191).
+// The same chunked tile sweep serves SSSP (apps/sssp_simd/sssp.cpp:344-445) and
+// hop relaxation (hops.hip); PageRank (apps/pageRank_simd/page_rank.cpp:128-199)
+// sums over the in-edges.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -77,7 +77,7 @@ __global__ __launch_bounds__(kBlock) void chunk_meta_kernel(const uint32_t *__re
 	}
 }
 
-static int dmalloc(gphi_ctx *ctx, void **p, size_t bytes, uint64_t *acc)
+int dmalloc(gphi_ctx *ctx, void **p, size_t bytes, uint64_t *acc)
 {
 	if (take_injected_alloc_failure()) {
 		*p = nullptr;
@@ -436,7 +436,8 @@ void free_traversal_state(gphi_graph *gr)
 	               (void **)&gr->trace,
 	               (void **)&gr->rank, (void **)&gr->b_front,
 	               (void **)&gr->b_seen, (void **)&gr->b_next, (void **)&gr->b_level, (void **)&gr->b_sums,
-	               (void **)&gr->b_live, (void **)&gr->b_touch, (void **)&gr->b_aux, (void **)&gr->sb_dist};
+	               (void **)&gr->b_live, (void **)&gr->b_touch, (void **)&gr->b_aux, (void **)&gr->sb_dist,
+	               (void **)&gr->hop};
 	for (void **p : ps) {
 		if (*p) (void)hipFree(*p);
 		*p = nullptr;
@@ -1719,136 +1720,6 @@ int run_pagerank(gphi_graph *gr, uint32_t iters, float damping, float init, floa
 	if (rank && (rc = out_words(ctx, gr->rank, nullptr, G.n, rank))) return rc;
 	GPHI_HIP(ctx, hipStreamSynchronize(s));
 	if (ms) *ms = ctx->ev_ok ? ev_ms(ctx->ev[0], ctx->ev[1]) : 0.f;
-	return GPHI_OK;
-}
-
-// ---------------------------------------------------------------------------
-// hop relaxation (apps/bellman-ford_simd/bellman-ford.cpp:129-191): full
-// sweeps of dist[t] = min(dist[t], dist[h]+1); a sweep that lowers nothing is
-// the fixpoint, where further sweeps would change nothing.
-// ---------------------------------------------------------------------------
-// A sweep over the tile arrays in their stored (row-major) order, the
-// reference's edge order: per edge, dist[t] = min(dist[t], dist[h]+1).  The
-// tile order keeps both ends of a chunk's edges inside one row and one column
-// block, so the distance reads hit cache; only an edge that lowers dist[t]
-// issues an atomicMin.  Two chunks per block iteration with every load issued
-// before any is used; blocks of XCD x (blockIdx % 8) walk the chunks c with
-// c / 64 % 8 == x.  Heads and tails are read in their 16-bit forms where
-// exact.  changed is set to 1 when some edge lowered a distance.
-__global__ __launch_bounds__(kBlock) void hop_sweep_kernel(const uint32_t *__restrict__ heads,
-                                                           const uint32_t *__restrict__ tails,
-                                                           const uint16_t *__restrict__ heads16,
-                                                           const uint16_t *__restrict__ tails16,
-                                                           const ChunkPack *__restrict__ pack,
-                                                           uint64_t nchunks, uint32_t n, uint32_t *dist,
-                                                           uint32_t *changed)
-{
-	const uint32_t wv = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-	const uint32_t xcd = blockIdx.x % kNumXcd, slot = blockIdx.x / kNumXcd, per = gridDim.x / kNumXcd;
-	const uint64_t groups = (nchunks + 63) / 64;
-	const uint64_t mine = groups / kNumXcd + (xcd < groups % kNumXcd ? 1 : 0);  // groups g = xcd + 8i
-	const uint64_t my_chunks = mine * 64;
-	bool lowered = false;
-	for (uint64_t i = slot; i < my_chunks; i += 2 * per) {
-		uint64_t cc[2];
-		bool ok[2];
-#pragma unroll
-		for (int q = 0; q < 2; ++q) {
-			const uint64_t k = i + (uint64_t)q * per;  // k-th chunk of this XCD
-			cc[q] = ((k / 64) * kNumXcd + xcd) * 64 + k % 64;
-			ok[q] = k < my_chunks && cc[q] < nchunks;
-		}
-		uint32_t h[16], t[16];
-#pragma unroll
-		for (int q = 0; q < 2; ++q) {
-			// heads and tails in their 16-bit forms where exact (pack is null
-			// when the graph has none)
-			const uint64_t c = ok[q] ? cc[q] : 0;
-			const PackSlot pk = pack ? pack_slot(pack, (uint32_t)c, wv) : PackSlot{0u, 0u, 0u, 0u};
-			uint32_t hv[8], tv[8];
-			load_edges(pk.flags & 1u, heads, heads16, c, threadIdx.x, true, true, hv);
-			load_edges(pk.flags & 2u, tails, tails16, c, threadIdx.x, true, true, tv);
-			decode_edges(pk.flags & 1u, pk.hbase, pk.hbase, hv);
-			decode_edges(pk.flags & 2u, pk.tb0, pk.tb1, tv);
-#pragma unroll
-			for (int j = 0; j < 8; ++j) {
-				// sentinel edges (head n) and absent chunks read vertex 0 and are masked
-				const bool e = ok[q] && hv[j] < n;
-				h[8 * q + j] = e ? hv[j] : 0u;
-				t[8 * q + j] = e ? tv[j] : 0u;
-			}
-		}
-		uint32_t dh[16], dt[16];
-#pragma unroll
-		for (int j = 0; j < 16; ++j) {
-			dh[j] = dist[h[j]];
-			dt[j] = dist[t[j]];
-		}
-#pragma unroll
-		for (int j = 0; j < 16; ++j) {
-			const bool e = ok[j / 8] && h[j] != t[j];
-			const uint32_t nd = dh[j] + 1;
-			if (e && (int32_t)nd < (int32_t)dt[j] && nd < atomicMin(dist + t[j], nd)) lowered = true;
-		}
-	}
-	// a plain store of 1, not an atomic: every writer stores the same value,
-	// and thousands of wavefronts would queue on one counter
-	if (__ballot(lowered) && lane_id() == 0) *changed = 1u;
-}
-
-int run_bellman_ford(gphi_graph *gr, uint32_t src, uint32_t max_sweeps, uint32_t *dist,
-                     uint32_t *sweeps_run, float *ms)
-{
-	gphi_ctx *ctx = gr->ctx;
-	DevGraph &G = gr->g;
-	if (src >= G.n) return set_error(ctx, GPHI_E_RANGE, "source %u >= N %u", src, G.n);
-	if (!G.has_tiles) return set_error(ctx, GPHI_E_STATE, "graph has no tile arrays");
-	hipStream_t s = ctx->stream;
-	int rc;
-	if (!gr->dist && (rc = dmalloc(ctx, (void **)&gr->dist, (size_t)G.n_pad * 4, nullptr))) return rc;
-	// one "lowered something" counter per sweep of a batch; the batch size,
-	// not max_sweeps, sizes the buffer
-	constexpr uint32_t kBatch = 4;
-	uint32_t *counts = nullptr;
-	if ((rc = dmalloc(ctx, (void **)&counts, kBatch * 4, nullptr))) return rc;
-	if (ctx->ev_ok) GPHI_HIP(ctx, hipEventRecord(ctx->ev[0], s));
-	fill_u32_kernel<<<grid_for(G.n_pad, kBlock, 4096), kBlock, 0, s>>>(gr->dist, G.n_pad, INT_MAX - 2);
-	uint32_t zero = 0;
-	GPHI_HIP(ctx, hipMemcpyAsync(gr->dist + src, &zero, 4, hipMemcpyHostToDevice, s));
-	const unsigned grid = kBfsDenseGrid;
-	uint32_t done = 0, run = 0;
-	uint32_t hcnt[kBatch];
-	int err = GPHI_OK;
-	while (run < max_sweeps && !done) {
-		const uint32_t nb = std::min<uint32_t>(kBatch, max_sweeps - run);
-		hipError_t e = hipMemsetAsync(counts, 0, kBatch * 4, s);
-		for (uint32_t k = 0; k < nb && e == hipSuccess; ++k) {
-			hop_sweep_kernel<<<grid, kBlock, 0, s>>>(G.heads, G.tails, G.heads16, G.tails16,
-			                                       G.heads16 ? G.pack : nullptr, G.nchunks, G.n, gr->dist,
-			                                       counts + k);
-			e = hipGetLastError();
-		}
-		if (e == hipSuccess) e = hipMemcpyAsync(hcnt, counts, nb * 4, hipMemcpyDeviceToHost, s);
-		if (e == hipSuccess) e = hipStreamSynchronize(s);
-		if (e != hipSuccess) {
-			err = hip_fail(ctx, e, "hop relaxation batch", __FILE__, __LINE__);
-			break;
-		}
-		for (uint32_t k = 0; k < nb; ++k) {
-			++run;
-			if (hcnt[k] == 0) {
-				done = 1;
-				break;
-			}
-		}
-	}
-	(void)hipFree(counts);
-	if (err) return err;
-	if (ctx->ev_ok) GPHI_HIP(ctx, hipEventRecord(ctx->ev[1], s));
-	if (dist && (rc = out_words(ctx, gr->dist, nullptr, G.n, dist))) return rc;
-	GPHI_HIP(ctx, hipStreamSynchronize(s));
-	if (ms) *ms = ctx->ev_ok ? ev_ms(ctx->ev[0], ctx->ev[1]) : 0.f;
-	if (sweeps_run) *sweeps_run = run;
 	return GPHI_OK;
 }
 

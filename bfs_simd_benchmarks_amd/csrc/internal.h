@@ -261,6 +261,8 @@ struct gphi_graph {
 	// multi-source SSSP (sssp_batch.hip): kSsspBatchMax distances per vertex
 	// (vertex-major, n_pad rows), then the sources
 	uint32_t *sb_dist = nullptr;
+	// hop relaxation (hops.hip): sweep records, row sweeps, vertex stamps
+	uint8_t *hop = nullptr;
 	// in-edge arrays of the pull steps (built once, independent of W and S)
 	uint32_t *in_off = nullptr, *in_src = nullptr;
 	// the weights of in_src's edges (build_in_weights): 1 byte when every
@@ -278,7 +280,10 @@ int set_error(gphi_ctx *ctx, int code, const char *fmt, ...);
 bool take_injected_alloc_failure();
 int hip_fail(gphi_ctx *ctx, hipError_t e, const char *what, const char *file, int line);
 
-// device-side entry points (device.hip)
+// device memory (GPHI_E_OOM when it is exhausted); *acc, if any, counts the bytes
+int dmalloc(gphi_ctx *ctx, void **p, size_t bytes, uint64_t *acc);
+
+// device-side entry points (device.hip, hops.hip)
 int upload_graph(gphi_ctx *ctx, const gphi_graph_desc *d, gphi_graph *gr);
 void free_graph_device(gphi_graph *gr);
 void free_traversal_state(gphi_graph *gr);
