@@ -172,6 +172,11 @@ __global__ __launch_bounds__(kBlock) void pack_chunks_kernel(const uint32_t *__r
 	}
 }
 
+void fill_words(gphi_ctx *ctx, uint32_t *p, uint64_t count, uint32_t value)
+{
+	fill_u32_kernel<<<grid_for(count, kBlock, 4096), kBlock, 0, ctx->stream>>>(p, count, value);
+}
+
 // largest weight, then the 8-bit copy of the tile-order weights
 __global__ __launch_bounds__(kBlock) void max_u32_kernel(const uint32_t *__restrict__ a, uint64_t n, uint32_t *out)
 {
@@ -1462,264 +1467,6 @@ int run_sssp(gphi_graph *gr, uint32_t src, uint32_t *dist, gphi_stats *st)
 		st->reached = 0;
 		st->edges_traversed = 0;
 	}
-	return GPHI_OK;
-}
-
-// ---------------------------------------------------------------------------
-// PageRank (FP32): contrib = rank/deg; sum[t] += contrib[h] over the
-// in-edges; rank = (1-d)/N + d*sum   (apps/pageRank_simd/page_rank.cpp:128-199,428-446)
-// ---------------------------------------------------------------------------
-__global__ void pr_prepare_kernel(uint32_t n, const float *__restrict__ rank, const uint32_t *__restrict__ deg,
-                                  float *__restrict__ contrib, float *__restrict__ sum)
-{
-	uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-	if (v < n) {
-		uint32_t d = deg[v];
-		contrib[v] = d ? rank[v] / (float)d : 0.f;
-		sum[v] = 0.f;
-	}
-}
-
-// PageRank sum (apps/pageRank_simd/page_rank.cpp:128-199 gathers
-// rank[h]/deg[h] into sum[t] over stripes of tile rows, each tile column
-// owned by one thread) over head bands (build_pr_bands), in band order, each
-// band adding its in-edges of every tail to sum[t].  A band's gathers all
-// fall in its window of contrib, which stays in L2, instead of spreading over
-// the whole vector.  The FP32 additions run in a fixed order, so an
-// iteration gives the same bits on every run: sum[t] = ((0 + band 0) +
-// band 1) + ...; a small pair is summed by one lane in edge order; within a
-// light pair kPullGroup lanes add in-edges g, g + kPullGroup, ... in turn and
-// the group adds its lanes in a fixed butterfly; a heavy pair's pieces (a
-// wavefront each, rounds of kPrUnroll * 64 in-edges) are summed the same way,
-// a one-piece pair's straight into sum, the others' into psum, which
-// pr_multi_kernel then adds in piece order (lane j takes pieces j, j + 64,
-// ..., then the butterfly).  Every tail appears at most once per band, so
-// the adds of one band never meet on a tail.  All loads of a lane are issued
-// before any gathered value is used.
-constexpr uint32_t kPullGroup = 8;
-constexpr uint32_t kPrSlots = kPullLight / kPullGroup;  // in-edges per lane of a light pair
-constexpr uint32_t kPrUnroll = 8;                       // loads in flight per lane of a heavy piece
-constexpr uint32_t kPrLightPerBlock = kBlock / kPullGroup;
-constexpr uint32_t kPrPiecesPerBlock = kBlock / 64;
-
-__global__ __launch_bounds__(kBlock) void pr_small_kernel(PrBand b, const uint32_t *__restrict__ lt,
-                                                          const uint32_t *__restrict__ llo,
-                                                          const uint8_t *__restrict__ lcnt,
-                                                          const uint32_t *__restrict__ src,
-                                                          const float *__restrict__ contrib, float *__restrict__ sum)
-{
-	const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-	if (i >= b.nsmall) return;
-	const uint32_t t = lt[b.small0 + i], lo = llo[b.small0 + i], cnt = lcnt[b.small0 + i];
-	uint32_t h[kPrSmall];
-#pragma unroll
-	for (uint32_t j = 0; j < kPrSmall; ++j) h[j] = j < cnt ? src[lo + j] : 0xFFFFFFFFu;
-	float c[kPrSmall];
-#pragma unroll
-	for (uint32_t j = 0; j < kPrSmall; ++j) c[j] = h[j] != 0xFFFFFFFFu ? contrib[h[j]] : 0.f;
-	float acc = 0.f;
-#pragma unroll
-	for (uint32_t j = 0; j < kPrSmall; ++j) acc += c[j];
-	sum[t] += acc;
-}
-
-__global__ __launch_bounds__(kBlock) void pr_light_kernel(PrBand b, const uint32_t *__restrict__ lt,
-                                                          const uint32_t *__restrict__ llo,
-                                                          const uint8_t *__restrict__ lcnt,
-                                                          const uint32_t *__restrict__ src,
-                                                          const float *__restrict__ contrib, float *__restrict__ sum)
-{
-	const uint32_t i = blockIdx.x * kPrLightPerBlock + threadIdx.x / kPullGroup, g = threadIdx.x % kPullGroup;
-	uint32_t t = 0, lo = 0, cnt = 0;
-	if (i < b.nlight) {
-		t = lt[b.light0 + i];
-		lo = llo[b.light0 + i];
-		cnt = lcnt[b.light0 + i];
-	}
-	uint32_t h[kPrSlots];
-#pragma unroll
-	for (uint32_t j = 0; j < kPrSlots; ++j) {
-		const uint32_t k = j * kPullGroup + g;
-		h[j] = k < cnt ? src[lo + k] : 0xFFFFFFFFu;
-	}
-	float c[kPrSlots];
-#pragma unroll
-	for (uint32_t j = 0; j < kPrSlots; ++j) c[j] = h[j] != 0xFFFFFFFFu ? contrib[h[j]] : 0.f;
-	float acc = 0.f;
-#pragma unroll
-	for (uint32_t j = 0; j < kPrSlots; ++j) acc += c[j];
-#pragma unroll
-	for (int o = kPullGroup / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, kPullGroup);
-	if (g == 0 && cnt) sum[t] += acc;
-}
-
-__device__ __forceinline__ float wave_sum_f32(float x)
-{
-	// xor butterfly: lanes l and l^o add the same two values, so every lane
-	// ends with the same bits
-#pragma unroll
-	for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-	return x;
-}
-
-// One piece p of a heavy pair, by one wavefront.  With kHot, heads below
-// `hot` read their contributions from s_hot (LDS) instead of contrib; the
-// values and their order are the same either way.
-template <bool kHot>
-__device__ __forceinline__ void pr_piece(uint32_t p, uint32_t lane, const uint4 *__restrict__ hp,
-                                         const uint32_t *__restrict__ pc, const uint32_t *__restrict__ src,
-                                         const float *__restrict__ contrib, const float *s_hot, uint32_t hot,
-                                         float *__restrict__ sum, float *__restrict__ psum)
-{
-	const uint32_t hi = pc[p];
-	const uint4 r = hp[hi];  // tail, first edge, count, first piece
-	const uint32_t k = p - r.w, e0 = r.y + k * kPullPiece, cnt = min(kPullPiece, r.z - k * kPullPiece);
-	float acc = 0.f;
-	for (uint32_t off = 0; off < cnt; off += 64 * kPrUnroll) {
-		uint32_t hh[kPrUnroll];
-#pragma unroll
-		for (uint32_t u = 0; u < kPrUnroll; ++u) {
-			const uint32_t j = off + u * 64 + lane;
-			hh[u] = j < cnt ? src[e0 + j] : 0xFFFFFFFFu;
-		}
-		float c[kPrUnroll];
-#pragma unroll
-		for (uint32_t u = 0; u < kPrUnroll; ++u) {
-			if (kHot && hh[u] < hot)
-				c[u] = s_hot[hh[u]];
-			else
-				c[u] = hh[u] != 0xFFFFFFFFu ? contrib[hh[u]] : 0.f;
-		}
-#pragma unroll
-		for (uint32_t u = 0; u < kPrUnroll; ++u) acc += c[u];
-	}
-	acc = wave_sum_f32(acc);
-	if (lane == 0) {
-		if (r.z <= kPullPiece)
-			sum[r.x] += acc;  // the pair's only piece
-		else
-			psum[p] = acc;
-	}
-}
-
-__global__ __launch_bounds__(kBlock) void pr_piece_kernel(PrBand b, const uint4 *__restrict__ hp,
-                                                          const uint32_t *__restrict__ pc,
-                                                          const uint32_t *__restrict__ src,
-                                                          const float *__restrict__ contrib, float *__restrict__ sum,
-                                                          float *__restrict__ psum)
-{
-	const uint32_t q = blockIdx.x * kPrPiecesPerBlock + (threadIdx.x >> 6);
-	if (q >= b.npieces) return;  // uniform per wavefront
-	pr_piece<false>(b.piece0 + q, threadIdx.x & 63, hp, pc, src, contrib, nullptr, 0, sum, psum);
-}
-
-// The pieces of the first band (heads from 0), whose lowest heads, the
-// highest out-degrees after the degree reordering, carry a large share of
-// its in-edges: every block first copies the contributions of heads below
-// kPrHot into LDS (144 KiB, one block per CU), so those gathers skip L2,
-// then walks the pieces, a wavefront each.
-constexpr uint32_t kPrHot = 36864;
-constexpr uint32_t kPrHotBlock = 1024;
-
-__global__ __launch_bounds__(kPrHotBlock) void pr_piece_hot_kernel(PrBand b, const uint4 *__restrict__ hp,
-                                                                   const uint32_t *__restrict__ pc,
-                                                                   const uint32_t *__restrict__ src,
-                                                                   const float *__restrict__ contrib,
-                                                                   float *__restrict__ sum, float *__restrict__ psum)
-{
-	__shared__ float s_hot[kPrHot];
-	const uint32_t hot = min(kPrHot, b.head_hi);  // head_lo is 0
-	for (uint32_t i = threadIdx.x; i < hot; i += kPrHotBlock) s_hot[i] = contrib[i];
-	__syncthreads();
-	constexpr uint32_t kWaves = kPrHotBlock / 64;
-	for (uint32_t q = blockIdx.x * kWaves + (threadIdx.x >> 6); q < b.npieces; q += gridDim.x * kWaves)
-		pr_piece<true>(b.piece0 + q, threadIdx.x & 63, hp, pc, src, contrib, s_hot, hot, sum, psum);
-}
-
-// a wavefront per heavy pair of more than one piece: its pieces' sums in
-// piece order
-__global__ __launch_bounds__(kBlock) void pr_multi_kernel(PrBand b, const uint32_t *__restrict__ multi,
-                                                          const uint4 *__restrict__ hp,
-                                                          const float *__restrict__ psum, float *__restrict__ sum)
-{
-	const uint32_t lane = threadIdx.x & 63;
-	const uint32_t q = blockIdx.x * kPrPiecesPerBlock + (threadIdx.x >> 6);
-	if (q >= b.nmulti) return;  // uniform per wavefront
-	const uint4 r = hp[multi[b.multi0 + q]];
-	const uint32_t np = (r.z + kPullPiece - 1) / kPullPiece;
-	float s = 0.f;
-	for (uint32_t j = lane; j < np; j += 64) s += psum[r.w + j];
-	s = wave_sum_f32(s);
-	if (lane == 0) sum[r.x] += s;
-}
-
-// rank = (1-d)/N + d*sum (page_rank.cpp:428-446), the next iteration's
-// contributions rank/deg, and sum cleared for it, in one pass
-__global__ void pr_apply_kernel(uint32_t n, float first, float damping, float *__restrict__ sum,
-                                const uint32_t *__restrict__ deg, float *__restrict__ rank,
-                                float *__restrict__ contrib)
-{
-	uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-	if (v < n) {
-		const float r = first + damping * sum[v];
-		sum[v] = 0.f;
-		rank[v] = r;
-		const uint32_t d = deg[v];
-		contrib[v] = d ? r / (float)d : 0.f;
-	}
-}
-
-int run_pagerank(gphi_graph *gr, uint32_t iters, float damping, float init, float *rank, float *ms)
-{
-	gphi_ctx *ctx = gr->ctx;
-	DevGraph &G = gr->g;
-	hipStream_t s = ctx->stream;
-	int rc;
-	if ((rc = build_in_edges(gr))) return rc;
-	if ((rc = build_pr_bands(gr))) return rc;
-	if (!gr->rank) {
-		// rank, sum, contrib (n_pad each), then the partial sums of the pieces
-		const size_t bytes = 3 * (size_t)G.n_pad * 4 + ((size_t)gr->pr_npieces + 1) * 4;
-		if ((rc = dmalloc(ctx, (void **)&gr->rank, bytes, nullptr))) return rc;
-		gr->sum = gr->rank + G.n_pad;
-		gr->contrib = gr->sum + G.n_pad;
-	}
-	float *psum = gr->contrib + G.n_pad;
-	uint32_t bits;
-	memcpy(&bits, &init, 4);
-	fill_u32_kernel<<<grid_for(G.n, kBlock, 4096), kBlock, 0, s>>>((uint32_t *)gr->rank, G.n, bits);
-	const float first = (1.0f - damping) / (float)G.n;
-	unsigned vgrid = grid_for(G.n, kBlock, 1u << 30);
-	static const unsigned hot_grid = resident_grid((const void *)pr_piece_hot_kernel, kPrHotBlock);
-	if (ctx->ev_ok) GPHI_HIP(ctx, hipEventRecord(ctx->ev[0], s));
-	pr_prepare_kernel<<<vgrid, kBlock, 0, s>>>(G.n, gr->rank, G.deg, gr->contrib, gr->sum);
-	for (uint32_t it = 0; it < iters; ++it) {
-		for (const PrBand &b : gr->pr_bands) {
-			if (b.nsmall)
-				pr_small_kernel<<<(b.nsmall + kBlock - 1) / kBlock, kBlock, 0, s>>>(
-				    b, gr->pr_lt, gr->pr_llo, gr->pr_lcnt, gr->pr_src, gr->contrib, gr->sum);
-			if (b.nlight)
-				pr_light_kernel<<<(b.nlight + kPrLightPerBlock - 1) / kPrLightPerBlock, kBlock, 0, s>>>(
-				    b, gr->pr_lt, gr->pr_llo, gr->pr_lcnt, gr->pr_src, gr->contrib, gr->sum);
-			if (b.npieces && b.head_lo == 0)
-				pr_piece_hot_kernel<<<std::min<unsigned>(hot_grid, (b.npieces + kPrHotBlock / 64 - 1) /
-				                                                      (kPrHotBlock / 64)),
-				                      kPrHotBlock, 0, s>>>(b, gr->pr_hp, gr->pr_pc, gr->pr_src, gr->contrib,
-				                                           gr->sum, psum);
-			else if (b.npieces)
-				pr_piece_kernel<<<(b.npieces + kPrPiecesPerBlock - 1) / kPrPiecesPerBlock, kBlock, 0, s>>>(
-				    b, gr->pr_hp, gr->pr_pc, gr->pr_src, gr->contrib, gr->sum, psum);
-			if (b.nmulti)
-				pr_multi_kernel<<<(b.nmulti + kPrPiecesPerBlock - 1) / kPrPiecesPerBlock, kBlock, 0, s>>>(
-				    b, gr->pr_multi, gr->pr_hp, psum, gr->sum);
-		}
-		pr_apply_kernel<<<vgrid, kBlock, 0, s>>>(G.n, first, damping, gr->sum, G.deg, gr->rank, gr->contrib);
-	}
-	GPHI_HIP(ctx, hipGetLastError());
-	if (ctx->ev_ok) GPHI_HIP(ctx, hipEventRecord(ctx->ev[1], s));
-	if (rank && (rc = out_words(ctx, gr->rank, nullptr, G.n, rank))) return rc;
-	GPHI_HIP(ctx, hipStreamSynchronize(s));
-	if (ms) *ms = ctx->ev_ok ? ev_ms(ctx->ev[0], ctx->ev[1]) : 0.f;
 	return GPHI_OK;
 }
 

@@ -158,26 +158,23 @@ struct DevGraph {
 };
 
 // PageRank head bands (build_pr_bands).  The heads are cut into bands
-// [head_lo, head_hi); within a band, the in-edges of a tail whose heads lie
-// in it form a pair (tail, first edge, count).  A small pair has 1..kPrSmall
-// in-edges, a light pair up to kPullLight, a heavy pair more, split into
-// pieces of kPullPiece; the heavy pairs of more than one piece are also
-// listed apart (multi).  Each class is in tail order; indices are global
-// over the band arrays.  The heads are copied band by band (pr_src): a
-// band's small pairs' heads from edge_small on, its light pairs' from
-// edge_light, its heavy pairs' from edge_heavy, each pair's ascending, so a
-// band's sweep streams one contiguous run of the copy.
+// [head_lo, head_hi); within a band, the in-edges of a tail whose heads lie in
+// it form a segment.  A band's segments are in tail order and its edges, in
+// segment order with heads ascending, one contiguous run of pr_src, swept in
+// tiles of kPrTile.  Indices are global over the band arrays; a band's
+// segments end with a sentinel (its edge end), its tiles with the last segment.
 constexpr uint32_t kSsspBatchMax = GPHI_SSSP_BATCH_MAX;  // distances per vertex of the SSSP batch
+constexpr uint32_t kPrTile = 2048;
 constexpr uint32_t kBandHeads = 1u << 19;  // heads per band window: 2 MiB of FP32 contributions
-constexpr uint32_t kPrSmall = 8;           // in-edges a lane sums alone
+// vertices up to which one band is swept: two bands at 1.6M vertices x 21 take
+// 124 us an iteration instead of 117, eight at 4.2M x 16 311 instead of 309, and
+// twice the set-up
+constexpr uint32_t kPrOneBand = 1u << 22;
 struct PrBand {
 	uint32_t head_lo, head_hi;
-	uint32_t small0, nsmall;
-	uint32_t light0, nlight;
-	uint32_t heavy0, nheavy;
-	uint32_t piece0, npieces;
-	uint32_t multi0, nmulti;
-	uint32_t edge_small, edge_light, edge_heavy;
+	uint32_t edge0, nedges;  // edge0 is a multiple of 4
+	uint32_t seg0, nseg;
+	uint32_t tile0, ntiles;
 };
 
 }  // namespace gphi
@@ -230,22 +227,17 @@ struct gphi_graph {
 	uint32_t *live_cnt = nullptr;
 	uint4 *trace = nullptr;    // per step: direction, |F|, sum deg(F), chunks swept
 	// PageRank: one allocation holding rank, sum and contrib (n_pad each) and
-	// the partial sums of the heavy pairs' pieces
+	// two partial sums per tile
 	float *rank = nullptr, *sum = nullptr, *contrib = nullptr;
 	// PageRank head bands (build_pr_bands; built once, independent of W and S):
-	// the heads band by band (pr_src), small and light pairs (tail, first
-	// edge in pr_src, count), heavy pairs {tail, first edge, count, first
-	// piece}, each piece's heavy pair, and the multi-piece heavy pairs; all in
-	// one allocation, pr_mem
+	// the heads band by band (pr_src; in_src itself when there is one band),
+	// each segment's first edge and tail, and the segment of each tile's first
+	// edge; one allocation, pr_mem
 	std::vector<gphi::PrBand> pr_bands;
 	void *pr_mem = nullptr;
-	uint32_t *pr_src = nullptr;
-	uint32_t *pr_lt = nullptr, *pr_llo = nullptr;
-	uint8_t *pr_lcnt = nullptr;
-	uint4 *pr_hp = nullptr;
-	uint32_t *pr_pc = nullptr, *pr_multi = nullptr;
-	uint32_t pr_npieces = 0;
-	uint64_t pr_bytes = 0;
+	const uint32_t *pr_src = nullptr;
+	uint32_t *pr_off = nullptr, *pr_tail = nullptr, *pr_tile = nullptr;
+	uint32_t pr_ntiles = 0;
 	// multi-source BFS (batch.hip): per-vertex source masks and uint8 levels
 	uint32_t batch_words = 0;  // 64-bit words per vertex the buffers were sized for
 	// leading mask words that front / next (and the touched bitmap) are known
@@ -283,7 +275,9 @@ int hip_fail(gphi_ctx *ctx, hipError_t e, const char *what, const char *file, in
 // device memory (GPHI_E_OOM when it is exhausted); *acc, if any, counts the bytes
 int dmalloc(gphi_ctx *ctx, void **p, size_t bytes, uint64_t *acc);
 
-// device-side entry points (device.hip, hops.hip)
+void fill_words(gphi_ctx *ctx, uint32_t *p, uint64_t count, uint32_t value);  // on ctx's stream
+
+// device-side entry points (device.hip, hops.hip, pagerank.hip)
 int upload_graph(gphi_ctx *ctx, const gphi_graph_desc *d, gphi_graph *gr);
 void free_graph_device(gphi_graph *gr);
 void free_traversal_state(gphi_graph *gr);
