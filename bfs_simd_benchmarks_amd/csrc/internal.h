@@ -128,6 +128,7 @@ constexpr size_t kCtrlBytes = sizeof(StepCtrl) + kLevelRing * sizeof(LevelRec);
 // 742 at 2^23 x 24 and 937 -> 951 at 2^24 x 16, where the live lists' balance
 // pays; SSSP 432 -> 167, 995 -> 773, 2914 -> 2557, 3539 -> 3319 and 4550 -> 4284,
 // 5022 -> 4572 us.
+constexpr uint32_t kTinyVerts = 8192, kTinyChunks = 32, kTinyThreads = 1024;  // one block runs all levels
 constexpr uint32_t kSmallVerts = 1u << 24;
 constexpr uint32_t kSmallChunksBfs = 1u << 15;
 constexpr uint32_t kSmallChunksSssp = 1u << 17;

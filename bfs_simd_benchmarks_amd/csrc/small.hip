@@ -239,12 +239,239 @@ __global__ __launch_bounds__(kThreads) void small_advance_kernel(Frontier t, uin
 	advance_block<kBfs, kThreads>(t, level);
 }
 
+// ---------------------------------------------------------------------------
+// tiny graphs: the whole traversal in one block
+// ---------------------------------------------------------------------------
+// With up to kTinyVerts vertices and kTinyChunks chunks of edges, a level's
+// work is smaller than the two launches it takes.  Here one block of 1024
+// threads runs all levels: frontier, visited set, queue and (SSSP) distances
+// live in LDS, a thread keeps the degrees and CSR offsets of its 8 vertices in
+// registers, and only edges, parents and levels cross to memory.  The steps,
+// the direction rule and the chunks a dense step takes are those of the
+// two-launch loop.  Whole calls, against that loop: BFS 89 -> 45 us at 1024
+// vertices (6 chunks), 106 -> 78 at 8000 (29), SSSP 175 -> 77 and 187 -> 155; past
+// 32 chunks the edges are more than one CU should read.
+struct TinyShared {
+	uint32_t cur[kTinyVerts / 32], hot[kTinyVerts / 32];  // frontier; its vertices with out-edges
+	uint32_t next[kTinyVerts / 32];                       // frontier of the next step
+	uint32_t visited[kTinyVerts / 32];                    // BFS
+	uint32_t off[kTinyVerts], base[kTinyVerts];           // queue: degree prefix, CSR offset
+	uint16_t queue[kTinyVerts];
+	uint16_t chunks[kTinyChunks];
+	uint32_t red[3][kTinyThreads / 64];
+	uint32_t nchunks;
+};
+
+// some vertex of [a, b) has its bit set in `bits` (cleared, with flip ~0), by one wavefront
+__device__ __forceinline__ bool any_bit(const uint32_t *bits, uint32_t flip, uint32_t a, uint32_t b, uint32_t lane)
+{
+	bool any = false;
+	for (uint32_t w = a / 32 + lane; w <= (b - 1) / 32; w += 64) {
+		uint32_t x = bits[w] ^ flip;
+		if (w == a / 32) x &= ~0u << (a % 32);
+		if (w == (b - 1) / 32) x &= ~0u >> (31 - (b - 1) % 32);
+		any |= x != 0;
+	}
+	return __ballot(any) != 0;
+}
+
+template <int kWeights>
+__global__ __launch_bounds__(kTinyThreads) void tiny_kernel(Trav t, uint32_t src)
+{
+	constexpr bool kBfs = kWeights == 0;
+	constexpr uint32_t kOwn = kTinyVerts / kTinyThreads;
+	static_assert(kOwn == 8, "a thread's vertices are a byte of the bitmaps");
+	__shared__ TinyShared s;
+	__shared__ uint32_t s_dist[kBfs ? 1 : kTinyVerts];
+	const uint32_t tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, v0 = tid * kOwn;
+	LevelBoard *board = t.board;
+	if (tid == 0) board->t_begin = wall_clock64();
+	uint32_t d[kOwn], base[kOwn];
+#pragma unroll
+	for (uint32_t k = 0; k < kOwn; ++k) {
+		const bool in = v0 + k < t.n;
+		d[k] = in ? t.deg[v0 + k] : 0u;
+		base[k] = in ? t.row_off[v0 + k] : 0u;
+		if (!kBfs) s_dist[v0 + k] = v0 + k == src ? 0u : (uint32_t)INT_MAX;
+	}
+	uint8_t *cur8 = reinterpret_cast<uint8_t *>(s.cur), *hot8 = reinterpret_cast<uint8_t *>(s.hot);
+	uint8_t *next8 = reinterpret_cast<uint8_t *>(s.next), *vis8 = reinterpret_cast<uint8_t *>(s.visited);
+	next8[tid] = vis8[tid] = src / kOwn == tid ? (uint8_t)(1u << (src % kOwn)) : 0;
+	if (kBfs && tid == 0) {
+		t.level[src] = 0;
+		t.parent[src] = (int32_t)src;
+	}
+	unsigned long long reached = 0, traversed = 0;
+	uint32_t level = 0;
+	for (;; ++level) {
+		__syncthreads();
+		// the next frontier becomes the current one; its queue
+		const uint32_t bits = next8[tid];
+		uint32_t q = 0, dsum = 0, hot = 0;
+#pragma unroll
+		for (uint32_t k = 0; k < kOwn; ++k)
+			if (((bits >> k) & 1u) && d[k]) {
+				++q;
+				dsum += d[k];
+				hot |= 1u << k;
+			}
+		cur8[tid] = (uint8_t)bits;
+		hot8[tid] = (uint8_t)hot;
+		next8[tid] = 0;
+		uint32_t qtot, dtot;
+		uint32_t pos = wave_excl_scan(q, &qtot), off = wave_excl_scan(dsum, &dtot);
+		const uint32_t ftot = wave_sum((uint32_t)__popc(bits));
+		if (lane == 0) {
+			s.red[0][wid] = ftot;
+			s.red[1][wid] = qtot;
+			s.red[2][wid] = dtot;
+		}
+		if (tid == 0) s.nchunks = 0;
+		__syncthreads();
+		uint32_t fsize = 0, qsize = 0, fdeg = 0;
+		for (uint32_t k = 0; k < kTinyThreads / 64; ++k) {
+			if (k < wid) {
+				pos += s.red[1][k];
+				off += s.red[2][k];
+			}
+			fsize += s.red[0][k];
+			qsize += s.red[1][k];
+			fdeg += s.red[2][k];
+		}
+		if (fsize == 0) break;  // uniform
+		reached += fsize;
+		traversed += fdeg;
+#pragma unroll
+		for (uint32_t k = 0; k < kOwn; ++k)
+			if ((hot >> k) & 1u) {
+				s.queue[pos] = (uint16_t)(v0 + k);
+				s.off[pos] = off;
+				s.base[pos] = base[k];
+				++pos;
+				off += d[k];
+			}
+		const bool dense = level > 0 && fsize + fdeg > t.threshold;  // the first step is sparse
+		uint32_t nlive = 0;
+		// edge u -> v, its weight from w
+		auto relax = [&](uint32_t u, uint32_t v, uint32_t w) {
+			const uint32_t bit = 1u << (v & 31);
+			if (kBfs) {
+				if ((s.visited[v >> 5] & bit) || (atomicOr(&s.visited[v >> 5], bit) & bit)) return;
+				t.parent[v] = (int32_t)u;
+				t.level[v] = (int32_t)level + 1;
+				atomicOr(&s.next[v >> 5], bit);
+			} else {
+				const uint32_t nd = s_dist[u] + w;
+				if (nd < s_dist[v] && nd < atomicMin(&s_dist[v], nd)) atomicOr(&s.next[v >> 5], bit);
+			}
+		};
+		if (!dense) {
+			__syncthreads();
+			// the frontier's edges, one per thread and round
+			for (uint32_t e = tid; e < fdeg; e += kTinyThreads) {
+				uint32_t a = 0, b = qsize;  // last entry with off <= e
+				while (b - a > 1) {
+					const uint32_t mid = (a + b) >> 1;
+					if (s.off[mid] <= e)
+						a = mid;
+					else
+						b = mid;
+				}
+				const uint32_t x = s.base[a] + (e - s.off[a]);
+				relax(s.queue[a], t.cols[x], kBfs ? 0u : t.csr_w[x]);
+			}
+		} else {
+			// the live chunks, a wavefront per chunk
+			for (uint32_t c = wid; c < t.nchunks; c += kTinyThreads / 64) {
+				const ChunkMeta md = t.meta[c];
+				if (md.row_lo > md.row_hi) continue;
+				bool live = md.row_hi - md.row_lo >= 16 ||
+				            any_bit(s.hot, 0u, md.row_lo * t.W, (uint32_t)min((uint64_t)(md.row_hi + 1) * t.W, (uint64_t)t.n), lane);
+				if (kBfs && live)
+					live = md.col_hi - md.col_lo >= 16 ||
+					       any_bit(s.visited, ~0u, md.col_lo * t.W, (uint32_t)min((uint64_t)(md.col_hi + 1) * t.W, (uint64_t)t.n), lane);
+				if (live && lane == 0) s.chunks[atomicAdd(&s.nchunks, 1u)] = (uint16_t)c;
+			}
+			__syncthreads();
+			nlive = s.nchunks;
+			// 4 edges per thread and round; padding edges have head n
+			constexpr uint32_t kQuads = kChunk / 4;
+			for (uint32_t x = tid; x < nlive * kQuads; x += kTinyThreads) {
+				const uint32_t at = s.chunks[x / kQuads] * kQuads + x % kQuads;
+				const uint4 h4 = reinterpret_cast<const uint4 *>(t.heads)[at];
+				const uint4 t4 = reinterpret_cast<const uint4 *>(t.tails)[at];
+				const uint32_t h[4] = {h4.x, h4.y, h4.z, h4.w}, v[4] = {t4.x, t4.y, t4.z, t4.w};
+				uint32_t w[4] = {0u, 0u, 0u, 0u};
+				if (kWeights == 1) {
+					const uint32_t w4 = reinterpret_cast<const uint32_t *>(t.coo_w8)[at];
+					w[0] = w4 & 0xFFu, w[1] = (w4 >> 8) & 0xFFu, w[2] = (w4 >> 16) & 0xFFu, w[3] = w4 >> 24;
+				} else if (kWeights == 4) {
+					const uint4 w4 = reinterpret_cast<const uint4 *>(t.coo_w)[at];
+					w[0] = w4.x, w[1] = w4.y, w[2] = w4.z, w[3] = w4.w;
+				}
+#pragma unroll
+				for (int j = 0; j < 4; ++j)
+					if (h[j] < t.n && ((s.cur[h[j] >> 5] >> (h[j] & 31)) & 1u)) relax(h[j], v[j], w[j]);
+			}
+		}
+		if (tid == 0 && level < GPHI_MAX_STEPS) {
+			uint4 *tr = board->trace + level;
+			tr->x = dense;
+			tr->y = fsize;
+			tr->z = fdeg;
+			tr->w = nlive;
+		}
+	}
+	// what the two-launch loop leaves in memory: state bytes, or distances
+	if (kBfs) {
+		const uint32_t b = vis8[tid];
+		uint2 f = make_uint2(0, 0);
+#pragma unroll
+		for (int k = 0; k < 4; ++k) {
+			f.x |= (((b >> k) & 1u) ? (uint32_t)kVisited : 0u) << (8 * k);
+			f.y |= (((b >> (4 + k)) & 1u) ? (uint32_t)kVisited : 0u) << (8 * k);
+		}
+		if (v0 < t.n_pad) reinterpret_cast<uint2 *>(t.flag)[tid] = f;
+	} else {
+#pragma unroll
+		for (uint32_t k = 0; k < kOwn; ++k)
+			if (v0 + k < t.n_pad) t.dist[v0 + k] = s_dist[v0 + k];
+	}
+	if (tid == 0) {
+		board->reached = reached;
+		board->traversed = traversed;
+		board->levels = level;
+		board->t_end = wall_clock64();
+		__hip_atomic_store(&board->progress, 3ull, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+	}
+}
+
 }  // namespace
 
 // whether the loop is the faster one (kSmallVerts)
 bool small_graph(const DevGraph &G, bool bfs)
 {
 	return G.n <= kSmallVerts && G.nchunks <= (bfs ? kSmallChunksBfs : kSmallChunksSssp);
+}
+
+static void small_stats(const gphi_ctx *ctx, gphi_stats *st, uint32_t *steps)
+{
+	const LevelBoard *board = ctx->h_board;
+	if (steps) *steps = board->levels;
+	if (st) {
+		const uint32_t ns = std::min<uint32_t>(board->levels, GPHI_MAX_STEPS);
+		st->steps = ns;
+		for (uint32_t k = 0; k < ns; ++k) {
+			const uint4 r = board->trace[k];
+			st->dir[k] = r.x;
+			st->fsize[k] = r.y;
+			st->fdeg[k] = r.z;
+			st->chunks[k] = r.w;
+		}
+		st->reached = board->reached;
+		st->edges_traversed = board->traversed;
+		st->total_ms = board_ms(ctx);
+	}
 }
 
 template <bool kBfs>
@@ -264,6 +491,21 @@ int small_level_loop(gphi_graph *gr, uint32_t src, gphi_stats *st, uint32_t *ste
 	t.heads16 = G.heads16, t.tails16 = G.tails16, t.coo_w8 = G.coo_w8;
 	t.meta = G.meta, t.pack = G.pack;
 	t.parent = gr->parent, t.dist = gr->dist;
+	if (G.n <= kTinyVerts && G.nchunks <= kTinyChunks) {
+		reset_board(board);
+		if (kBfs)
+			tiny_kernel<0><<<1, kTinyThreads, 0, s>>>(t, src);
+		else if (G.coo_w8)
+			tiny_kernel<1><<<1, kTinyThreads, 0, s>>>(t, src);
+		else
+			tiny_kernel<4><<<1, kTinyThreads, 0, s>>>(t, src);
+		GPHI_HIP(ctx, hipGetLastError());
+		unsigned long long p;
+		const int rc = wait_progress(ctx, &board->progress, 0, &p);
+		if (rc) return rc;
+		small_stats(ctx, st, steps);
+		return GPHI_OK;
+	}
 	// Every block is resident at once.  A block takes runs of chunks, as long
 	// as they leave no block with more than a tenth over its share.
 	static const unsigned resident[3] = {resident_grid(reinterpret_cast<const void *>(small_expand_kernel<0>)),
@@ -295,21 +537,7 @@ int small_level_loop(gphi_graph *gr, uint32_t src, gphi_stats *st, uint32_t *ste
 		return GPHI_OK;
 	});
 	if (rc) return rc;
-	if (steps) *steps = board->levels;
-	if (st) {
-		const uint32_t ns = std::min<uint32_t>(board->levels, GPHI_MAX_STEPS);
-		st->steps = ns;
-		for (uint32_t k = 0; k < ns; ++k) {
-			const uint4 r = board->trace[k];
-			st->dir[k] = r.x;
-			st->fsize[k] = r.y;
-			st->fdeg[k] = r.z;
-			st->chunks[k] = r.w;
-		}
-		st->reached = board->reached;
-		st->edges_traversed = board->traversed;
-		st->total_ms = board_ms(ctx);
-	}
+	small_stats(ctx, st, steps);
 	return GPHI_OK;
 }
 template int small_level_loop<true>(gphi_graph *, uint32_t, gphi_stats *, uint32_t *);

@@ -1,5 +1,6 @@
-"""The two-launch level loop of small graphs (per-level timing off): levels,
-parents, trace and distances against the oracle where its shares can go wrong
+"""The level loops of small graphs (per-level timing off), two launches per
+level and, up to 8192 vertices and 32 chunks of 2048 edges, one launch in all:
+levels, parents, trace and distances against the oracle where they can go wrong
 -- vertex counts around a lane's 8, a wavefront's 512 and a block's 2048 or
 8192 vertices, tile widths that split a lane's vertices, chunk counts around
 a block's share, frontiers without out-edges, and paths past the ring of
@@ -40,7 +41,7 @@ def upload(ctx, g, weighted=False):
 
 
 @pytest.mark.parametrize("n,m,W,S", [(7, 9, 2, 1), (8, 20, 3, 2), (511, 1500, 12, 4), (512, 2048, 64, 2),
-                                     (2049, 9000, 100, 3), (8191, 40000, 512, 4), (8193, 200000, 1000, 8),
+                                     (2049, 9000, 100, 3), (8191, 40000, 512, 4), (8192, 60000, 5, 40), (8192, 66000, 300, 4), (8193, 200000, 1000, 8),
                                      (270_001, 600_000, 1024, 16), (300_000, 4_000_000, 4096, 16)])
 def test_bfs(quiet, n, m, W, S):
     g = random_graph(n, m, W, S, n)
@@ -76,7 +77,8 @@ def test_bfs_long_path(quiet, n):
         gg.free()
 
 
-@pytest.mark.parametrize("n,m,W,S,wmax", [(7, 9, 2, 1, 1), (513, 3000, 12, 4, 255), (8193, 200000, 1000, 8, 255),
+@pytest.mark.parametrize("n,m,W,S,wmax", [(7, 9, 2, 1, 1), (513, 3000, 12, 4, 255), (8192, 50000, 70, 4, 255),
+                                          (8000, 50000, 70000, 4, 1 << 20), (8193, 200000, 1000, 8, 255),
                                           (8193, 200000, 512, 8, 1 << 20), (270_001, 2_000_000, 1024, 16, 255)])
 def test_sssp(quiet, n, m, W, S, wmax):
     g = random_graph(n, m, W, S, n + 1, wmax)
