@@ -113,6 +113,7 @@ void gphi_close(gphi_ctx *ctx)
 	if (ctx->ev_ok)
 		for (auto &ev : ctx->ev) (void)hipEventDestroy(ev);
 	if (ctx->h_ctrl) (void)hipHostFree(ctx->h_ctrl);
+	if (ctx->d_word) (void)hipFree(ctx->d_word);
 	if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
 	delete ctx;
 	gphi::out_context_closed();

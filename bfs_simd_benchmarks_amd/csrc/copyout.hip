@@ -11,6 +11,9 @@
 //             else 8, as level + 1 with 0 for unreached; widened by the host.
 //             The host's first touch of the array then sets the pace (about
 //             100 GB/s over 8 threads), not the link.
+//   distances: 4, 8 or 16 bits when the largest one fits, found by a pass over
+//             them first (from kNarrowBytes of output on), as distance + 1 with
+//             0 for unreached
 //   others  : 4-byte words as they are
 //
 // A slot is finished when the flag beside it holds its sequence number: a
@@ -42,6 +45,7 @@ constexpr uint32_t kSlots = 24;
 constexpr uint32_t kParts = 8;         // pieces of a slot the host threads take
 constexpr uint32_t kMaxHelpers = 11;   // host threads beside the caller's
 constexpr uint64_t kHelperBytes = 2u << 20;  // a helper per this much output (starting one takes about 20 us)
+constexpr uint64_t kNarrowBytes = 1u << 20;  // distances: output from which a pass for the largest pays (10 us)
 constexpr unsigned kFillGrid = 256;    // blocks that fill a slot: enough to keep the link busy
 
 __global__ void slot_done_kernel(unsigned long long *flag, unsigned long long seq)
@@ -138,10 +142,59 @@ __global__ __launch_bounds__(kBlock) void fill_words_kernel(const uint4 *__restr
 	}
 }
 
+// the largest of n distances that is not `none`, into *word (0 before)
+__global__ __launch_bounds__(kBlock) void max_dist_kernel(const uint4 *__restrict__ dist, uint64_t n, uint32_t none,
+                                                          uint32_t *word)
+{
+	uint32_t m = 0;
+	for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < n / 4; i += (uint64_t)gridDim.x * kBlock) {
+		const uint4 x = dist[i];
+		m = max(max(m, x.x == none ? 0u : x.x), x.y == none ? 0u : x.y);
+		m = max(max(m, x.z == none ? 0u : x.z), x.w == none ? 0u : x.w);
+	}
+#pragma unroll
+	for (int o = 32; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o, 64));
+	if (threadIdx.x % 64 == 0 && m) atomicMax(word, m);
+}
+// *word into the slot, and cleared for the next pass
+__global__ void report_word_kernel(uint32_t *word, uint32_t *out)
+{
+	*out = *word;
+	*word = 0;
+}
+
+__device__ __forceinline__ uint32_t dist_code(uint32_t d, uint32_t none) { return d == none ? 0u : d + 1; }
+
+// n distances from `first` (a multiple of 32), 32 per lane (the array is padded)
+template <int kBits>
+__global__ __launch_bounds__(kBlock) void fill_dist_kernel(const uint32_t *__restrict__ dist, uint32_t none,
+                                                           uint64_t first, uint64_t count, uint4 *__restrict__ out)
+{
+	for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < (count + 31) / 32;
+	     i += (uint64_t)gridDim.x * kBlock) {
+		const uint4 *p = reinterpret_cast<const uint4 *>(dist + first + i * 32);
+		constexpr int kPer = 32 / kBits;  // codes per word
+		uint32_t w[kBits];
+#pragma unroll
+		for (int j = 0; j < kBits; ++j) w[j] = 0;
+#pragma unroll
+		for (int q = 0; q < 8; ++q) {
+			const uint4 x = p[q];
+			const uint32_t d[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+			for (int j = 0; j < 4; ++j) w[(4 * q + j) / kPer] |= dist_code(d[j], none) << (kBits * ((4 * q + j) % kPer));
+		}
+#pragma unroll
+		for (int j = 0; j < kBits / 4; ++j)
+			out[i * (kBits / 4) + j] = make_uint4(w[4 * j], w[4 * j + 1], w[4 * j + 2], w[4 * j + 3]);
+	}
+}
+
 // rows of a vertex-major array (kSsspBatchMax words per vertex): a slot holds
 // the rows' values of `count` vertices from `first`, row by row; a lane per
 // vertex, so its reads share cache lines and a wavefront's writes of a row are
-// consecutive
+// consecutive.  (In 16-bit codes the rows take as long: the host's first touch
+// of them sets the pace.)
 __global__ __launch_bounds__(kBlock) void fill_vertex_rows_kernel(const uint32_t *__restrict__ src, uint32_t k,
                                                                   uint32_t first, uint32_t count,
                                                                   uint32_t *__restrict__ out)
@@ -215,6 +268,56 @@ void widen(const uint8_t *p, uint64_t i, uint64_t count, int32_t *dst)
 		for (; k + 16 <= count; k += 16) widen16(_mm_loadu_si128(reinterpret_cast<const __m128i *>(q + k)), dst + k);
 		for (; k < count; ++k) dst[k] = (int32_t)q[k] - 1;
 	}
+}
+
+// codes (distance + 1, 0 unreached) to distances: 4 words at a time
+inline __m128i decode4(__m128i x, __m128i none)
+{
+	const __m128i zero = _mm_cmpeq_epi32(x, _mm_setzero_si128());
+	return _mm_or_si128(_mm_and_si128(zero, none), _mm_andnot_si128(zero, _mm_sub_epi32(x, _mm_set1_epi32(1))));
+}
+inline void decode16(__m128i x, __m128i none, uint32_t *dst)  // 16 bytes
+{
+	const __m128i zero = _mm_setzero_si128();
+	const __m128i a = _mm_unpacklo_epi8(x, zero), b = _mm_unpackhi_epi8(x, zero);
+	__m128i *o = reinterpret_cast<__m128i *>(dst);
+	_mm_storeu_si128(o, decode4(_mm_unpacklo_epi16(a, zero), none));
+	_mm_storeu_si128(o + 1, decode4(_mm_unpackhi_epi16(a, zero), none));
+	_mm_storeu_si128(o + 2, decode4(_mm_unpacklo_epi16(b, zero), none));
+	_mm_storeu_si128(o + 3, decode4(_mm_unpackhi_epi16(b, zero), none));
+}
+
+// element i of p (kBits each) to dst, for count elements from an even element
+template <int kBits>
+void decode(const uint8_t *p, uint64_t i, uint64_t count, uint32_t none, uint32_t *dst)
+{
+	const __m128i nn = _mm_set1_epi32((int)none), low = _mm_set1_epi8(15), zero = _mm_setzero_si128();
+	const uint8_t *q = p + i * kBits / 8;
+	auto at = [&](uint64_t k) -> uint32_t {
+		if (kBits == 4) return (q[k / 2] >> (4 * (k & 1))) & 15u;
+		if (kBits == 8) return q[k];
+		return (uint32_t)q[2 * k] | (uint32_t)q[2 * k + 1] << 8;
+	};
+	uint64_t k = 0;
+	for (; k + 32 <= count; k += 32) {
+		if (kBits == 4) {
+			const __m128i x = _mm_loadu_si128(reinterpret_cast<const __m128i *>(q + k / 2));
+			const __m128i a = _mm_and_si128(x, low), b = _mm_and_si128(_mm_srli_epi16(x, 4), low);
+			decode16(_mm_unpacklo_epi8(a, b), nn, dst + k);
+			decode16(_mm_unpackhi_epi8(a, b), nn, dst + k + 16);
+		} else if (kBits == 8) {
+			decode16(_mm_loadu_si128(reinterpret_cast<const __m128i *>(q + k)), nn, dst + k);
+			decode16(_mm_loadu_si128(reinterpret_cast<const __m128i *>(q + k + 16)), nn, dst + k + 16);
+		} else {
+			for (int j = 0; j < 4; ++j) {
+				const __m128i x = _mm_loadu_si128(reinterpret_cast<const __m128i *>(q + 2 * k + 16 * j));
+				__m128i *o = reinterpret_cast<__m128i *>(dst + k + 8 * j);
+				_mm_storeu_si128(o, decode4(_mm_unpacklo_epi16(x, zero), nn));
+				_mm_storeu_si128(o + 1, decode4(_mm_unpackhi_epi16(x, zero), nn));
+			}
+		}
+	}
+	for (; k < count; ++k) dst[k] = at(k) ? at(k) - 1 : none;
 }
 
 // Pinned slots, leased for one copy-out.  Making a ring takes 0.3 ms (one
@@ -403,6 +506,46 @@ int out_level_rows(gphi_ctx *ctx, Src src, uint32_t n, uint32_t nrows, T *const 
 	    });
 }
 
+template <int kBits>
+int out_codes(gphi_ctx *ctx, const uint32_t *dev, uint32_t none, uint32_t n, uint32_t *dst)
+{
+	const uint64_t per = kSlotBytes * 8 / kBits, nslots = (n + per - 1) / per;
+	hipStream_t s = ctx->stream;
+	return stream_out(
+	    ctx, nslots, (uint64_t)n * 4,
+	    [&](uint64_t i, uint8_t *slot) {
+		    const uint64_t count = std::min<uint64_t>(per, n - i * per);
+		    fill_dist_kernel<kBits><<<fill_grid(count / 32 + 1), kBlock, 0, s>>>(dev, none, i * per, count,
+		                                                                        reinterpret_cast<uint4 *>(slot));
+	    },
+	    [&](uint64_t i, uint32_t part, const uint8_t *slot) {
+		    uint64_t lo, hi;
+		    part_range(std::min<uint64_t>(per, n - i * per), part, &lo, &hi);
+		    if (lo < hi) decode<kBits>(slot, lo, hi - lo, none, dst + i * per + lo);
+	    });
+}
+
+// the largest of n (a multiple of 4) distances that is not `none`
+int largest_dist(gphi_ctx *ctx, const uint32_t *dev, uint64_t n, uint32_t none, uint32_t *out)
+{
+	hipStream_t s = ctx->stream;
+	if (!ctx->d_word) {
+		int rc = dmalloc(ctx, (void **)&ctx->d_word, 4, nullptr);
+		if (rc) return rc;
+		fill_words(ctx, ctx->d_word, 1, 0);
+	}
+	return stream_out(
+	    ctx, 1, 4,
+	    [&](uint64_t, uint8_t *slot) {
+		    max_dist_kernel<<<(unsigned)std::min<uint64_t>(512, n / 4 / kBlock + 1), kBlock, 0, s>>>(
+		        reinterpret_cast<const uint4 *>(dev), n, none, ctx->d_word);
+		    report_word_kernel<<<1, 1, 0, s>>>(ctx->d_word, reinterpret_cast<uint32_t *>(slot));
+	    },
+	    [&](uint64_t, uint32_t part, const uint8_t *slot) {
+		    if (part == 0) memcpy(out, slot, 4);
+	    });
+}
+
 }  // namespace
 
 int out_words(gphi_ctx *ctx, const void *dev, const uint8_t *state, uint32_t n, void *dst)
@@ -442,6 +585,18 @@ int out_batch_rows(gphi_graph *gr, const uint32_t *slots, uint32_t deepest, uint
 }
 template int out_batch_rows(gphi_graph *, const uint32_t *, uint32_t, uint32_t, uint8_t *const *);
 template int out_batch_rows(gphi_graph *, const uint32_t *, uint32_t, uint32_t, int32_t *const *);
+
+int out_dist(gphi_ctx *ctx, const uint32_t *dev, uint32_t none, uint32_t n, uint32_t n_pad, uint32_t *dst)
+{
+	if ((uint64_t)n * 4 < kNarrowBytes) return out_words(ctx, dev, nullptr, n, dst);
+	uint32_t top = 0;
+	int rc = largest_dist(ctx, dev, n_pad, none, &top);
+	if (rc) return rc;
+	if (top < 15) return out_codes<4>(ctx, dev, none, n, dst);
+	if (top < 255) return out_codes<8>(ctx, dev, none, n, dst);
+	if (top < 65535) return out_codes<16>(ctx, dev, none, n, dst);
+	return out_words(ctx, dev, nullptr, n, dst);
+}
 
 int out_sssp_rows(gphi_graph *gr, uint32_t k, uint32_t *const *rows)
 {

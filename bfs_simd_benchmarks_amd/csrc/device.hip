@@ -1460,7 +1460,7 @@ int run_sssp(gphi_graph *gr, uint32_t src, uint32_t *dist, gphi_stats *st)
 	if (!gr->dist && (rc = dmalloc(ctx, (void **)&gr->dist, (size_t)G.n_pad * 4, nullptr))) return rc;
 	if (st) memset(st, 0, sizeof(*st));
 	if ((rc = frontier_loop<false>(gr, src, st, nullptr))) return rc;
-	if (dist && (rc = out_words(ctx, gr->dist, nullptr, G.n, dist))) return rc;
+	if (dist && (rc = out_dist(ctx, gr->dist, INT_MAX, G.n, G.n_pad, dist))) return rc;
 	if (st) {
 		// reached = vertices with a finite distance (a vertex may be expanded
 		// several times by a label-correcting sweep, so the trace overcounts)

@@ -241,7 +241,7 @@ int run_bellman_ford(gphi_graph *gr, uint32_t src, uint32_t max_sweeps, uint32_t
 		return GPHI_OK;
 	});
 	if (rc) return rc;
-	if (dist && (rc = out_words(ctx, gr->dist, nullptr, G.n, dist))) return rc;
+	if (dist && (rc = out_dist(ctx, gr->dist, kHopInf, G.n, G.n_pad, dist))) return rc;
 	if (ms) *ms = board_ms(ctx);
 	if (sweeps_run) *sweeps_run = ctx->h_board->levels;
 	return GPHI_OK;

@@ -191,6 +191,7 @@ struct gphi_ctx {
 	gphi::StepCtrl *h_ctrl = nullptr;
 	gphi::LevelBoard *h_board = nullptr;  // in h_ctrl's allocation, written by small.hip's kernels
 	double wall_clock_khz = 1e5;          // rate of the device wall clock
+	uint32_t *d_word = nullptr;           // a device word of copyout.hip
 	// per-step timing: [0] start, [1] init done, [2+2k] sweep k done, [3+2k] update k
 	// done, [2*MAX+4+k] chunk selection of dense step k done
 	hipEvent_t ev[3 * GPHI_MAX_STEPS + 4];
@@ -321,6 +322,8 @@ int out_bfs_levels(gphi_graph *gr, uint32_t deepest, int32_t *levels);
 // 255 (uint8) or -1 (int32)
 template <class T>
 int out_batch_rows(gphi_graph *gr, const uint32_t *slots, uint32_t deepest, uint32_t nrows, T *const *rows);
+// n distances of an array of n_pad, unreached ones `none` (in the padding too)
+int out_dist(gphi_ctx *ctx, const uint32_t *dev, uint32_t none, uint32_t n, uint32_t n_pad, uint32_t *dst);
 // the first k sources' distances of the multi-source SSSP (null rows are skipped)
 int out_sssp_rows(gphi_graph *gr, uint32_t k, uint32_t *const *rows);
 // gphi_open / gphi_close: the staging memory is freed with the last context

@@ -101,3 +101,32 @@ def test_concurrent_contexts():
     for t in ths:
         t.join()
     assert not bad
+
+
+@pytest.mark.parametrize("top", [14, 15, 254, 255, 65_534, 65_535, 70_000])
+@pytest.mark.parametrize("n", [262_144, 300_013])
+def test_distances_by_width(ctx, top, n):
+    """A star whose largest distance is `top`: 4, 8 or 16 bits per distance on
+    the way, or whole words; every third vertex is unreached."""
+    rng = np.random.default_rng(top)
+    t = np.flatnonzero(np.arange(n) % 3 != 2)[1:].astype(np.uint32)
+    w = rng.integers(1, top + 1, len(t)).astype(np.uint32)
+    w[:2] = (top, 1)
+    deg = np.zeros(n, np.uint32)
+    deg[0] = len(t)
+    g = ctx.graph_from_arrays(n, deg, W=4096, S=16, csr_edges=t, csr_weights=w)
+    g.retile(4096, 16)
+    try:
+        print(f"case: copy-out top={top} n={n}", flush=True)
+        ref = np.full(n, O.INT_MAX, np.uint32)
+        ref[0], ref[t] = 0, w
+        assert np.array_equal(g.sssp(0)[0], ref)
+        rows, _ = g.sssp_batch([0, 1, 0])
+        one = np.full(n, O.INT_MAX, np.uint32)
+        one[1] = 0
+        assert np.array_equal(rows[0], ref) and np.array_equal(rows[1], one) and np.array_equal(rows[2], ref)
+        hops = np.full(n, O.INT_MAX - 2, np.uint32)
+        hops[0], hops[t] = 0, 1
+        assert np.array_equal(g.bellman_ford(0)[0], hops)
+    finally:
+        g.free()
