@@ -1099,7 +1099,7 @@ int BatchRun::begin(gphi_graph *g, uint32_t capacity, const uint32_t *srcs, uint
 	const bool clean = prev_clean >= mask_words;
 	gr->batch_clean_words = 0;  // until this traversal ends
 	const Batch t = make_batch(gr);
-	reset_board(ctx->h_board);
+	if ((rc = reset_board(ctx))) return rc;
 	batch_clear_kernel<<<(unsigned)std::min<uint64_t>(grid_n(items), 16384), kBlock, 0, s>>>(
 	    t, mask_words, G.n_words, (1 + kLiveSlots) * kLiveStride, clean);
 	GPHI_HIP(ctx, hipGetLastError());
@@ -1187,6 +1187,7 @@ int BatchRun::step(const uint32_t *srcs, uint32_t k)
 	if (used + k > cap) return set_error(ctx, GPHI_E_ARG, "no free slot for %u more sources", k);
 	const uint32_t next_level = levels + 1;
 	const Batch t = make_batch(gr);
+	ctx->board_busy = true;
 	enqueue_expand(gr, nw, t, levels);
 	int rc = seed(srcs, k, next_level);
 	if (rc) return rc;
@@ -1196,6 +1197,7 @@ int BatchRun::step(const uint32_t *srcs, uint32_t k)
 	GPHI_HIP(ctx, hipGetLastError());
 	unsigned long long p;
 	if ((rc = wait_progress(ctx, &board->step_seq, seq - 1, &p))) return rc;
+	ctx->board_busy = false;
 	if (board->err) return set_error(ctx, GPHI_E_RANGE, "a batched BFS deeper than 254 levels does not fit uint8 levels");
 	for (uint32_t i = 0; i < nw; ++i) live[i] = board->live[i];
 	levels = next_level;

@@ -459,7 +459,8 @@ int stream_out(gphi_ctx *ctx, uint64_t nslots, uint64_t out_bytes, Fill fill, Ta
 	take_parts(true);
 	for (uint32_t i = 0; i < nh; ++i) helpers[i].join();
 	if (rc) {
-		// the device failed with fills under way: the ring is not used again
+		// fills may be under way: the ring goes back if they end, and is not used again otherwise
+		if (hipStreamSynchronize(s) == hipSuccess) return_ring(one, ring);
 		return rc;
 	}
 	return_ring(one, ring);

@@ -447,7 +447,6 @@ void free_traversal_state(gphi_graph *gr)
 		if (*p) (void)hipFree(*p);
 		*p = nullptr;
 	}
-	gr->rec = nullptr;                // inside ctrl's allocation
 	gr->sum = gr->contrib = nullptr;  // inside rank's allocation
 	gr->b_scount = nullptr;  // inside b_touch's allocation
 	gr->batch_words = 0;
@@ -512,11 +511,11 @@ static int alloc_state(gphi_graph *gr)
 	if ((rc = dmalloc(ctx, (void **)&gr->cur, (size_t)G.n_words * 4, nullptr))) return rc;
 	if ((rc = dmalloc(ctx, (void **)&gr->row_stamp, ((size_t)G.side + 1) * 4, nullptr))) return rc;
 	if ((rc = dmalloc(ctx, (void **)&gr->col_unvis, ((size_t)G.side + 1) * 4, nullptr))) return rc;
-	if ((rc = dmalloc(ctx, (void **)&gr->queue, 2 * (size_t)queue_stride(G.n_pad, G.m) * 4, nullptr))) return rc;
-	if ((rc = dmalloc(ctx, (void **)&gr->qoff, 2 * (size_t)queue_stride(G.n_pad, G.m) * 4, nullptr))) return rc;
+	gr->queue_len = queue_stride(G.n_pad, G.m);
+	if ((rc = dmalloc(ctx, (void **)&gr->queue, 2 * (size_t)gr->queue_len * 4, nullptr))) return rc;
+	if ((rc = dmalloc(ctx, (void **)&gr->qoff, 2 * (size_t)gr->queue_len * 4, nullptr))) return rc;
 	if ((rc = dmalloc(ctx, (void **)&gr->tile_lo, 2 * (size_t)tile_lo_stride(G.m) * 4, nullptr))) return rc;
-	if ((rc = dmalloc(ctx, (void **)&gr->ctrl, kCtrlBytes, nullptr))) return rc;
-	gr->rec = reinterpret_cast<LevelRec *>(gr->ctrl + 1);
+	if ((rc = dmalloc(ctx, (void **)&gr->ctrl, sizeof(StepCtrl), nullptr))) return rc;
 	const size_t list_cap = live_list_cap(G.nchunks);
 	if ((rc = dmalloc(ctx, (void **)&gr->live, list_cap * kNumXcd * 4 + 4, nullptr))) return rc;
 	if ((rc = dmalloc(ctx, (void **)&gr->live_cnt, kLiveCntBytes, nullptr))) return rc;

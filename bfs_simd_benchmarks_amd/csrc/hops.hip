@@ -234,7 +234,7 @@ int run_bellman_ford(gphi_graph *gr, uint32_t src, uint32_t max_sweeps, uint32_t
 	t.board = ctx->h_board;
 	static const unsigned resident = resident_grid(reinterpret_cast<const void *>(hop_sweep_kernel));
 	const unsigned grid = (unsigned)std::min<uint64_t>(resident, std::max<uint64_t>((G.nchunks + kHopRun - 1) / kHopRun, 1));
-	reset_board(ctx->h_board);
+	if ((rc = reset_board(ctx))) return rc;
 	hop_init_kernel<<<(unsigned)std::min<uint32_t>(G.n_pad / kBlock, 4096), kBlock, 0, s>>>(t, G.side, src);
 	rc = follow_levels(ctx, [&](uint32_t i) {
 		hop_sweep_kernel<<<grid, kBlock, 0, s>>>(t, i + 1, max_sweeps);

@@ -92,8 +92,8 @@ struct QueueBufs {
 	uint32_t *queue, *qoff, *tile_lo;  // half 0
 	uint32_t qstride, tstride;         // half 1 starts this many entries later
 };
-// an entry per vertex, or (the sparse-source queue of batch.hip) per vertex and
-// kSparseTile out-edges begun
+// an entry per vertex is enough for one traversal; the sparse-source queue of
+// batch.hip takes one per vertex and kSparseTile out-edges begun
 inline uint32_t queue_stride(uint32_t n_pad, uint64_t m) { return n_pad + (uint32_t)(m / kSparseTile); }
 inline uint32_t tile_lo_stride(uint64_t m) { return (uint32_t)(m / kSparseTile + 2); }
 
@@ -121,7 +121,8 @@ struct LevelBoard {
 	unsigned long long step_seq;        // as of the step (BatchRun::step) with this number
 	uint4 trace[GPHI_MAX_STEPS];  // per step: direction, |F|, sum deg(F), chunks swept
 };
-constexpr size_t kCtrlBytes = sizeof(StepCtrl) + kLevelRing * sizeof(LevelRec);
+// the ring lies in the memory of gphi_graph::trace, which only the five-kernel loop uses
+static_assert(kLevelRing * sizeof(LevelRec) <= (GPHI_MAX_STEPS + 1) * sizeof(uint4), "the ring fits the trace");
 // The graphs it serves (2048-edge chunks).  Measured against the five-kernel
 // loop without output: BFS 214 -> 96 us at 2^10 vertices (edge factor 16),
 // 326 -> 212 at 2^20, 549 -> 524 at 2^23 x 8, 840 -> 613 at 2^24 x 4, but 723 ->
@@ -189,7 +190,8 @@ struct gphi_ctx {
 	std::string last;
 	// pinned host control block for per-step readback
 	gphi::StepCtrl *h_ctrl = nullptr;
-	gphi::LevelBoard *h_board = nullptr;  // in h_ctrl's allocation, written by small.hip's kernels
+	gphi::LevelBoard *h_board = nullptr;  // in h_ctrl's allocation, written by the kernels of levels.h
+	bool board_busy = false;              // a traversal's kernels may still write the board
 	double wall_clock_khz = 1e5;          // rate of the device wall clock
 	uint32_t *d_word = nullptr;           // a device word of copyout.hip
 	// per-step timing: [0] start, [1] init done, [2+2k] sweep k done, [3+2k] update k
@@ -214,20 +216,21 @@ struct gphi_graph {
 	uint32_t *cur = nullptr;      // frontier bitmap of the current step
 	uint32_t *row_stamp = nullptr, *col_unvis = nullptr;
 	// sparse-step queue, two halves each (QueueBufs): queue / qoff of
-	// 2 * n_pad entries, tile_lo of 2 * (m / kSparseTile + 2)
+	// 2 * queue_len entries, tile_lo of 2 * (m / kSparseTile + 2)
 	uint32_t *queue = nullptr, *qoff = nullptr, *tile_lo = nullptr;
+	uint32_t queue_len = 0;
 	gphi::QueueBufs queue_bufs() const
 	{
-		return gphi::QueueBufs{queue, qoff, tile_lo, gphi::queue_stride(g.n_pad, g.m), gphi::tile_lo_stride(g.m)};
+		return gphi::QueueBufs{queue, qoff, tile_lo, queue_len, gphi::tile_lo_stride(g.m)};
 	}
 	gphi::StepCtrl *ctrl = nullptr;
-	gphi::LevelRec *rec = nullptr;  // in ctrl's allocation (kCtrlBytes)
+	gphi::LevelRec *rec() const { return reinterpret_cast<gphi::LevelRec *>(trace); }  // kLevelRing entries
 	uint4 *blk_cnt = nullptr;  // per update block: |F|, queue entries, degree sum
 	uint2 *blk_base = nullptr; // per update block: queue and degree prefix
 	uint2 *wave_cnt = nullptr; // per update wavefront: queue entries, degree sum
 	uint32_t *live = nullptr;  // per-XCD lists of live chunks of a dense step
 	uint32_t *live_cnt = nullptr;
-	uint4 *trace = nullptr;    // per step: direction, |F|, sum deg(F), chunks swept
+	uint4 *trace = nullptr;    // five-kernel loop, per step: direction, |F|, sum deg(F), chunks swept
 	// PageRank: one allocation holding rank, sum and contrib (n_pad each) and
 	// two partial sums per tile
 	float *rank = nullptr, *sum = nullptr, *contrib = nullptr;

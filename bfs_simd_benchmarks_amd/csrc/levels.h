@@ -236,7 +236,7 @@ inline Frontier make_frontier(gphi_graph *gr, uint32_t threshold)
 	f.flag = gr->flag, f.cur = gr->cur, f.row_stamp = gr->row_stamp;
 	f.level = gr->level, f.visited = gr->visited, f.col_unvis = gr->col_unvis;
 	f.qb = gr->queue_bufs();
-	f.rec = gr->rec;
+	f.rec = gr->rec();
 	f.board = gr->ctx->h_board;
 	return f;
 }
@@ -265,8 +265,16 @@ inline int wait_progress(gphi_ctx *ctx, const unsigned long long *word, unsigned
 	}
 }
 
-// before the kernel that opens a traversal is launched
-inline void reset_board(LevelBoard *b) { __atomic_store_n(&b->progress, 0ull, __ATOMIC_RELEASE); }
+// Before the kernel that opens a traversal is launched.  One that returned an
+// error before its end may have kernels in flight that still write the board
+// (after an end is reported none does): those are waited for.
+inline int reset_board(gphi_ctx *ctx)
+{
+	if (ctx->board_busy) GPHI_HIP(ctx, hipStreamSynchronize(ctx->stream));
+	ctx->board_busy = true;
+	__atomic_store_n(&ctx->h_board->progress, 0ull, __ATOMIC_RELEASE);
+	return GPHI_OK;
+}
 
 // enqueue(level) launches a level; until the device reports the end
 template <class F>
@@ -282,7 +290,10 @@ int follow_levels(gphi_ctx *ctx, F enqueue)
 		unsigned long long p;
 		const int rc = wait_progress(ctx, &ctx->h_board->progress, started, &p);
 		if (rc) return rc;
-		if (p & 1ull) return GPHI_OK;
+		if (p & 1ull) {
+			ctx->board_busy = false;
+			return GPHI_OK;
+		}
 		started = (uint32_t)(p >> 1);
 	}
 }

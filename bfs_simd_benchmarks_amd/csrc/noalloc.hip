@@ -48,8 +48,9 @@ __global__ __launch_bounds__(kBlock) void bfs_copy_out_kernel(uint32_t n, const 
 }
 
 // The state buffers of the BFS level loop laid out from `base` in 256-byte
-// aligned pieces, the same sizes gphi_bfs allocates; returns the bytes they
-// take.  base == nullptr only measures.
+// aligned pieces, the sizes gphi_bfs allocates but for the queue, which needs
+// no more than an entry per vertex here; returns the bytes they take.
+// base == nullptr only measures.
 size_t carve_state(const DevGraph &G, uint8_t *base, gphi_graph *t)
 {
 	size_t off = 0;
@@ -67,11 +68,11 @@ size_t carve_state(const DevGraph &G, uint8_t *base, gphi_graph *t)
 	t->cur = (uint32_t *)take((size_t)G.n_words * 4);
 	t->row_stamp = (uint32_t *)take(((size_t)G.side + 1) * 4);
 	t->col_unvis = (uint32_t *)take(((size_t)G.side + 1) * 4);
-	t->queue = (uint32_t *)take(2 * (size_t)queue_stride(G.n_pad, G.m) * 4);  // two halves (QueueBufs)
-	t->qoff = (uint32_t *)take(2 * (size_t)queue_stride(G.n_pad, G.m) * 4);
+	t->queue_len = G.n_pad;
+	t->queue = (uint32_t *)take(2 * (size_t)t->queue_len * 4);  // two halves (QueueBufs)
+	t->qoff = (uint32_t *)take(2 * (size_t)t->queue_len * 4);
 	t->tile_lo = (uint32_t *)take(2 * (size_t)tile_lo_stride(G.m) * 4);
-	t->ctrl = (StepCtrl *)take(kCtrlBytes);
-	t->rec = reinterpret_cast<LevelRec *>(t->ctrl + 1);
+	t->ctrl = (StepCtrl *)take(sizeof(StepCtrl));
 	t->live = (uint32_t *)take((size_t)live_list_capacity(G.nchunks) * kNumXcd * 4 + 4);
 	t->live_cnt = (uint32_t *)take(kLiveCntBytes);
 	t->trace = (uint4 *)take((GPHI_MAX_STEPS + 1) * sizeof(uint4));

@@ -448,10 +448,21 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_kernel(Trav t, uint32_t src
 
 }  // namespace
 
-// whether the loop is the faster one (kSmallVerts)
+// blocks of small_expand_kernel that are resident at once (bfs, 1-byte and 32-bit weights)
+static unsigned expand_resident(const DevGraph &G, bool bfs)
+{
+	static const unsigned resident[3] = {resident_grid(reinterpret_cast<const void *>(small_expand_kernel<0>)),
+	                                     resident_grid(reinterpret_cast<const void *>(small_expand_kernel<1>)),
+	                                     resident_grid(reinterpret_cast<const void *>(small_expand_kernel<4>))};
+	return resident[bfs ? 0 : G.coo_w8 ? 1 : 2];
+}
+
+// whether the loop is the faster one (kSmallVerts) and a block's list holds its
+// share of the chunks (on a card cut into partitions it may not)
 bool small_graph(const DevGraph &G, bool bfs)
 {
-	return G.n <= kSmallVerts && G.nchunks <= (bfs ? kSmallChunksBfs : kSmallChunksSssp);
+	return G.n <= kSmallVerts && G.nchunks <= (bfs ? kSmallChunksBfs : kSmallChunksSssp) &&
+	       G.nchunks <= (uint64_t)expand_resident(G, bfs) * kBlock;
 }
 
 static void small_stats(const gphi_ctx *ctx, gphi_stats *st, uint32_t *steps)
@@ -491,8 +502,9 @@ int small_level_loop(gphi_graph *gr, uint32_t src, gphi_stats *st, uint32_t *ste
 	t.heads16 = G.heads16, t.tails16 = G.tails16, t.coo_w8 = G.coo_w8;
 	t.meta = G.meta, t.pack = G.pack;
 	t.parent = gr->parent, t.dist = gr->dist;
+	int rc = reset_board(ctx);
+	if (rc) return rc;
 	if (G.n <= kTinyVerts && G.nchunks <= kTinyChunks) {
-		reset_board(board);
 		if (kBfs)
 			tiny_kernel<0><<<1, kTinyThreads, 0, s>>>(t, src);
 		else if (G.coo_w8)
@@ -501,29 +513,23 @@ int small_level_loop(gphi_graph *gr, uint32_t src, gphi_stats *st, uint32_t *ste
 			tiny_kernel<4><<<1, kTinyThreads, 0, s>>>(t, src);
 		GPHI_HIP(ctx, hipGetLastError());
 		unsigned long long p;
-		const int rc = wait_progress(ctx, &board->progress, 0, &p);
-		if (rc) return rc;
+		if ((rc = wait_progress(ctx, &board->progress, 0, &p))) return rc;
+		ctx->board_busy = false;
 		small_stats(ctx, st, steps);
 		return GPHI_OK;
 	}
 	// Every block is resident at once.  A block takes runs of chunks, as long
 	// as they leave no block with more than a tenth over its share.
-	static const unsigned resident[3] = {resident_grid(reinterpret_cast<const void *>(small_expand_kernel<0>)),
-	                                     resident_grid(reinterpret_cast<const void *>(small_expand_kernel<1>)),
-	                                     resident_grid(reinterpret_cast<const void *>(small_expand_kernel<4>))};
-	const unsigned grid = (unsigned)std::min<uint64_t>(resident[kBfs ? 0 : G.coo_w8 ? 1 : 2],
-	                                                   std::max<uint64_t>(G.nchunks, 1));
+	const unsigned grid = (unsigned)std::min<uint64_t>(expand_resident(G, kBfs), std::max<uint64_t>(G.nchunks, 1));
 	for (t.run = kDenseRun;; t.run /= 2) {
 		const uint32_t nruns = (t.nchunks + t.run - 1) / t.run;
 		t.slots = (nruns + grid - 1) / grid * t.run;
-		if (t.run == 1 || (uint64_t)t.slots * grid <= t.nchunks + t.nchunks / 10) break;
+		if (t.run == 1 || (t.slots <= kBlock && (uint64_t)t.slots * grid <= t.nchunks + t.nchunks / 10)) break;
 	}
-	if (t.slots > kBlock) return set_error(ctx, GPHI_E_STATE, "%u chunks exceed the small level loop", t.nchunks);
 	const unsigned adv = advance_threads(G.n_pad), nblk = advance_blocks(G.n_pad);
-	reset_board(board);
 	const uint64_t items = std::max<uint64_t>({G.n_pad / (kBfs ? 16 : 1), G.n_words, G.side});
 	small_init_kernel<kBfs><<<(unsigned)std::min<uint64_t>((items + kBlock - 1) / kBlock, 2048), kBlock, 0, s>>>(t, src);
-	const int rc = follow_levels(ctx, [&](uint32_t level) {
+	rc = follow_levels(ctx, [&](uint32_t level) {
 		if (kBfs)
 			small_expand_kernel<0><<<grid, kBlock, 0, s>>>(t, level);
 		else if (G.coo_w8)

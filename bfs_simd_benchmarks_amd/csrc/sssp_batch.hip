@@ -349,7 +349,7 @@ int run_sssp_batch(gphi_graph *gr, const uint32_t *srcs, uint32_t k, uint32_t *c
 	const unsigned push_blocks = (unsigned)std::min<uint64_t>(G.m / kSparseTile + 1, kSsspGrid);
 	const unsigned grid = std::max(t.heavy_blocks + light_blocks, push_blocks);
 	const unsigned adv = advance_threads(G.n_pad), nblk = advance_blocks(G.n_pad);
-	reset_board(ctx->h_board);
+	if ((rc = reset_board(ctx))) return rc;
 	const uint64_t items = std::max<uint64_t>((uint64_t)G.n_pad * kSsspBatchMax / 4, G.n_words);
 	ssspb_clear_kernel<<<(unsigned)std::min<uint64_t>((items + kBlock - 1) / kBlock, 16384), kBlock, 0, s>>>(t, G.n_words);
 	SsspSeeds seeds = {};

@@ -5,6 +5,8 @@ levels, parents, trace and distances against the oracle where they can go wrong
 8192 vertices, tile widths that split a lane's vertices, chunk counts around
 a block's share, frontiers without out-edges, and paths past the ring of
 level records."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -90,4 +92,41 @@ def test_sssp(quiet, n, m, W, S, wmax):
             ref = O.sssp_dijkstra(g.n, g.deg, g.cols, g.cw, src)
             assert np.array_equal(d, ref), np.flatnonzero(d != ref)[:10]
     finally:
+        gg.free()
+
+
+@pytest.mark.parametrize("n,m,W,S", [(8192, 60000, 64, 4), (40_000, 90_000, 512, 4), (600, 2000, 50, 2)])
+def test_noalloc_state_of_another_graph(quiet, n, m, W, S):
+    """The scratch array holds what the call before left in it, whatever loop
+    that one took, and a relaxed capture on another stream stays whole (the other
+    modes forbid the wait for the result)."""
+    hip = C.CDLL("/opt/rocm/lib/libamdhip64.so")
+    g = random_graph(n, m, W, S, n)
+    gg = upload(quiet, g)
+    lv, pa, stream, graph = C.c_void_p(), C.c_void_p(), C.c_void_p(), C.c_void_p()
+    assert hip.hipMalloc(C.byref(lv), C.c_size_t(4 * n)) == 0
+    assert hip.hipMalloc(C.byref(pa), C.c_size_t(4 * n)) == 0
+    assert hip.hipStreamCreateWithFlags(C.byref(stream), 1) == 0
+    try:
+        for timing, src in ((False, 0), (True, n - 1), (False, n // 2)):
+            print(f"case: noalloc n={n} timing={timing} src={src}", flush=True)
+            quiet.set_level_timing(timing)
+            st = G.Stats()
+            assert hip.hipStreamBeginCapture(stream, 2) == 0
+            rc = quiet.lib.gphi_bfs_noalloc(gg.h, src, lv, pa, C.byref(st))
+            assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+            assert hip.hipGraphDestroy(graph) == 0
+            quiet.check(rc)
+            got, par = np.empty(n, np.int32), np.empty(n, np.int32)
+            assert hip.hipMemcpy(C.c_void_p(got.ctypes.data), lv, C.c_size_t(4 * n), 2) == 0
+            assert hip.hipMemcpy(C.c_void_p(par.ctypes.data), pa, C.c_size_t(4 * n), 2) == 0
+            ref = O.bfs_levels(g.n, g.deg, g.cols, src)
+            assert np.array_equal(got, ref)
+            assert O.check_parents(g.n, g.deg, g.cols, src, got, par) == 0
+            assert np.array_equal(st.trace(), O.bfs_hybrid(g, src, 20)[2])
+    finally:
+        quiet.set_level_timing(False)
+        hip.hipFree(lv)
+        hip.hipFree(pa)
+        hip.hipStreamDestroy(stream)
         gg.free()
