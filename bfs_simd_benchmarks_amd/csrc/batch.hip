@@ -61,7 +61,7 @@ constexpr uint8_t kUnreached = 255;
 typedef unsigned long long u64;
 
 // the sources of a dense step whose frontiers have few out-edges (sparse
-// sources, batch_live_kernel); their mask sits beside the live mask
+// sources, reduce_live); their mask sits beside the live mask
 constexpr uint32_t kSparseWord = 4;     // live[4..7]: the sparse sources of the next frontier
 constexpr uint32_t kSparseCount = 8;    // live[8]: entries of the sparse-source queue
 // sparse: fewer than M / 1536 frontier out-edges (estimated).  Measured at

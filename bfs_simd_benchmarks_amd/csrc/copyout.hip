@@ -324,14 +324,16 @@ void decode(const uint8_t *p, uint64_t i, uint64_t count, uint32_t none, uint32_
 // slot) to 1 ms (kSlots), which would be paid on every context's first call,
 // so finished copy-outs leave theirs for the next: up to kIdleRings of each
 // size stay with the process while it has a context, and none after that.
+// Single slots are what the lanes of a server lease at the same time: with two
+// kept, 59 queries on graphs of 16384 vertices took 2.0 ms, with sixteen 1.35.
 struct Ring {
 	uint8_t *mem = nullptr;      // the slots, then their flags, a line apart
 	uint32_t slots = 0;
 	unsigned long long seq = 0;  // sequence number of the slot filled last
 };
-constexpr size_t kIdleRings = 2;
+constexpr uint32_t kIdleRings[2] = {2, 16};  // of kSlots slots, of one: 128 MiB in all
 std::mutex g_ring_mu;  // guards the three below
-Ring g_idle[2][kIdleRings];
+Ring g_idle[2][16];
 uint32_t g_idle_count[2] = {0, 0};
 uint32_t g_contexts = 0;
 
@@ -360,7 +362,7 @@ void return_ring(bool one, const Ring &r)
 {
 	{
 		std::lock_guard<std::mutex> lk(g_ring_mu);
-		if (g_idle_count[one] < kIdleRings) {
+		if (g_idle_count[one] < kIdleRings[one]) {
 			g_idle[one][g_idle_count[one]++] = r;
 			return;
 		}
