@@ -588,10 +588,8 @@ __global__ void init_source_kernel(uint32_t src, uint32_t W, const uint32_t *__r
 		ctrl->qsize = d ? 1 : 0;
 		ctrl->dir = 0;
 		ctrl->done = 0;
-		ctrl->blocks_done = 0;
 		ctrl->facc = 0;
 		ctrl->qpack = 0;
-		ctrl->changed = 0;
 		ctrl->chunks = 0;
 		ctrl->level = 0;
 		ctrl->queued = 0;

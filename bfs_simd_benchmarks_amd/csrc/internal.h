@@ -51,7 +51,7 @@ struct ChunkPack {
 	uint32_t tbase[8];  // per group of kPackGroup edges
 };
 
-// Control block of one frontier traversal (128 bytes).  The level loop runs
+// Control block of one traversal in the five-kernel loop (128 bytes).  The level loop runs
 // on the device: every kernel of a level reads the direction, the level and
 // the queue sizes here, and the host reads the block back only every few
 // levels to see whether the traversal is done.
@@ -61,17 +61,14 @@ struct StepCtrl {
 	uint32_t qsize;         // queue entries (frontier vertices with outdeg > 0)
 	uint32_t dir;           // direction chosen for expanding it
 	uint32_t done;          // frontier empty
-	uint32_t blocks_done;   // last-block detection
 	uint32_t facc;          // accumulator: |F|
-	uint32_t err;           // multi-source BFS: a level would not fit its uint8 levels
 	unsigned long long qpack;  // accumulator: (queue count << 32) | degree sum
-	uint32_t changed;       // hop relaxation: edges that lowered a distance
 	uint32_t chunks;        // chunks on the live lists of the last dense sweep
 	uint32_t level;         // the step being expanded (device-driven loop)
 	uint32_t queued;        // BFS: the step expanded last built the next queue itself
 	unsigned long long reached, traversed;  // sums of |F| and of sum deg(F) over the steps
 	uint32_t col_stale;     // BFS: column counts miss the vertices of queue-building steps
-	uint32_t pad[13];
+	uint32_t pad[15];
 };
 
 // A BFS sparse step whose frontier's edges fill at most this many CSR-push
@@ -188,7 +185,7 @@ struct gphi_ctx {
 	std::mutex mu;
 	gphi::Error err{0, ""};
 	std::string last;
-	// pinned host control block for per-step readback
+	// pinned host copy of the control block
 	gphi::StepCtrl *h_ctrl = nullptr;
 	gphi::LevelBoard *h_board = nullptr;  // in h_ctrl's allocation, written by the kernels of levels.h
 	bool board_busy = false;              // a traversal's kernels may still write the board
