@@ -889,7 +889,7 @@ __device__ __forceinline__ void sparse_push_block(
 				// as in the dense sweep: an edge that beats the dist[v] it read
 				// lowers it (no return needed) and marks v, which then ends the
 				// step below a value read during it, i.e. improved
-				const uint32_t nd = dist[u] + csr_w[idx];
+				const uint32_t nd = path_sum(dist[u], csr_w[idx]);
 				if (nd < dist[v]) {
 					atomicMin(dist + v, nd);
 					flag[v] = 1;
@@ -1376,7 +1376,7 @@ static int frontier_loop(gphi_graph *gr, uint32_t src, gphi_stats *st, uint32_t 
 		GPHI_HIP(ctx, hipMemcpyAsync(hc, gr->ctrl, sizeof(StepCtrl), hipMemcpyDeviceToHost, s));
 		GPHI_HIP(ctx, hipStreamSynchronize(s));
 		if (hc->done) break;
-		if (enq > G.n + 2 + kLevelGroup) return set_error(ctx, GPHI_E_STATE, "frontier loop did not terminate");
+		if (enq > level_limit(G.n) + kLevelGroup) return set_error(ctx, GPHI_E_STATE, "frontier loop did not terminate");
 	}
 	const uint32_t steps = hc->level;  // frontiers expanded
 	if (steps_out) *steps_out = steps;

@@ -28,6 +28,20 @@ constexpr int kNumXcd = 8;              // MI355X: 8 XCDs, blocks dispatched rou
 constexpr uint32_t kLiveCntStride = 32;
 constexpr size_t kLiveCntBytes = (size_t)kNumXcd * kLiveCntStride * 4;
 
+// dist[u] + w of a relaxation.  A weight is any 32-bit number, and a sum past
+// 2^32 stays at the top, above every distance, where it lowers nothing.  (One
+// that wrapped would pass for a short path, and the edges of a cycle could lower
+// each other's ends for ever.)
+__host__ __device__ inline uint32_t path_sum(uint32_t d, uint32_t w)
+{
+	const uint32_t x = d + w;
+	return x < d ? UINT32_MAX : x;
+}
+
+// A traversal whose relaxations are sums as above has at most n frontiers; a
+// loop that passes this many has lost its way and stops with GPHI_E_STATE.
+__host__ __device__ inline uint64_t level_limit(uint32_t n) { return (uint64_t)n + 2; }
+
 struct Error {
 	int code;
 	std::string msg;

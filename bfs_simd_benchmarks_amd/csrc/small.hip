@@ -155,7 +155,7 @@ __device__ __forceinline__ void small_push(uint32_t *s_mem, const Trav &t, uint3
 			uint32_t nd[kPer], dv[kPer];
 #pragma unroll
 			for (int r = 0; r < kPer; ++r) {
-				nd[r] = on[r] ? t.dist[uu[r]] + t.csr_w[ix[r]] : UINT32_MAX;
+				nd[r] = on[r] ? path_sum(t.dist[uu[r]], t.csr_w[ix[r]]) : UINT32_MAX;
 				dv[r] = t.dist[vv[r]];
 			}
 #pragma unroll
@@ -303,6 +303,7 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_kernel(Trav t, uint32_t src
 	}
 	unsigned long long reached = 0, traversed = 0;
 	uint32_t level = 0;
+	bool over = false;
 	for (;; ++level) {
 		__syncthreads();
 		// the next frontier becomes the current one; its queue
@@ -338,7 +339,8 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_kernel(Trav t, uint32_t src
 			qsize += s.red[1][k];
 			fdeg += s.red[2][k];
 		}
-		if (fsize == 0) break;  // uniform
+		over = fsize != 0 && level > level_limit(t.n);
+		if (fsize == 0 || over) break;  // uniform
 		reached += fsize;
 		traversed += fdeg;
 #pragma unroll
@@ -361,7 +363,7 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_kernel(Trav t, uint32_t src
 				t.level[v] = (int32_t)level + 1;
 				atomicOr(&s.next[v >> 5], bit);
 			} else {
-				const uint32_t nd = s_dist[u] + w;
+				const uint32_t nd = path_sum(s_dist[u], w);
 				if (nd < s_dist[v] && nd < atomicMin(&s_dist[v], nd)) atomicOr(&s.next[v >> 5], bit);
 			}
 		};
@@ -441,6 +443,7 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_kernel(Trav t, uint32_t src
 		board->reached = reached;
 		board->traversed = traversed;
 		board->levels = level;
+		board->err = over;
 		board->t_end = wall_clock64();
 		__hip_atomic_store(&board->progress, 3ull, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 	}
@@ -515,6 +518,7 @@ int small_level_loop(gphi_graph *gr, uint32_t src, gphi_stats *st, uint32_t *ste
 		unsigned long long p;
 		if ((rc = wait_progress(ctx, &board->progress, 0, &p))) return rc;
 		ctx->board_busy = false;
+		if (board->err) return set_error(ctx, GPHI_E_STATE, "frontier loop did not terminate");
 		small_stats(ctx, st, steps);
 		return GPHI_OK;
 	}
@@ -529,7 +533,8 @@ int small_level_loop(gphi_graph *gr, uint32_t src, gphi_stats *st, uint32_t *ste
 	const unsigned adv = advance_threads(G.n_pad), nblk = advance_blocks(G.n_pad);
 	const uint64_t items = std::max<uint64_t>({G.n_pad / (kBfs ? 16 : 1), G.n_words, G.side});
 	small_init_kernel<kBfs><<<(unsigned)std::min<uint64_t>((items + kBlock - 1) / kBlock, 2048), kBlock, 0, s>>>(t, src);
-	rc = follow_levels(ctx, [&](uint32_t level) {
+	rc = follow_levels(ctx, [&](uint32_t level) -> int {
+		if (level > level_limit(G.n) + kAhead) return set_error(ctx, GPHI_E_STATE, "frontier loop did not terminate");
 		if (kBfs)
 			small_expand_kernel<0><<<grid, kBlock, 0, s>>>(t, level);
 		else if (G.coo_w8)

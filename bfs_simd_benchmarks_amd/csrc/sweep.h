@@ -440,7 +440,11 @@ __device__ __forceinline__ void sssp_dense_walk(
 		const uint32_t hit_n = v1 ? frontier_bits(hn, inw_n, s_win, wlo_n, wlen_n, cur) : 0u;
 		uint32_t better = 0;
 #pragma unroll
-		for (int j = 0; j < 8; ++j) better |= (uint32_t)(dh[j] + weight_of<kW8>(w, j) < dt[j]) << j;
+		for (int j = 0; j < 8; ++j) {
+			// (a byte added to a distance stays below 2^32)
+			const uint32_t x = weight_of<kW8>(w, j), nd = kW8 ? dh[j] + x : path_sum(dh[j], x);
+			better |= (uint32_t)(nd < dt[j]) << j;
+		}
 		better &= hit;
 		// stage B: chunk k's relaxations
 #pragma unroll
