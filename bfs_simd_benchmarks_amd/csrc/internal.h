@@ -108,6 +108,18 @@ struct QueueBufs {
 inline uint32_t queue_stride(uint32_t n_pad, uint64_t m) { return n_pad + (uint32_t)(m / kSparseTile); }
 inline uint32_t tile_lo_stride(uint64_t m) { return (uint32_t)(m / kSparseTile + 2); }
 
+// The direction rule of the level loop of levels.h, |F| + sum deg(F) > M /
+// T_RATIO (apps/bfs_simd/bfs.cpp:829-834), with the sum in 64 bits: M may be
+// anything below 2^32.  The advance drops the queue of a frontier whose degrees
+// alone pass the threshold, so such a step has to be dense; in 32 bits |F| could
+// take the sum past 2^32 and back under the threshold, and the step would read a
+// queue that was never written.
+__host__ __device__ inline bool queue_dropped(uint32_t fdeg, uint32_t threshold) { return fdeg > threshold; }
+__host__ __device__ inline bool dense_step(uint32_t fsize, uint32_t fdeg, uint32_t threshold)
+{
+	return (uint64_t)fsize + fdeg > threshold;
+}
+
 // The level loop of levels.h.  LevelRec: a level's totals, the
 // accumulators the level before adds to; a ring over the levels, whose entry
 // half a ring ahead is cleared as a level starts.  LevelBoard: what the

@@ -19,8 +19,7 @@ namespace gphi {
 
 constexpr uint32_t kAhead = 2;  // levels enqueued past the one the device has started
 
-// What a level's expansion reads of its totals: the direction by the rule
-// |F| + sum deg(F) > M / T_RATIO in uint32 arithmetic (apps/bfs_simd/bfs.cpp:829-834)
+// What a level's expansion reads of its totals, and the direction (dense_step)
 struct Step {
 	uint32_t fsize, fdeg, qsize;
 	bool dense;
@@ -48,7 +47,7 @@ __device__ __forceinline__ Step step_of(const Frontier &t, uint32_t level)
 	const LevelRec *r = rec_of(t, level);
 	const unsigned long long qp = r->qpack;
 	const uint32_t f = r->fsize, d = (uint32_t)qp;
-	return Step{f, d, (uint32_t)(qp >> 32), f + d > t.threshold};
+	return Step{f, d, (uint32_t)(qp >> 32), dense_step(f, d, t.threshold)};
 }
 
 // The start of a level, one thread: the previous step's chunk count and this
@@ -183,7 +182,7 @@ __device__ __forceinline__ void advance_block(const Frontier &t, uint32_t level)
 		if (f) atomicAdd(&nr->fsize, f);
 		if (qb) {
 			base = atomicAdd(&nr->qpack, ((unsigned long long)qb << 32) | db);
-			if ((uint32_t)base + db > t.threshold) base = ~0ull;  // the next step is dense
+			if (queue_dropped((uint32_t)base + db, t.threshold)) base = ~0ull;  // the next step is dense
 		}
 		s_base = base;
 	}

@@ -352,7 +352,7 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_kernel(Trav t, uint32_t src
 				++pos;
 				off += d[k];
 			}
-		const bool dense = level > 0 && fsize + fdeg > t.threshold;  // the first step is sparse
+		const bool dense = level > 0 && dense_step(fsize, fdeg, t.threshold);  // the first step is sparse
 		uint32_t nlive = 0;
 		// edge u -> v, its weight from w
 		auto relax = [&](uint32_t u, uint32_t v, uint32_t w) {

@@ -35,3 +35,25 @@ int main()
 	return 0;
 }
 """)
+
+
+def test_a_dropped_queue_means_a_dense_step(tmp_path):
+    """M may be anything below 2^32, and |F| + sum deg(F) more than that."""
+    run_cpp(tmp_path, r"""
+#include "internal.h"
+int main()
+{
+	const uint32_t m = UINT32_MAX;
+	const uint32_t fs[] = {1, 2, 1000, 1u << 25, UINT32_MAX};
+	const uint32_t ds[] = {0, 1, m / 20 - 1, m / 20, m / 20 + 1, m / 2, m / 2 + 1, m - (1u << 25), m - 1, m};
+	for (uint32_t threshold : {0u, 1u, m / 20, m / 2, m})
+		for (uint32_t f : fs)
+			for (uint32_t d : ds) {
+				if (gphi::queue_dropped(d, threshold) && !gphi::dense_step(f, d, threshold))
+					return printf("|F| %u, degrees %u, threshold %u: no queue for a sparse step\n", f, d, threshold), 1;
+				// without a wrap it is the rule in 32 bits
+				if (f + d >= f && gphi::dense_step(f, d, threshold) != (f + d > threshold)) return 1;
+			}
+	return 0;
+}
+""")
