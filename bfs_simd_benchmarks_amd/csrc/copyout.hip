@@ -28,22 +28,17 @@
 #include <sched.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cstring>
 #include <mutex>
-#include <system_error>
-#include <thread>
 
 #include "internal.h"
+#include "slots.h"
 
 namespace gphi {
 
 namespace {
 
 constexpr size_t kSlotBytes = 2u << 20;
-constexpr uint32_t kSlots = 24;
-constexpr uint32_t kParts = 8;         // pieces of a slot the host threads take
-constexpr uint32_t kMaxHelpers = 11;   // host threads beside the caller's
 constexpr uint64_t kHelperBytes = 2u << 20;  // a helper per this much output (starting one takes about 20 us)
 constexpr uint64_t kNarrowBytes = 1u << 20;  // distances: output from which a pass for the largest pays (10 us)
 constexpr unsigned kFillGrid = 256;    // blocks that fill a slot: enough to keep the link busy
@@ -402,71 +397,29 @@ int stream_out(gphi_ctx *ctx, uint64_t nslots, uint64_t out_bytes, Fill fill, Ta
 	auto slot = [&](uint64_t i) { return mem + (i % R) * kSlotBytes; };
 	const unsigned long long seq0 = ring.seq + 1;  // slot i is filled when its flag is seq0 + i
 	ring.seq += nslots;
-	std::atomic<uint64_t> next{0}, ready{0};
-	std::atomic<uint32_t> taken[kSlots];
-	for (auto &x : taken) x.store(0);
-	std::atomic<bool> stop{false};
-	const uint64_t all = nslots * kParts;
-	// takes the next part; waits (or not) until its slot is filled
-	auto take_parts = [&](bool wait) {
-		for (;;) {
-			uint64_t p = next.load(std::memory_order_relaxed);
-			if (p >= all || stop.load(std::memory_order_relaxed)) return;
-			if (ready.load(std::memory_order_acquire) <= p / kParts) {
-				if (!wait) return;
-				_mm_pause();
-				continue;
-			}
-			if (!next.compare_exchange_weak(p, p + 1, std::memory_order_relaxed)) continue;
-			take(p / kParts, (uint32_t)(p % kParts), (const uint8_t *)slot(p / kParts));
-			taken[p / kParts % R].fetch_add(1, std::memory_order_release);
-		}
-	};
-	std::thread helpers[kMaxHelpers];
-	uint32_t nh = 0;
-	uint64_t issued = 0, spin = 0;
-	auto issue = [&] {
-		// a slot is filled again once its last contents were taken
-		while (issued < nslots &&
-		       (issued < R || taken[issued % R].load(std::memory_order_acquire) == issued / R * kParts)) {
-			fill(issued, slot(issued));
-			slot_done_kernel<<<1, 1, 0, s>>>(flag(issued), seq0 + issued);
-			++issued;
-		}
-	};
-	issue();
-	const uint32_t want = helper_count(nslots, out_bytes);
-	try {
-		for (; nh < want; ++nh) helpers[nh] = std::thread(take_parts, true);
-	} catch (const std::system_error &) {
-		// fewer helpers: the calling thread takes every part that is left
-	}
-	while (ready.load(std::memory_order_relaxed) < nslots) {
-		const uint64_t r = ready.load(std::memory_order_relaxed);
-		if (r < issued && __atomic_load_n(flag(r), __ATOMIC_ACQUIRE) >= seq0 + r) {
-			ready.store(r + 1, std::memory_order_release);
-			spin = 0;
-		} else if (++spin % 4096 == 0) {
-			const hipError_t e = hipStreamQuery(s);
-			if (e != hipSuccess && e != hipErrorNotReady) {
-				rc = hip_fail(ctx, e, "copy-out", __FILE__, __LINE__);
-				break;
-			}
-		}
-		issue();
-		if (nh == 0) take_parts(false);
-		_mm_pause();
-	}
-	if (rc) stop.store(true);
-	take_parts(true);
-	for (uint32_t i = 0; i < nh; ++i) helpers[i].join();
+	rc = run_slots(
+	    nslots, R, helper_count(nslots, out_bytes),
+	    [&](uint64_t i) -> int {
+		    fill(i, slot(i));
+		    slot_done_kernel<<<1, 1, 0, s>>>(flag(i), seq0 + i);
+		    GPHI_HIP(ctx, hipGetLastError());
+		    return GPHI_OK;
+	    },
+	    [&](uint64_t i) { return __atomic_load_n(flag(i), __ATOMIC_ACQUIRE) >= seq0 + i; },
+	    [&](bool *idle) -> int {
+		    const hipError_t e = hipStreamQuery(s);
+		    if (e != hipSuccess && e != hipErrorNotReady) return hip_fail(ctx, e, "copy-out", __FILE__, __LINE__);
+		    *idle = e == hipSuccess;
+		    return GPHI_OK;
+	    },
+	    [&](uint64_t i, uint32_t part) { take(i, part, (const uint8_t *)slot(i)); });
+	if (rc == kSlotsStalled) rc = set_error(ctx, GPHI_E_STATE, "copy-out made no progress");
 	if (rc) {
 		// fills may be under way: the ring goes back if they end, and is not used again otherwise
 		if (hipStreamSynchronize(s) == hipSuccess) return_ring(one, ring);
 		return rc;
 	}
 	return_ring(one, ring);
-	GPHI_HIP(ctx, hipGetLastError());
 	return GPHI_OK;
 }
 

@@ -57,3 +57,68 @@ int main()
 	return 0;
 }
 """)
+
+
+SLOTS_MAIN = r"""
+#include "slots.h"
+#include <cstdio>
+#include <cstdlib>
+using namespace gphi;
+static void need(bool ok, const char *what)
+{
+	if (!ok) printf("%s\n", what), exit(1);
+}
+"""
+
+
+def test_slots_in_turn(tmp_path):
+    """Every part of every slot is taken once, from what its own fill left."""
+    run_cpp(tmp_path, SLOTS_MAIN + r"""
+int main()
+{
+	for (uint32_t R : {1u, 3u, kSlots})
+		for (uint32_t nh : {0u, 1u, 5u, kMaxHelpers})
+			for (uint64_t n : {1ull, 2ull, 3ull, 25ull, 200ull}) {
+				// the device: what was issued, in order, a while later
+				uint64_t slot[kSlots] = {}, issued = 0, done = 0, delay = 0;
+				std::atomic<uint32_t> got[200 * kParts] = {};
+				const int rc = run_slots(
+				    n, R, nh, [&](uint64_t i) { return need(i == issued++, "issued in order"), 0; },
+				    [&](uint64_t i) {
+					    if (done < issued && ++delay % 7 == 0) slot[done % R] = done + 1, ++done;
+					    return i < done;
+				    },
+				    [&](bool *idle) { return *idle = done == issued, 0; },
+				    [&](uint64_t i, uint32_t part) {
+					    need(slot[i % R] == i + 1, "a part of another fill");
+					    got[i * kParts + part].fetch_add(1);
+				    });
+				need(rc == 0, "ends well");
+				for (uint64_t k = 0; k < n * kParts; ++k) need(got[k] == 1, "each part once");
+			}
+	return 0;
+}
+""")
+
+
+@pytest.mark.parametrize("what", ["refused", "never filled", "stream error"])
+def test_slots_end_when_the_device_does_not_fill_them(tmp_path, what):
+    """A launch that is refused, a stream that goes idle with a slot not filled,
+    a stream in error: the run ends with that, every thread with it."""
+    run_cpp(tmp_path, SLOTS_MAIN + f"""
+int main()
+{{
+	const bool refused = {int(what == "refused")}, error = {int(what == "stream error")};
+""" + r"""
+	for (uint64_t bad : {0ull, 5ull, 30ull})
+		for (uint32_t nh : {0u, 3u}) {
+			uint64_t issued = 0;
+			const int rc = run_slots(
+			    40, 8, nh, [&](uint64_t i) { return refused && i == bad ? -5 : (++issued, 0); },
+			    [&](uint64_t i) { return i < bad && i < issued; },
+			    [&](bool *idle) { return *idle = !error, error ? -6 : 0; }, [](uint64_t, uint32_t) {});
+			need(rc == (refused ? -5 : error ? -6 : kSlotsStalled), "ends with the error");
+		}
+	return 0;
+}
+""", timeout=20)
