@@ -5,10 +5,12 @@
 // carved out of one fixed device array per GPU instead of buffers the library
 // allocates, for callers that cannot call hipMalloc.  Every call on a GPU
 // shares that GPU's array; a process-wide lock per device serialises the
-// calls, and each call's kernels are done before it returns (the level loop
-// reads its control block back), so the next call finds the array free.  The
-// array keeps the last call's contents: everything that must start at zero is
-// cleared by the traversal's own init kernels, none by hipMemsetAsync.
+// calls, and a call waits for its stream before it gives the lock up, also
+// after an error, so the next call, on whatever context, finds the array free.
+// (Where that wait is itself refused, as beside a capture in global mode, the
+// next call waits for the device.)  The array keeps the last call's contents:
+// everything that must start at zero is cleared by the traversal's own init
+// kernels, none by hipMemsetAsync.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -31,6 +33,7 @@ std::mutex g_scratch_mu;                        // guards g_scratch_ptr / g_scra
 void *g_scratch_ptr[kNoAllocMaxDevices];        // device address of `scratch` per device
 std::string g_scratch_err[kNoAllocMaxDevices];  // why an address is missing
 std::mutex g_scratch_use[kNoAllocMaxDevices];   // one no-alloc traversal per device at a time
+bool g_scratch_busy[kNoAllocMaxDevices];        // under it: kernels of a call may still run on `scratch`
 
 // level and parent of every vertex < n into the caller's arrays; -1 for the
 // vertices the traversal did not reach (state 0)
@@ -132,16 +135,21 @@ int run_bfs_noalloc(gphi_graph *gr, uint32_t src, int32_t *levels_dev, int32_t *
 		                 G.n, (unsigned long long)G.m, need, kNoAllocScratchBytes);
 	carve_state(G, base, &t);
 	std::lock_guard<std::mutex> use(g_scratch_use[dev]);
+	if (g_scratch_busy[dev]) GPHI_HIP(ctx, hipDeviceSynchronize());
+	g_scratch_busy[dev] = true;
 	if (st) memset(st, 0, sizeof(*st));
-	int rc = bfs_level_loop(&t, src, st);
-	if (rc) return rc;
 	hipStream_t s = ctx->stream;
-	if (levels_dev || parents_dev) {
+	int rc = bfs_level_loop(&t, src, st);
+	if (rc == GPHI_OK && (levels_dev || parents_dev)) {
 		const unsigned grid = (unsigned)std::min<uint64_t>(((uint64_t)G.n + kBlock - 1) / kBlock, 8192);
 		bfs_copy_out_kernel<<<grid, kBlock, 0, s>>>(G.n, t.flag, t.level, t.parent, levels_dev, parents_dev);
+		const hipError_t e = hipGetLastError();
+		if (e != hipSuccess) rc = hip_fail(ctx, e, "no-allocation BFS", __FILE__, __LINE__);
 	}
-	GPHI_HIP(ctx, hipGetLastError());
-	GPHI_HIP(ctx, hipStreamSynchronize(s));
+	const hipError_t drained = hipStreamSynchronize(s);
+	if (drained == hipSuccess) g_scratch_busy[dev] = false;
+	if (rc) return rc;
+	GPHI_HIP(ctx, drained);
 	return GPHI_OK;
 }
 

@@ -130,3 +130,37 @@ def test_noalloc_state_of_another_graph(quiet, n, m, W, S):
         hip.hipFree(pa)
         hip.hipStreamDestroy(stream)
         gg.free()
+
+
+def test_noalloc_after_a_refused_call_of_another_context(quiet):
+    """A capture in global mode refuses the wait for a call's kernels, which may
+    then still run on the scratch array: the next call, on another context and
+    another graph, finds it free."""
+    hip = C.CDLL("/opt/rocm/lib/libamdhip64.so")
+    big, small = random_graph(270_001, 600_000, 1024, 16, 5), random_graph(20_000, 60_000, 100, 4, 6)
+    lv, stream, graph = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    assert hip.hipMalloc(C.byref(lv), C.c_size_t(4 * small.n)) == 0
+    assert hip.hipStreamCreateWithFlags(C.byref(stream), 1) == 0
+    with G.Context(0) as other:
+        other.set_level_timing(False)
+        a, b = upload(quiet, big), upload(other, small)
+        try:
+            for src in (0, 1, 7):
+                print(f"case: noalloc after a refused call src={src}", flush=True)
+                assert hip.hipStreamBeginCapture(stream, 0) == 0
+                rc = quiet.lib.gphi_bfs_noalloc(a.h, src, None, None, None)
+                hip.hipStreamEndCapture(stream, C.byref(graph))    # invalidated by the refused wait
+                hip.hipGetLastError()
+                assert rc == -5, rc
+                other.check(other.lib.gphi_bfs_noalloc(b.h, src, lv, None, None))
+                got = np.empty(small.n, np.int32)
+                assert hip.hipMemcpy(C.c_void_p(got.ctypes.data), lv, C.c_size_t(4 * small.n), 2) == 0
+                assert np.array_equal(got, O.bfs_levels(small.n, small.deg, small.cols, src))
+                st = G.Stats()
+                quiet.check(quiet.lib.gphi_bfs_noalloc(a.h, src, None, None, C.byref(st)))
+                assert st.reached == int((O.bfs_levels(big.n, big.deg, big.cols, src) >= 0).sum())
+        finally:
+            hip.hipFree(lv)
+            hip.hipStreamDestroy(stream)
+            a.free()
+            b.free()
