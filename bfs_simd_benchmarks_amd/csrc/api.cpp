@@ -76,8 +76,8 @@ int gphi_open(const gphi_opts *opts, gphi_ctx **out)
 	}
 	if ((e = hipSetDevice(ctx->device)) != hipSuccess ||
 	    (e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking)) != hipSuccess ||
-	    (e = hipHostMalloc((void **)&ctx->h_ctrl, sizeof(gphi::StepCtrl) + sizeof(gphi::LevelBoard),
-	                       hipHostMallocDefault)) != hipSuccess) {
+	    (e = gphi::pinned_alloc((void **)&ctx->h_ctrl, sizeof(gphi::StepCtrl) + sizeof(gphi::LevelBoard))) !=
+	        hipSuccess) {
 		int rc = set_error(nullptr, GPHI_E_HIP, "gphi_open: %s", hipGetErrorString(e));
 		if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
 		delete ctx;

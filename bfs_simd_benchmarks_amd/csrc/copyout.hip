@@ -343,7 +343,7 @@ int lease_ring(gphi_ctx *ctx, bool one, Ring *out)
 		}
 	}
 	const uint32_t slots = one ? 1 : kSlots;
-	const hipError_t e = hipHostMalloc((void **)&out->mem, slots * (kSlotBytes + 128), hipHostMallocPortable);
+	const hipError_t e = pinned_alloc((void **)&out->mem, slots * (kSlotBytes + 128));
 	if (e != hipSuccess) {
 		out->mem = nullptr;
 		return set_error(ctx, GPHI_E_OOM, "pinned staging of %u slots: %s", slots, hipGetErrorString(e));

@@ -305,6 +305,14 @@ int dmalloc(gphi_ctx *ctx, void **p, size_t bytes, uint64_t *acc);
 
 void fill_words(gphi_ctx *ctx, uint32_t *p, uint64_t count, uint32_t value);  // on ctx's stream
 
+// Pinned memory that kernels write while the host looks at it (the level board,
+// staging slots and their flags): asked for as coherent, which a plain request
+// is only if the environment's HIP_HOST_COHERENT does not say otherwise.
+inline hipError_t pinned_alloc(void **p, size_t bytes)
+{
+	return hipHostMalloc(p, bytes, hipHostMallocPortable | hipHostMallocCoherent);
+}
+
 // device-side entry points (device.hip, hops.hip, pagerank.hip)
 int upload_graph(gphi_ctx *ctx, const gphi_graph_desc *d, gphi_graph *gr);
 void free_graph_device(gphi_graph *gr);

@@ -122,3 +122,22 @@ int main()
 	return 0;
 }
 """, timeout=20)
+
+
+def test_pinned_memory_is_coherent(tmp_path):
+    """The host polls words that kernels write: every pinned allocation asks for
+    coherent memory, whatever HIP_HOST_COHERENT says."""
+    run_cpp(tmp_path, r"""
+#include "internal.h"
+static unsigned seen;
+extern "C" hipError_t hipHostMalloc(void **p, size_t, unsigned flags) { return seen = flags, *p = nullptr, hipSuccess; }
+int main()
+{
+	void *p;
+	if (gphi::pinned_alloc(&p, 64) != hipSuccess || !(seen & hipHostMallocCoherent)) return 1;
+	return 0;
+}
+""")
+    calls = [(f.name, line) for f in sorted(B.CSRC.iterdir()) for line in f.read_text().splitlines()
+             if "hipHostMalloc(" in line]
+    assert len(calls) == 1 and calls[0][0] == "internal.h", calls
