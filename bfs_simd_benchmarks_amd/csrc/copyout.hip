@@ -365,16 +365,17 @@ void return_ring(bool one, const Ring &r)
 	(void)hipHostFree(r.mem);
 }
 
+// helpers a copy-out is worth, and those the process may have at one time
 uint32_t helper_count(uint64_t nslots, uint64_t out_bytes)
 {
-	uint64_t t = std::min<uint64_t>(kMaxHelpers, out_bytes / kHelperBytes);
-	if (nslots <= 1 && out_bytes < 4 * kHelperBytes) t = 0;
-	if (t) {
-		cpu_set_t set;
-		const int cpus = sched_getaffinity(0, sizeof set, &set) == 0 ? CPU_COUNT(&set) : 1;
-		t = std::min<uint64_t>(t, (uint64_t)std::max(cpus - 1, 0));
-	}
-	return (uint32_t)t;
+	if (nslots <= 1 && out_bytes < 4 * kHelperBytes) return 0;
+	return (uint32_t)std::min<uint64_t>(kMaxHelpers, out_bytes / kHelperBytes);
+}
+uint32_t helper_limit()
+{
+	cpu_set_t set;
+	const int cpus = sched_getaffinity(0, sizeof set, &set) == 0 ? CPU_COUNT(&set) : 1;
+	return (uint32_t)std::min<int>(kAllHelpers, std::max(cpus - 1, 0));
 }
 
 // fill(slot number, slot) enqueues the kernel that fills a slot; take(slot
@@ -397,8 +398,9 @@ int stream_out(gphi_ctx *ctx, uint64_t nslots, uint64_t out_bytes, Fill fill, Ta
 	auto slot = [&](uint64_t i) { return mem + (i % R) * kSlotBytes; };
 	const unsigned long long seq0 = ring.seq + 1;  // slot i is filled when its flag is seq0 + i
 	ring.seq += nslots;
+	const uint32_t want = helper_count(nslots, out_bytes);
 	rc = run_slots(
-	    nslots, R, helper_count(nslots, out_bytes),
+	    nslots, R, want, want ? helper_limit() : 0,
 	    [&](uint64_t i) -> int {
 		    fill(i, slot(i));
 		    slot_done_kernel<<<1, 1, 0, s>>>(flag(i), seq0 + i);

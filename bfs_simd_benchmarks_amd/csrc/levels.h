@@ -13,6 +13,7 @@
 
 #include <algorithm>
 
+#include "slots.h"
 #include "sweep.h"
 
 namespace gphi {
@@ -248,6 +249,7 @@ inline int wait_progress(gphi_ctx *ctx, const unsigned long long *word, unsigned
                          unsigned long long *out)
 {
 	uint32_t idle = 0;
+	Turn turn;
 	for (uint32_t spin = 1;; ++spin) {
 		const unsigned long long p = __atomic_load_n(word, __ATOMIC_ACQUIRE);
 		if ((p >> 1) > seen) {
@@ -260,7 +262,7 @@ inline int wait_progress(gphi_ctx *ctx, const unsigned long long *word, unsigned
 			// an idle stream has published every enqueued level
 			if (e == hipSuccess && ++idle > 2) return set_error(ctx, GPHI_E_STATE, "level loop made no progress");
 		}
-		__builtin_ia32_pause();
+		turn.wait();
 	}
 }
 

@@ -83,7 +83,7 @@ int main()
 				uint64_t slot[kSlots] = {}, issued = 0, done = 0, delay = 0;
 				std::atomic<uint32_t> got[200 * kParts] = {};
 				const int rc = run_slots(
-				    n, R, nh, [&](uint64_t i) { return need(i == issued++, "issued in order"), 0; },
+				    n, R, nh, kAllHelpers, [&](uint64_t i) { return need(i == issued++, "issued in order"), 0; },
 				    [&](uint64_t i) {
 					    if (done < issued && ++delay % 7 == 0) slot[done % R] = done + 1, ++done;
 					    return i < done;
@@ -114,7 +114,7 @@ int main()
 		for (uint32_t nh : {0u, 3u}) {
 			uint64_t issued = 0;
 			const int rc = run_slots(
-			    40, 8, nh, [&](uint64_t i) { return refused && i == bad ? -5 : (++issued, 0); },
+			    40, 8, nh, kAllHelpers, [&](uint64_t i) { return refused && i == bad ? -5 : (++issued, 0); },
 			    [&](uint64_t i) { return i < bad && i < issued; },
 			    [&](bool *idle) { return *idle = !error, error ? -6 : 0; }, [](uint64_t, uint32_t) {});
 			need(rc == (refused ? -5 : error ? -6 : kSlotsStalled), "ends with the error");
@@ -141,3 +141,67 @@ int main()
     calls = [(f.name, line) for f in sorted(B.CSRC.iterdir()) for line in f.read_text().splitlines()
              if "hipHostMalloc(" in line]
     assert len(calls) == 1 and calls[0][0] == "internal.h", calls
+
+
+def test_copy_outs_at_once_share_their_helpers(tmp_path):
+    """Eight calls that would each start 11 threads have 5 between them."""
+    run_cpp(tmp_path, SLOTS_MAIN + r"""
+#include <cstring>
+static int threads()
+{
+	char line[128];
+	int n = 0;
+	FILE *f = fopen("/proc/self/status", "r");
+	while (f && fgets(line, sizeof line, f))
+		if (!strncmp(line, "Threads:", 8)) n = atoi(line + 8);
+	if (f) fclose(f);
+	return n;
+}
+int main()
+{
+	constexpr int kCalls = 8;
+	std::atomic<int> most{0}, running{0};
+	std::thread calls[kCalls];
+	for (auto &c : calls)
+		c = std::thread([&] {
+			for (++running; running < kCalls;) sched_yield();
+			std::atomic<uint32_t> parts{0};
+			const int rc = run_slots(
+			    100, kSlots, kMaxHelpers, 5, [](uint64_t) { return 0; }, [](uint64_t) { return true; },
+			    [](bool *idle) { return *idle = false, 0; },
+			    [&](uint64_t, uint32_t part) {
+				    ++parts;
+				    if (part) return;
+				    const int n = threads();
+				    for (int m = most; m < n && !most.compare_exchange_weak(m, n);) {}
+			    });
+			need(rc == 0 && parts == 100 * kParts, "each part once");
+		});
+	for (auto &c : calls) c.join();
+	need(most > 1 && most <= 1 + kCalls + 5, "helpers within the limit");
+	need(lease_helpers(11, 5) == 5 && lease_helpers(1, 5) == 0, "all were given back");
+	return 0;
+}
+""")
+
+
+def test_waits_give_the_core_away(tmp_path):
+    """A slot that is filled only once the waiting threads have yielded."""
+    run_cpp(tmp_path, SLOTS_MAIN + r"""
+static std::atomic<int> yields{0};
+extern "C" int sched_yield() noexcept { return ++yields, 0; }
+int main()
+{
+	for (uint32_t nh : {0u, 2u}) {
+		yields = 0;
+		const int rc = run_slots(
+		    3, 1, nh, kAllHelpers, [](uint64_t) { return 0; }, [](uint64_t i) { return yields > 10 * (int)(i + 1); },
+		    [](bool *idle) { return *idle = false, 0; }, [](uint64_t, uint32_t) {});
+		need(rc == 0, "ends well");
+	}
+	Turn t;
+	for (int i = yields = 0; i < 4096; ++i) t.wait();
+	need(yields > 0, "a long wait yields");
+	return 0;
+}
+""", timeout=20)
