@@ -473,15 +473,6 @@ void free_graph_device(gphi_graph *gr)
 		if (p) (void)hipFree(p);
 }
 
-
-// Capacity of one XCD's live-chunk list: chunk selection hands out chunks in
-// groups of 64 (a wavefront's), group g to XCD g % 8.
-static uint32_t live_list_cap(uint64_t nchunks)
-{
-	const uint64_t groups = (nchunks + kBlock - 1) / kBlock;
-	return (uint32_t)((groups + kNumXcd - 1) / kNumXcd * kBlock);
-}
-
 // ---------------------------------------------------------------------------
 // traversal state
 // ---------------------------------------------------------------------------
@@ -516,7 +507,7 @@ static int alloc_state(gphi_graph *gr)
 	if ((rc = dmalloc(ctx, (void **)&gr->qoff, 2 * (size_t)gr->queue_len * 4, nullptr))) return rc;
 	if ((rc = dmalloc(ctx, (void **)&gr->tile_lo, 2 * (size_t)tile_lo_stride(G.m) * 4, nullptr))) return rc;
 	if ((rc = dmalloc(ctx, (void **)&gr->ctrl, sizeof(StepCtrl), nullptr))) return rc;
-	const size_t list_cap = live_list_cap(G.nchunks);
+	const size_t list_cap = live_list_capacity(G.nchunks);
 	if ((rc = dmalloc(ctx, (void **)&gr->live, list_cap * kNumXcd * 4 + 4, nullptr))) return rc;
 	if ((rc = dmalloc(ctx, (void **)&gr->live_cnt, kLiveCntBytes, nullptr))) return rc;
 	if ((rc = dmalloc(ctx, (void **)&gr->trace, (GPHI_MAX_STEPS + 1) * sizeof(uint4), nullptr))) return rc;
@@ -1323,7 +1314,7 @@ static int frontier_loop(gphi_graph *gr, uint32_t src, gphi_stats *st, uint32_t 
 	// enqueues kLevelGroup levels at a time and reads the control block back
 	// once per group, not once per level.
 	const unsigned nblk = G.n_pad / kPadVerts;
-	const uint32_t list_cap = live_list_cap(G.nchunks);
+	const uint32_t list_cap = live_list_capacity(G.nchunks);
 	const unsigned sgrid = (unsigned)std::max<uint64_t>(1, (G.nchunks + kBlock - 1) / kBlock);
 	// every block of the sweep resident at once (blocks of a run-interleaved
 	// list walk all have the same work), a multiple of the XCD count
@@ -1443,8 +1434,6 @@ int run_bfs(gphi_graph *gr, uint32_t src, int32_t *levels, int32_t *parents, gph
 }
 
 int bfs_level_loop(gphi_graph *gr, uint32_t src, gphi_stats *st) { return frontier_loop<true>(gr, src, st, nullptr); }
-
-uint32_t live_list_capacity(uint64_t nchunks) { return live_list_cap(nchunks); }
 
 int run_sssp(gphi_graph *gr, uint32_t src, uint32_t *dist, gphi_stats *st)
 {

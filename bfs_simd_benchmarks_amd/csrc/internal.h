@@ -108,6 +108,14 @@ struct QueueBufs {
 inline uint32_t queue_stride(uint32_t n_pad, uint64_t m) { return n_pad + (uint32_t)(m / kSparseTile); }
 inline uint32_t tile_lo_stride(uint64_t m) { return (uint32_t)(m / kSparseTile + 2); }
 
+// Entries of one XCD's live-chunk list: chunk selection hands out chunks in
+// groups of 64 (a wavefront's), group g to XCD g % 8.
+inline uint32_t live_list_capacity(uint64_t nchunks)
+{
+	const uint64_t groups = (nchunks + kBlock - 1) / kBlock;
+	return (uint32_t)((groups + kNumXcd - 1) / kNumXcd * kBlock);
+}
+
 // The direction rule of the level loop of levels.h, |F| + sum deg(F) > M /
 // T_RATIO (apps/bfs_simd/bfs.cpp:829-834), with the sum in 64 bits: M may be
 // anything below 2^32.  The advance drops the queue of a frontier whose degrees
@@ -181,6 +189,20 @@ struct DevGraph {
 	uint8_t *coo_w8 = nullptr;  // 8-bit tile-order weights when every weight is below 256
 	uint64_t device_bytes = 0;
 };
+
+// No less than what a lane of the server allocates besides the graph: the
+// single-source arrays (~42 bytes per vertex, the tile rows' and columns', and
+// what grows with the edges: queue, tile partition, live-chunk lists), the
+// multi-source masks, levels and bitmaps for max_batch sources, and the in-edge
+// arrays of their pull steps (4 bytes per edge, 12 per vertex, pieces).
+inline uint64_t lane_state_bytes(const DevGraph &G, uint32_t max_batch)
+{
+	const uint64_t nw = max_batch <= 64 ? 1 : max_batch <= 128 ? 2 : 4;
+	const uint64_t in_edges = max_batch > 1 ? 4 * G.m + 12 * (uint64_t)G.n_pad + G.m / 256 : 0;
+	const uint64_t queues = 4ull * 4 * (queue_stride(G.n_pad, G.m) - G.n_pad) + 2ull * 4 * tile_lo_stride(G.m) +
+	                        4ull * kNumXcd * live_list_capacity(G.nchunks);
+	return (uint64_t)G.n_pad * (42 + 3 * 8 * nw + 64 * nw + 1) + 8 * ((uint64_t)G.side + 1) + queues + in_edges;
+}
 
 // PageRank head bands (build_pr_bands).  The heads are cut into bands
 // [head_lo, head_hi); within a band, the in-edges of a tail whose heads lie in
@@ -365,7 +387,6 @@ void out_context_opened();
 void out_context_closed();
 // blocks of `block` threads of a kernel that fit the device at once, a multiple of the XCD count
 unsigned resident_grid(const void *kernel, unsigned block = kBlock);
-uint32_t live_list_capacity(uint64_t nchunks);  // entries of one XCD's live-chunk list
 int run_bfs_batch(gphi_graph *gr, const uint32_t *srcs, uint32_t k, uint8_t *levels, gphi_stats *st);
 // the multi-source state of gr for nw mask words: traversal state, in-edge
 // arrays, masks, levels (idempotent)

@@ -205,3 +205,45 @@ int main()
 	return 0;
 }
 """, timeout=20)
+
+
+def test_lane_estimate_covers_its_allocations(tmp_path):
+    """The server admits a graph by an estimate of its lanes' memory: it is no
+    less than what the lanes allocate, for few edges and for many per vertex."""
+    run_cpp(tmp_path, r"""
+#include "internal.h"
+#include <algorithm>
+using namespace gphi;
+int main()
+{
+	for (uint32_t n : {1000u, 8000u, 50000u, 3000000u, 33554432u})
+		for (uint64_t ef : {1ull, 16ull, 100ull, 1000ull, 4000ull})
+			for (uint32_t W : {16u, 512u, 4096u})
+				for (uint32_t k : {1u, 64u, 256u}) {
+					DevGraph G;
+					G.n = n, G.m = n * ef, G.W = W;
+					if (G.m >= 1ull << 32 || ef >= n) continue;
+					G.n_pad = n / kPadVerts * kPadVerts + kPadVerts;
+					G.nchunks = (G.m + kChunk - 1) / kChunk;
+					G.side = (n + W - 1) / W;
+					const uint64_t np = G.n_pad, nblk = np / kPadVerts, nw = k <= 64 ? 1 : k <= 128 ? 2 : 4;
+					// levels, parents, distances, state bytes, two bitmaps, row stamps and column counts
+					uint64_t sum = 3 * 4 * np + np + 2 * np / 8 + 2 * 4 * ((uint64_t)G.side + 1);
+					// queue and degree prefix, tile partition, live lists, counters, trace, scan blocks
+					sum += 2 * 2 * 4 * (uint64_t)queue_stride(G.n_pad, G.m) + 2 * 4 * (uint64_t)tile_lo_stride(G.m) +
+					       4 * kNumXcd * (uint64_t)live_list_capacity(G.nchunks) + 4 + kLiveCntBytes +
+					       sizeof(StepCtrl) + 16 * (GPHI_MAX_STEPS + 1) + nblk * (16 + 8 + 4 * 8);
+					if (k > 1) {
+						// masks, levels, touched bitmap and counts, live slots, start levels
+						sum += (3 * 8 + 64) * nw * np + np / 8 + 64 * 256 * 4 + 65 * 128 + 257 * 4 + 16;
+						// in-edges, their offsets; pieces of up to kPullPiece of vertices above kPullLight
+						sum += 4 * G.m + 4 * ((uint64_t)n + 1);
+						sum += 8 * (1 + G.m / kPullPiece + std::min<uint64_t>(n, G.m / kPullLight));
+					}
+					if (lane_state_bytes(G, k) < sum)
+						return printf("n %u, m %llu, W %u, %u sources: %llu of %llu bytes\n", n, (unsigned long long)G.m, W,
+						              k, (unsigned long long)lane_state_bytes(G, k), (unsigned long long)sum), 1;
+				}
+	return 0;
+}
+""")
