@@ -830,6 +830,7 @@ __global__ __launch_bounds__(kBlock) void batch_clear_kernel(Batch t, uint64_t m
 {
 	const uint64_t stride = (uint64_t)gridDim.x * kBlock;
 	const uint64_t i0 = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+	if (i0 == 0) t.board->t_begin = wall_clock64();
 	// clean: the last traversal on these buffers ran to its end, which leaves
 	// front, next and the touched bitmap all zero (only seen keeps its bits)
 	for (uint64_t i = i0; i < mask_words; i += stride) {
@@ -853,10 +854,7 @@ __global__ __launch_bounds__(kBlock) void batch_clear_kernel(Batch t, uint64_t m
 		t.rec[i0] = r;
 	}
 	if (i0 < 2) t.totals[i0] = 0;
-	if (i0 == 0) {
-		*t.failed = 0;
-		t.board->t_begin = wall_clock64();
-	}
+	if (i0 == 0) *t.failed = 0;
 }
 
 // ---- the four launches of a level ----

@@ -53,6 +53,7 @@ struct Hops {
 __global__ __launch_bounds__(kBlock) void hop_init_kernel(Hops t, uint32_t side, uint32_t src)
 {
 	const uint32_t stride = gridDim.x * kBlock, i0 = blockIdx.x * kBlock + threadIdx.x;
+	if (i0 == 0) t.board->t_begin = wall_clock64();
 	for (uint32_t i = i0; i < t.n_pad; i += stride) t.dist[i] = i == src ? 0u : kHopInf;
 	// sweep 0 lowered the source.  (A byte left from 256 sweeps ago, or from
 	// here, may match a later sweep's: its edges are then looked at again.)
@@ -64,7 +65,6 @@ __global__ __launch_bounds__(kBlock) void hop_init_kernel(Hops t, uint32_t side,
 		r.fsize = i0 == 0;
 		t.rec[i0] = r;
 	}
-	if (i0 == 0) t.board->t_begin = wall_clock64();
 }
 
 // a head row of the chunk was lowered in sweep k - 1 or, as far as this block

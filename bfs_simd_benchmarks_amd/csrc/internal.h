@@ -146,7 +146,9 @@ static_assert(sizeof(LevelRec) == 256, "LevelRec is two lines");
 struct LevelBoard {
 	unsigned long long progress;  // (levels started << 1) | ended
 	unsigned long long reached, traversed;
-	unsigned long long t_begin, t_end;  // device wall clock
+	// device wall clock: the first block of the kernel that sets the state up, as
+	// it starts; the kernel that sees the end
+	unsigned long long t_begin, t_end;
 	uint32_t levels, err;
 	unsigned long long live[4];         // multi-source: sources with a non-empty frontier,
 	unsigned long long step_seq;        // as of the step (BatchRun::step) with this number

@@ -52,6 +52,7 @@ __global__ __launch_bounds__(kBlock) void small_init_kernel(Trav t, uint32_t src
 	const uint32_t d = t.deg[src];
 	const uint32_t nf = t.n_pad / 16, ntile = (d + kSparseTile - 1) / kSparseTile;
 	const uint32_t stride = gridDim.x * kBlock, i0 = blockIdx.x * kBlock + threadIdx.x;
+	if (i0 == 0) t.board->t_begin = wall_clock64();
 	if (!kBfs)
 		for (uint32_t i = i0; i < t.n_pad; i += stride) t.dist[i] = i == src ? 0u : (uint32_t)INT_MAX;
 	for (uint32_t i = i0; i < max(max(nf, t.n_words), max(t.side, ntile + 1)); i += stride) {
@@ -89,7 +90,6 @@ __global__ __launch_bounds__(kBlock) void small_init_kernel(Trav t, uint32_t src
 		}
 		t.qb.queue[0] = src;
 		t.qb.qoff[0] = 0;
-		t.board->t_begin = wall_clock64();
 	}
 }
 

@@ -92,6 +92,7 @@ __global__ __launch_bounds__(kBlock) void ssspb_clear_kernel(SsspBatch t, uint32
 {
 	const uint64_t stride = (uint64_t)gridDim.x * kBlock;
 	const uint64_t i0 = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+	if (i0 == 0) t.board->t_begin = wall_clock64();
 	for (uint64_t i = i0; i < (uint64_t)t.n_pad * kSsspBatchMax / 4; i += stride)
 		reinterpret_cast<uint4 *>(t.dist)[i] = make_uint4(kInf, kInf, kInf, kInf);
 	for (uint64_t i = i0; i < t.n_pad / 16; i += stride) reinterpret_cast<uint4 *>(t.flag)[i] = make_uint4(0, 0, 0, 0);
@@ -101,7 +102,6 @@ __global__ __launch_bounds__(kBlock) void ssspb_clear_kernel(SsspBatch t, uint32
 		if (i0 == UINT32_MAX % kLevelRing) r.fsize = 1;
 		t.rec[i0] = r;
 	}
-	if (i0 == 0) t.board->t_begin = wall_clock64();
 }
 
 // source i at slot i: distance 0, in the first frontier

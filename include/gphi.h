@@ -77,7 +77,7 @@ typedef struct gphi_stats {
 	float update_ms[GPHI_MAX_STEPS];     /* frontier update kernel time */
 	uint32_t chunks[GPHI_MAX_STEPS];     /* 2048-edge chunks a dense step swept (0 if sparse) */
 	float init_ms;                       /* state initialisation (device) */
-	float total_ms;                      /* init + all steps (device events) */
+	float total_ms;                      /* init + all steps, on the device (events or its clock) */
 	uint64_t reached;                    /* vertices with a finite result */
 	uint64_t edges_traversed;            /* sum of outdeg over reached vertices */
 } gphi_stats;

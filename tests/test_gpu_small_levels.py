@@ -164,3 +164,27 @@ def test_noalloc_after_a_refused_call_of_another_context(quiet):
             hip.hipStreamDestroy(stream)
             a.free()
             b.free()
+
+
+def test_total_time_includes_the_initialisation(quiet):
+    """total_ms is init and steps: with nothing to traverse, an SSSP takes longer
+    than a BFS by the 64 MiB of distances that its initialisation writes, 3.9 us
+    at the 17 TB/s of the Infinity Cache (8.4 at HBM's 8 TB/s)."""
+    n = 1 << 24
+    deg = np.zeros(n, np.uint32)
+    deg[1] = 1
+    gg = quiet.graph_from_arrays(n, deg, W=4096, S=16, csr_edges=np.array([2], np.uint32),
+                                 csr_weights=np.array([1], np.uint32))
+    gg.retile(4096, 16)
+    try:
+        print("case: total_ms of an empty SSSP and BFS", flush=True)
+        ms = {False: [], True: []}
+        st = G.Stats()
+        for i in range(60):
+            call = (quiet.lib.gphi_sssp if i % 2 else quiet.lib.gphi_bfs)
+            quiet.check(call(gg.h, 0, None, C.byref(st)) if i % 2 else call(gg.h, 0, None, None, C.byref(st)))
+            ms[bool(i % 2)].append(st.total_ms)
+        sssp, bfs = np.median(ms[True]), np.median(ms[False])
+        assert sssp - bfs >= 0.0039, (sssp, bfs)
+    finally:
+        gg.free()
