@@ -10,7 +10,7 @@
 //   levels  : 4 bits per level below 15 (every level of a shallow traversal),
 //             else 8, as level + 1 with 0 for unreached; widened by the host.
 //             The host's first touch of the array then sets the pace (about
-//             100 GB/s over 8 threads), not the link.
+//             100 GB/s over 8 threads; up to 12 take part), not the link.
 //   distances: 4, 8 or 16 bits when the largest one fits, found by a pass over
 //             them first (from kNarrowBytes of output on), as distance + 1 with
 //             0 for unreached

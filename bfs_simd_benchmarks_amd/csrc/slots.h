@@ -21,8 +21,8 @@ constexpr uint32_t kAllHelpers = 22;   // threads that help the copy-outs of a p
 constexpr int kSlotsStalled = 1;       // run_slots: nothing is under way that would fill the next slot
 
 // One turn of a wait for memory that a kernel or another thread writes: the
-// first ones, about 50 us, keep the core; later ones give it to whoever wants it,
-// above all to the threads this one waits for.
+// first ones, some tens of microseconds, keep the core; later ones give it to
+// whoever wants it, above all to the threads this one waits for.
 struct Turn {
 	uint32_t n = 0;
 	void wait()
@@ -37,7 +37,9 @@ struct Turn {
 
 // Helpers of the copy-outs under way, over the process: several calls at once
 // (the lanes of a server, contexts of several threads) share the cores that one
-// call may use, instead of each taking as many.
+// call may use, instead of each taking as many.  Batches of 64 sources with rows
+// of 2^20 levels on 16 cores, a round of one batch per context: 6 contexts 20 ->
+// 6.8 ms, 12 contexts 54 -> 13.7, one or two as before.
 inline std::atomic<uint32_t> g_helpers{0};
 inline uint32_t lease_helpers(uint32_t want, uint32_t limit)
 {
